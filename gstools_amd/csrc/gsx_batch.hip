@@ -60,7 +60,7 @@ __device__ __forceinline__ void batch_tile(const gsx_batch_item& it, Pts pts, in
 #pragma unroll
         for (int c = 0; c < NOUT; ++c) acc[p][c] = 0.0;
     }
-    const double xseg = segment_xmax<D, PPT>(pts, P, p0, own, s_wmax);
+    const double xseg = segment_xmax<D, kThreads, kThreads * PPT>(pts, P, p0, own, s_wmax);
     fp32_item_sum<D, PPT, INCOMPR, CHUNK>(it.N, it.cov, it.z1, it.z2, nullptr, xseg, x, acc, tabd, tabf,
                                           s_nmagic);
 #pragma unroll

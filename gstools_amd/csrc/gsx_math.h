@@ -72,11 +72,19 @@ GSX_HD double horner(const double (&c)[NC], double s) {
 
 GSX_HD uint32_t lo_word(double v) { return (uint32_t)__builtin_bit_cast(uint64_t, v); }
 
-// Flip the sign of v when bit 0 of `odd` is set (one 32-bit XOR of the high word).
+// Flip the sign of v when bit 0 of `odd` is set: adding that bit at bit 31 of the
+// high word is the same as XOR there (the carry falls off).  On the GPU one
+// v_lshl_add_u32, written out because the compiler otherwise joins the halves
+// into a 64-bit add or keeps a shift and an XOR.
 GSX_HD double flip_sign_if(double v, uint32_t odd) {
-    uint64_t b = __builtin_bit_cast(uint64_t, v);
-    b ^= (uint64_t)(odd << 31) << 32;
-    return __builtin_bit_cast(double, b);
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    uint32_t hi = (uint32_t)(b >> 32);
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_lshl_add_u32 %0, %1, 31, %0" : "+v"(hi) : "v"(odd));
+#else
+    hi += odd << 31;
+#endif
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | (uint32_t)b);
 }
 
 // cos(theta - phi) for |theta| <= kFastPhaseMax, |phi| <= pi, with

@@ -20,11 +20,16 @@
 // spectrum factor f_j multiplying each term; it is folded into the amplitude
 // when the table is built (fac == nullptr for the randomisation method).
 //
+// Launches of few points share the modes of a point out over the waves of a
+// block instead (k_forward_*_split); both forms add the same partial sums in the
+// same order, so a point's value does not depend on the launch it is part of.
+//
 // FP64 path: the phase is the reference's exact product-then-add sequence;
 // cos(t - phi) uses the two-term Cody-Waite reduction of gsx_math.h with phi
 // folded into the reduction (no rounding of t - phi at large |t|).  A wave
 // whose |x|_inf * max_j |k_j|_1 may exceed 2^45 takes a per-term guarded path
-// that falls back to the library sincos for |t| > 2^46.
+// that falls back to the library sincos for |t| > 2^46.  The mode sum runs over
+// groups of 64 modes, each from zero, added in order.
 //
 // FP32 path (gsx_fp32sum.h): the phase is computed in revolutions in FP64
 // (t = k/2pi . x - phi/2pi, three FMAs), reduced by magic addition (the low
@@ -42,6 +47,7 @@
 namespace gsx {
 
 constexpr int kChunk = 256;  // modes per LDS chunk (== kThreads: one mode per thread to build)
+constexpr int kGroupF64 = 64;  // modes per FP64 partial sum
 constexpr double kSafeK1X = 0x1.0p+45;  // |k|_1 |x|_inf bound of the FP64 fast path
 
 // cos(theta - phi) at any |theta|: the fast reduction where it is exact, else the
@@ -67,6 +73,81 @@ struct TabF64 {
     static constexpr int kW = INCOMPR ? 2 * D + 2 : D + 3;
     static constexpr int kStride = (kW + 1) & ~1;  // 16-byte aligned rows
 };
+
+// Table row of mode j; returns |k_j|_1.
+template <int D, bool INCOMPR>
+__device__ __forceinline__ double f64_build_row(int64_t N, int64_t j, const double* __restrict__ cov,
+                                                const double* __restrict__ z1, const double* __restrict__ z2,
+                                                const double* __restrict__ fac, double* t) {
+    double k[D];
+    double k1 = 0.0, k2 = 0.0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        k[d] = cov[d * N + j];
+        t[d] = k[d];
+        k1 += fabs(k[d]);
+        k2 += k[d] * k[d];
+    }
+    const double u1 = z1[j], u2 = z2[j];
+    const double phi = atan2(u2, u1);
+    const double a = fac ? fac[j] * hypot(u1, u2) : hypot(u1, u2);
+    if constexpr (INCOMPR) {
+        t[D] = phi;
+        t[D + 1] = phi * kInvPi;
+#pragma unroll
+        for (int c = 0; c < D; ++c) {
+            const double proj = (c == 0 ? 1.0 : 0.0) - k[c] * k[0] / k2;
+            t[D + 2 + c] = proj * a;
+        }
+    } else {
+        t[D] = a;
+        t[D + 1] = phi;
+        t[D + 2] = phi * kInvPi;
+    }
+    return k1;
+}
+
+// Table rows [m0, m1) into the partial sums of one mode group.  SAFE: every
+// phase lies within the fast reduction; else each term is checked and falls
+// back to the library sincos.
+template <int D, int PPT, bool INCOMPR, bool SAFE>
+__device__ __forceinline__ void f64_group_sum(const double* tab, int m0, int m1, const double (&x)[PPT][D],
+                                              double (&part)[PPT][INCOMPR ? D : 1]) {
+    using T = TabF64<D, INCOMPR>;
+    constexpr int NOUT = INCOMPR ? D : 1;
+#pragma unroll
+    for (int p = 0; p < PPT; ++p)
+#pragma unroll
+        for (int c = 0; c < NOUT; ++c) part[p][c] = 0.0;
+    auto term = [&](int m) {
+        const double* t = tab + m * T::kStride;
+        double k[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) k[d] = t[d];
+        const double phi = INCOMPR ? t[D] : t[D + 1];
+        const double phipi = INCOMPR ? t[D + 1] : t[D + 2];
+        double w[NOUT];
+#pragma unroll
+        for (int c = 0; c < NOUT; ++c) w[c] = INCOMPR ? t[D + 2 + c] : t[D];
+#pragma unroll
+        for (int p = 0; p < PPT; ++p) {
+            const double th = phase_exact<D>(k, x[p]);
+            const double cs = SAFE ? cos_shifted(th, phi, phipi) : cos_shifted_any(th, phi, phipi);
+#pragma unroll
+            for (int c = 0; c < NOUT; ++c) part[p][c] = fma_(w[c], cs, part[p][c]);
+        }
+    };
+    int m = m0;
+    if constexpr (SAFE) {
+        // two modes per iteration (by hand: the compiler does not unroll a loop of
+        // unknown length around inline assembly)
+        for (; m + 1 < m1; m += 2) {
+            term(m);
+            term(m + 1);
+        }
+    }
+    for (; m < m1; ++m) term(m);
+}
 
 template <int D, int PPT, bool INCOMPR, class Pts>
 __global__ __launch_bounds__(kThreads) void k_forward_f64(Pts pts, int64_t N, int64_t P,
@@ -105,84 +186,26 @@ __global__ __launch_bounds__(kThreads) void k_forward_f64(Pts pts, int64_t N, in
         __syncthreads();
         if (threadIdx.x == 0) s_kmax = 0ull;
         __syncthreads();
-        if ((int)threadIdx.x < cnt) {
-            const int64_t j = j0 + threadIdx.x;
-            double* t = tab + threadIdx.x * T::kStride;
-            double k[D];
-            double k1 = 0.0, k2 = 0.0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                k[d] = cov[d * N + j];
-                t[d] = k[d];
-                k1 += fabs(k[d]);
-                k2 += k[d] * k[d];
-            }
-            const double u1 = z1[j], u2 = z2[j];
-            const double phi = atan2(u2, u1);
-            const double a = fac ? fac[j] * hypot(u1, u2) : hypot(u1, u2);
-            if constexpr (INCOMPR) {
-                t[D] = phi;
-                t[D + 1] = phi * kInvPi;
-#pragma unroll
-                for (int c = 0; c < D; ++c) {
-                    const double proj = (c == 0 ? 1.0 : 0.0) - k[c] * k[0] / k2;
-                    t[D + 2 + c] = proj * a;
-                }
-            } else {
-                t[D] = a;
-                t[D + 1] = phi;
-                t[D + 2] = phi * kInvPi;
-            }
-            lds_max_u64(&s_kmax, k1);
-        }
+        if ((int)threadIdx.x < cnt)
+            lds_max_u64(&s_kmax, f64_build_row<D, INCOMPR>(N, j0 + threadIdx.x, cov, z1, z2, fac,
+                                                           tab + threadIdx.x * T::kStride));
         __syncthreads();
         const double kmax = __longlong_as_double((long long)s_kmax);
         bool safe = true;
 #pragma unroll
         for (int p = 0; p < PPT; ++p) safe = safe && (xmax[p] * kmax <= kSafeK1X);
-
-        if (__all(safe)) {
-            for (int m = 0; m < cnt; ++m) {
-                const double* t = tab + m * T::kStride;
-                double k[D];
+        const bool all_safe = __all(safe);
+        for (int m0 = 0; m0 < cnt; m0 += kGroupF64) {
+            const int m1 = m0 + kGroupF64 < cnt ? m0 + kGroupF64 : cnt;
+            double part[PPT][NOUT];
+            if (all_safe)
+                f64_group_sum<D, PPT, INCOMPR, true>(tab, m0, m1, x, part);
+            else
+                f64_group_sum<D, PPT, INCOMPR, false>(tab, m0, m1, x, part);
 #pragma unroll
-                for (int d = 0; d < D; ++d) k[d] = t[d];
-                if constexpr (INCOMPR) {
-                    const double phi = t[D], phipi = t[D + 1];
-                    double w[D];
+            for (int p = 0; p < PPT; ++p)
 #pragma unroll
-                    for (int c = 0; c < D; ++c) w[c] = t[D + 2 + c];
-#pragma unroll
-                    for (int p = 0; p < PPT; ++p) {
-                        const double cs = cos_shifted(phase_exact<D>(k, x[p]), phi, phipi);
-#pragma unroll
-                        for (int c = 0; c < D; ++c) acc[p][c] = fma_(w[c], cs, acc[p][c]);
-                    }
-                } else {
-                    const double a = t[D], phi = t[D + 1], phipi = t[D + 2];
-#pragma unroll
-                    for (int p = 0; p < PPT; ++p)
-                        acc[p][0] = fma_(a, cos_shifted(phase_exact<D>(k, x[p]), phi, phipi), acc[p][0]);
-                }
-            }
-        } else {
-            // Guarded path: library sincos for phases beyond the fast reduction.
-            for (int m = 0; m < cnt; ++m) {
-                const double* t = tab + m * T::kStride;
-                double k[D];
-#pragma unroll
-                for (int d = 0; d < D; ++d) k[d] = t[d];
-                const double phi = INCOMPR ? t[D] : t[D + 1];
-                const double phipi = INCOMPR ? t[D + 1] : t[D + 2];
-                for (int p = 0; p < PPT; ++p) {
-                    const double cs = cos_shifted_any(phase_exact<D>(k, x[p]), phi, phipi);
-                    if constexpr (INCOMPR) {
-                        for (int c = 0; c < D; ++c) acc[p][c] = fma_(t[D + 2 + c], cs, acc[p][c]);
-                    } else {
-                        acc[p][0] = fma_(t[D], cs, acc[p][0]);
-                    }
-                }
-            }
+                for (int c = 0; c < NOUT; ++c) acc[p][c] += part[p][c];
         }
     }
 
@@ -193,6 +216,90 @@ __global__ __launch_bounds__(kThreads) void k_forward_f64(Pts pts, int64_t N, in
 #pragma unroll
             for (int c = 0; c < NOUT; ++c) out[c * P + i] = acc[p][c];
         }
+    }
+}
+
+// Few points: the mode groups of a point are shared out over the waves of a
+// block, 16 groups (1024 modes) at a time, and over L equal parts of each
+// wave's lanes: a block of 1024 / L threads holds PB = 64 / L * PPT points.
+// Every (group, point) partial sum goes through LDS and the groups are added in
+// order, so a point's value is the same bits as in k_forward_f64.
+constexpr int kSplitModes = 1024;
+
+template <int D, int PPT, int L, bool INCOMPR, class Pts>
+__global__ __launch_bounds__(kSplitModes / L) void k_forward_f64_split(Pts pts, int64_t N, int64_t P,
+                                                                       const double* __restrict__ cov,
+                                                                       const double* __restrict__ z1,
+                                                                       const double* __restrict__ z2,
+                                                                       const double* __restrict__ fac,
+                                                                       double* __restrict__ out) {
+    using T = TabF64<D, INCOMPR>;
+    constexpr int NOUT = INCOMPR ? D : 1;
+    constexpr int kT = kSplitModes / L;             // threads
+    constexpr int kG = kSplitModes / kGroupF64;     // groups at a time
+    constexpr int kLP = 64 / L;                     // lanes (and points per PPT) of a part
+    constexpr int kPB = kLP * PPT;                  // points of the block
+    static_assert(kPB * NOUT <= kT, "one thread adds the groups of one output");
+    __shared__ __align__(16) double tab[kSplitModes * T::kStride];
+    __shared__ double s_part[kG][kPB * NOUT];
+    __shared__ unsigned long long s_kmax;
+
+    const int t = (int)threadIdx.x;
+    const int lane = t & 63, wave = t >> 6;
+    const int grp = wave * L + lane / kLP;          // this lane's group of the 16
+    const int64_t p0 = (int64_t)blockIdx.x * kPB;
+    double x[PPT][D];
+    double xmax = 0.0;
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) {
+        const int64_t i = p0 + p * kLP + lane % kLP;
+        if (i < P) {
+            pts.get(i, x[p]);
+        } else {
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[p][d] = 0.0;
+        }
+    }
+    // NaN coordinates are left out of the bound (fmax), as in k_forward_f64
+#pragma unroll
+    for (int p = 0; p < PPT; ++p)
+#pragma unroll
+        for (int d = 0; d < D; ++d) xmax = fmax(xmax, fabs(x[p][d]));
+    double acc = 0.0;  // output t of the block: component t / kPB of point t % kPB
+
+    for (int64_t j0 = 0; j0 < N; j0 += kSplitModes) {
+        const int cnt = (int)(N - j0 < kSplitModes ? N - j0 : kSplitModes);
+        if (t == 0) s_kmax = 0ull;
+        __syncthreads();  // also: the last chunk's table and partial sums are no longer read
+#pragma unroll
+        for (int q = 0; q < L; ++q) {
+            const int m = t + q * kT;
+            if (m < cnt)
+                lds_max_u64(&s_kmax,
+                            f64_build_row<D, INCOMPR>(N, j0 + m, cov, z1, z2, fac, tab + m * T::kStride));
+        }
+        __syncthreads();
+        const double kmax = __longlong_as_double((long long)s_kmax);
+        const int m0 = grp * kGroupF64 < cnt ? grp * kGroupF64 : cnt;
+        const int m1 = m0 + kGroupF64 < cnt ? m0 + kGroupF64 : cnt;
+        double part[PPT][NOUT];
+        if (__all(xmax * kmax <= kSafeK1X))
+            f64_group_sum<D, PPT, INCOMPR, true>(tab, m0, m1, x, part);
+        else
+            f64_group_sum<D, PPT, INCOMPR, false>(tab, m0, m1, x, part);
+#pragma unroll
+        for (int p = 0; p < PPT; ++p)
+#pragma unroll
+            for (int c = 0; c < NOUT; ++c) s_part[grp][c * kPB + p * kLP + lane % kLP] = part[p][c];
+        __syncthreads();
+        if (t < kPB * NOUT) {
+            const int groups = (cnt + kGroupF64 - 1) / kGroupF64;
+            for (int g = 0; g < groups; ++g) acc += s_part[g][t];
+        }
+    }
+    if (t < kPB * NOUT) {
+        const int64_t i = p0 + t % kPB;
+        if (i < P) out[(int64_t)(t / kPB) * P + i] = acc;
     }
 }
 
@@ -230,7 +337,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
 #pragma unroll
         for (int c = 0; c < NOUT; ++c) acc[p][c] = 0.0;
     }
-    const double xseg = segment_xmax<D, PPT>(pts, P, p0, own, s_wmax);
+    const double xseg = segment_xmax<D, kThreads, kThreads * PPT>(pts, P, p0, own, s_wmax);
     fp32_item_sum<D, PPT, INCOMPR, kChunk>(N, cov, z1, z2, fac, xseg, x, acc, tabd, tabf, s_nmagic);
 
 #pragma unroll
@@ -243,6 +350,87 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3))) v
     }
 }
 
+// Few points: the mode groups of a point are shared out over the block's waves,
+// 1024 modes (8 groups) at a time, two waves per group (the first takes the
+// group's first run of at most kSub modes, the second the others); a block of
+// 1024 threads holds PB = 64 PPT points.  The FP32 partial sums of every run (at
+// most three per group) go through LDS and are added into the FP64 accumulator
+// in order, so a point's value is the same bits as in k_forward_f32.
+template <int D, int PPT, bool INCOMPR, class Pts>
+__global__ __launch_bounds__(kSplitModes) void k_forward_f32_split(
+    Pts pts, int64_t N, int64_t P, const double* __restrict__ cov, const double* __restrict__ z1,
+    const double* __restrict__ z2, const double* __restrict__ fac, float* __restrict__ out) {
+    constexpr int NOUT = INCOMPR ? D : 1;
+    constexpr int kG = kSplitModes / kGroup;
+    constexpr int kRuns = 3;          // runs of <= kSub modes in a group of two ordered parts
+    constexpr int kPB = 64 * PPT;
+    static_assert(kGroup == 2 * kSub, "two parts of a group: at most three runs");
+    static_assert(kPB * NOUT <= kSplitModes, "one thread adds the runs of one output");
+    __shared__ double tabd[kSplitModes * (D + 1)];
+    __shared__ float tabf[kSplitModes * NOUT];
+    __shared__ float s_part[kG * kRuns][kPB * NOUT];
+    __shared__ double s_wmax[kSplitModes / 64];
+    __shared__ int s_nmagic[kSplitModes / 64];
+
+    const int t = (int)threadIdx.x;
+    const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int grp = wave >> 1, half = wave & 1;
+    const int64_t p0 = (int64_t)blockIdx.x * kPB;
+    double x[PPT][D];
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) {
+        const int64_t i = p0 + p * 64 + lane;
+        if (i < P) {
+            pts.get(i, x[p]);
+        } else {
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[p][d] = 0.0;
+        }
+    }
+    const double xseg = segment_xmax<D, kSplitModes, kPB>(pts, P, p0, 0.0, s_wmax);
+    double acc = 0.0;  // output t of the block: component t / kPB of point t % kPB
+
+    for (int64_t j0 = 0; j0 < N; j0 += kSplitModes) {
+        const int cnt = (int)(N - j0 < kSplitModes ? N - j0 : kSplitModes);
+        fp32_build_table<D, INCOMPR>(N, j0, cnt, cov, z1, z2, fac, xseg, tabd, tabf, s_nmagic);
+        const int g0 = grp * kGroup;
+        if (g0 < cnt) {
+            const int ge = g0 + kGroup < cnt ? g0 + kGroup : cnt;
+            const int gm = g0 + s_nmagic[2 * grp] + s_nmagic[2 * grp + 1];
+            // runs in order: magic modes [g0, gm) then the others [gm, ge), kSub at a time
+            int m = g0;
+#pragma unroll 1
+            for (int run = 0; run < kRuns; ++run) {
+                const int top = m < gm ? gm : ge;
+                const int me = m + kSub < top ? m + kSub : top;
+                if ((run == 0) == (half == 0)) {
+                    float part[PPT][NOUT];
+                    if (m < gm)
+                        sub_run_f32<D, PPT, NOUT, true>(tabd, tabf, m, me, x, part);
+                    else
+                        sub_run_f32<D, PPT, NOUT, false>(tabd, tabf, m, me, x, part);
+#pragma unroll
+                    for (int p = 0; p < PPT; ++p)
+#pragma unroll
+                        for (int c = 0; c < NOUT; ++c)
+                            s_part[grp * kRuns + run][c * kPB + p * 64 + lane] = part[p][c];
+                }
+                m = me;
+            }
+        }
+        __syncthreads();
+        if (t < kPB * NOUT) {
+            // runs past a group's last one hold +0, which changes nothing
+            const int runs = (cnt + kGroup - 1) / kGroup * kRuns;
+            for (int r = 0; r < runs; ++r) acc += (double)s_part[r][t];
+        }
+    }
+    if (t < kPB * NOUT) {
+        const int64_t i = p0 + t % kPB;
+        if (i < P) out[(int64_t)(t / kPB) * P + i] = (float)acc;
+    }
+}
+
 // ------------------------------------------------------------ launchers -----
 constexpr int kPptF64 = 2;
 // FP32 points per thread: 8 for the scalar sum (the per-block mode tables and
@@ -252,14 +440,63 @@ constexpr int kPptF64 = 2;
 template <bool INCOMPR>
 constexpr int ppt_f32() { return INCOMPR ? 4 : 8; }
 
+template <int D, int PPT, int L, bool INCOMPR, class Pts>
+int launch_f64_split(Pts pts, int64_t N, int64_t P, const double* cov, const double* z1, const double* z2,
+                     const double* fac, double* out, hipStream_t s) {
+    const int64_t blocks = ceil_div(P, (int64_t)(64 / L * PPT));
+    hipLaunchKernelGGL((k_forward_f64_split<D, PPT, L, INCOMPR, Pts>), dim3((unsigned)blocks), dim3(kSplitModes / L),
+                       0, s, pts, N, P, cov, z1, z2, fac, out);
+    return launch_status();
+}
+
+template <int D, int PPT, bool INCOMPR, class Pts>
+int launch_f32_split(Pts pts, int64_t N, int64_t P, const double* cov, const double* z1, const double* z2,
+                     const double* fac, float* out, hipStream_t s) {
+    const int64_t blocks = ceil_div(P, (int64_t)(64 * PPT));
+    hipLaunchKernelGGL((k_forward_f32_split<D, PPT, INCOMPR, Pts>), dim3((unsigned)blocks), dim3(kSplitModes), 0, s,
+                       pts, N, P, cov, z1, z2, fac, out);
+    return launch_status();
+}
+
+// Whether the split kernels serve (N, P).  A plain block walks all N modes for
+// its 512 (FP64) or 2048 / 1024 (FP32 scalar / incompressible) points, so up to
+// one block per CU a launch takes the time of one block whatever P is (10^4
+// points, 1000 modes, 2D: FP64 130 us, FP32 119 us); a split launch takes rounds
+// of 256 blocks (24 and 14 us).  Fits of the measured times (us; 2D and 3D, 64 to
+// 4096 modes, 1 to 10^6 points; C chunks of 1024 modes, R rounds):
+//   FP64  plain N / 7.7      split R (8 C + N / 46)
+//   FP32  plain 5 + N / 8.9  split R (12 C + N / 56)
+// The plain fits hold up to 131072 (FP64), 524288 (FP32) and 262144 (FP32
+// incompressible) points; the rounds that the inequalities allow end before.
+template <bool F64>
+inline bool split_pays(int64_t N, int64_t P, int64_t round_points) {
+    const double R = (double)ceil_div(P, round_points), C = (double)ceil_div(N, (int64_t)kSplitModes);
+    const double n = (double)N;
+    if (R > 4.0) return false;
+    return F64 ? R * (8.0 * C + n / 46.0) <= n / 7.7 : R * (12.0 * C + n / 56.0) <= 5.0 + n / 8.9;
+}
+
 template <int D, bool INCOMPR, class Pts, class OutT>
 int launch_forward(Pts pts, int64_t N, int64_t P, const double* cov, const double* z1,
                    const double* z2, const double* fac, OutT* out, hipStream_t s) {
     if constexpr (sizeof(OutT) == 8) {
+        // the smallest blocks that keep the launch within one round of 256
+        if (split_pays<true>(N, P, 256 * 128)) {
+            if (P <= 256 * 32) return launch_f64_split<D, 1, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+            if (P <= 256 * 64) return launch_f64_split<D, 2, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+            return launch_f64_split<D, 2, 1, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+        }
         const int64_t blocks = ceil_div(P, (int64_t)kThreads * kPptF64);
         hipLaunchKernelGGL((k_forward_f64<D, kPptF64, INCOMPR, Pts>), dim3((unsigned)blocks),
                            dim3(kThreads), 0, s, pts, N, P, cov, z1, z2, fac, out);
     } else {
+        constexpr int big = INCOMPR ? 4 : 8;  // points per thread of the largest split block
+        if (split_pays<false>(N, P, 256 * 64 * big)) {
+            if (P <= 256 * 64) return launch_f32_split<D, 1, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+            if (P <= 256 * 128) return launch_f32_split<D, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+            if (P <= 256 * 256) return launch_f32_split<D, 4, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+            return launch_f32_split<D, big, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
+        }
         constexpr int ppt = ppt_f32<INCOMPR>();
         const int64_t blocks = ceil_div(P, (int64_t)kThreads * ppt);
         hipLaunchKernelGGL((k_forward_f32<D, ppt, INCOMPR, Pts>), dim3((unsigned)blocks),

@@ -221,3 +221,25 @@ def test_config2_sample_fp64_fp32():
     rel_max, rel_rms = oracle.rel_errors(got32, ref)
     _say(f"config 2 fp32 rel_max={rel_max:.3e} rel_rms={rel_rms:.3e}")
     assert rel_max <= FP32_TOL and rel_rms <= FP32_TOL
+
+
+@pytest.mark.parametrize("incompr", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("d,n", [(2, 64), (3, 200), (2, 1500), (3, 1025)])
+def test_split_launches_equal_plain_launch(d, n, precision, incompr):
+    """Launches of few points share each point's modes out over a block's waves; their values
+    equal those of a launch too large for that, bit for bit, at the edges of the block sizes.
+    One far point per 2048-point segment keeps the FP32 phase bound of every prefix the same
+    and puts some modes of every group on the other phase reduction."""
+    big = 600_001  # plain launch for every n here
+    rs = np.random.RandomState(n)
+    cov = torch.from_numpy(rs.standard_cauchy(size=(d, n))).cuda()
+    z1, z2 = torch.from_numpy(rs.normal(size=(2, n))).cuda()
+    pos = torch.from_numpy(rs.uniform(-200.0, 200.0, size=(d, big))).cuda()
+    pos[:, ::2048] *= 5e3
+    fn = summate_incompr_device if incompr else summate_device
+    want = fn(cov, z1, z2, pos, precision).reshape(-1, big)
+    assert bool(torch.isfinite(want).all())
+    for p in (1, 31, 33, 64, 65, 127, 129, 8192, 8193, 16385, 32769, 65537, 131073):
+        got = fn(cov, z1, z2, pos[:, :p].contiguous(), precision).reshape(-1, p)
+        assert torch.equal(got, want[:, :p]), (p, precision)
