@@ -11,6 +11,10 @@
 //   est(f[m,k] - f[m,j]) (x^2 or sqrt|x|) and one count.  The comparisons
 //   are written exactly as there, so a NaN distance falls in every bin.
 //
+// One field on Euclidean distances without directions has its own pair kernel
+// (gsx_vario_iso.hip); the one here serves several fields, directions and
+// great-circle distances.
+//
 // Pair kernel: a persistent grid walks the upper triangle of 256 x 256 point
 // tiles (tile (tj, tk), tk >= tj, round robin over blocks).  Thread t owns
 // point j = 256 tj + t (coordinates and field values in registers); the k
@@ -29,7 +33,7 @@
 // write per-tile partials reduced in a fixed order.
 #include <type_traits>
 
-#include "gsx_internal.h"
+#include "gsx_vario.h"
 
 namespace gsx {
 
@@ -68,38 +72,6 @@ __device__ __forceinline__ double haversine(double lat_j, double lon_j, double c
 
 __device__ __forceinline__ double vario_est(int cressie, double x) { return cressie ? sqrt(fabs(x)) : x * x; }
 
-// Largest b with e[b] <= x for non-decreasing e[0..B]; -1 if x < e[0].
-__device__ __forceinline__ int64_t upper_edge(const double* e, int64_t B, double x) {
-    int64_t lo = 0, hi = B + 1;  // answer in [lo - 1, hi - 1]
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (e[mid] <= x)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo - 1;
-}
-
-// T(e) = the smallest double x >= 0 with sqrt(x) >= e (sqrt correctly rounded,
-// hence monotone): sqrt(d2) >= e exactly when d2 >= T(e), so bins can be found on
-// squared distances with the reference's sqrt-then-compare decisions.  e <= 0
-// gives -1 (every d2 >= 0 passes), e = +inf gives +inf, NaN stays NaN.
-__device__ double sq_threshold(double e) {
-    if (e != e) return e;
-    if (e <= 0.0) return -1.0;
-    double x = e * e;
-    while (sqrt(x) < e) x = nextafter(x, __builtin_inf());
-    for (;;) {
-        const double y = nextafter(x, 0.0);
-        if (y >= 0.0 && sqrt(y) >= e && y < x)
-            x = y;
-        else
-            break;
-    }
-    return x;
-}
-
 // Q(tol) = the smallest double q in [0, 1) with acos(q) < tol (acos non-increasing):
 // for q in [0, 1), acos(q) < tol exactly when q >= Q(tol); 1.0 when no q in [0, 1)
 // qualifies (tol <= 0 or NaN), 0.0 when every one does.  Bisection over the bit
@@ -118,15 +90,6 @@ __device__ double acos_threshold(double tol) {
     return __longlong_as_double(hi);
 }
 
-// Smallest-index form of the bin search for non-decreasing edges: g in [-1, B]
-// with e[g] <= x < e[g+1] (e[-1] = -inf, e[B+1] = +inf), starting from a guess
-// (uniform edges: the guess is exact but for rounding, so the loops run 0-1 times).
-__device__ __forceinline__ int bin_from_guess(const double* e, int B, double x, int g) {
-    while (g >= 0 && e[g] > x) --g;
-    while (g < B && e[g + 1] <= x) ++g;
-    return g;
-}
-
 // One pair into slot idx of this thread's histogram row: LDS adds without a
 // return value.  The row is the thread's own and adds to one location are
 // ordered as the program issues them, so every slot adds its pairs in pair
@@ -136,16 +99,12 @@ __device__ __forceinline__ void hist_add(double* h_sum, unsigned* h_cnt, int idx
     __hip_atomic_fetch_add(&h_cnt[idx], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// FAST: one field, no directions; a block whose edges are non-decreasing runs a
-// straight-line pair loop (the general loop covers everything else).
-// CRESSIE selects the estimator of the FAST loop at compile time (a runtime flag
-// would be if-converted into computing both estimators for every pair).
 // HAV: (lat, lon) points in degrees, great-circle distances (general loop, DIM 2,
 // a third staged row holds cos(lat)).
 // DIRF: directional estimate of one field with non-decreasing edges: waves whose
 // points and staged tile are all finite run a straight-line loop over four pairs
 // per step and the directions in turn (others take the general loop).
-template <int DIM, bool FAST, bool CRESSIE, bool HAV = false, bool DIRF = false>
+template <int DIM, bool CRESSIE, bool HAV = false, bool DIRF = false>
 __global__ __launch_bounds__(kVT) void k_vario_pairs(VarioArgs a, const double* __restrict__ f,
                                                      const double* __restrict__ edges,
                                                      const double* __restrict__ pos,
@@ -166,8 +125,8 @@ __global__ __launch_bounds__(kVT) void k_vario_pairs(VarioArgs a, const double* 
     // [0, 1)), sqrt(bd) < bandwidth <=> bd < s_tol[1] (bd >= 0 or NaN)
     double* s_tol = s_thp + (a.B + 3);
     double* s_dirs = s_tol + 2;
-    static_assert(!HAV || (DIM == 2 && !FAST), "haversine distances: 2D, general loop");
-    static_assert(!DIRF || (!FAST && !HAV), "directional straight-line loop: its own variant");
+    static_assert(!HAV || DIM == 2, "haversine distances: 2D, general loop");
+    static_assert(!DIRF || !HAV, "directional straight-line loop: its own variant");
     constexpr int NPOS = HAV ? DIM + 1 : DIM;  // staged coordinate rows
     // staged tile: coordinates then field values, rows of kVT, then kVPad zeros;
     // a read up to 7 entries past a row lands in the next row or in the pad
@@ -200,7 +159,7 @@ __global__ __launch_bounds__(kVT) void k_vario_pairs(VarioArgs a, const double* 
     bool mono = true;
     for (int64_t i = 0; i < a.B; ++i) mono = mono && (s_edges[i] <= s_edges[i + 1]);
     // near-uniform edges: bin guess from the spacing (exactness comes from the edge checks)
-    const int Bi = (int)a.B, NHi = (int)NH, h0i = (int)a.h0;
+    const int Bi = (int)a.B, NHi = (int)NH;
     const double e0 = s_edges[0];
     const double w = Bi > 0 ? (s_edges[Bi] - e0) / Bi : 0.0;
     // uniform: every edge within w/4 of e0 + i w, and w not below 4e-6 of the edge
@@ -219,8 +178,6 @@ __global__ __launch_bounds__(kVT) void k_vario_pairs(VarioArgs a, const double* 
     const int64_t d_last = a.directional ? (a.h1 - 1) / a.B : 0;
     const int64_t d_first = a.directional ? (a.separate ? 0 : a.h0 / a.B) : 0;
 
-    double nan_sum = 0.0;  // NaN-distance pairs of this thread (every bin takes them)
-    unsigned nan_cnt = 0u;
     const int64_t ntp = a.nt * a.nt;
     for (int64_t tt = blockIdx.x; tt < ntp; tt += gridDim.x) {
         const int64_t tj = tt / a.nt, tk = tt - tj * a.nt;
@@ -257,98 +214,6 @@ __global__ __launch_bounds__(kVT) void k_vario_pairs(VarioArgs a, const double* 
 #pragma unroll
         for (int m = 0; m < kVFields; ++m) fj[m] = (m < a.F) ? f[m * a.P + j] : 0.0;
         const int kstart = (tj == tk) ? t + 1 : 0;
-        if constexpr (FAST) {
-            if (mono) {
-                const double fj0 = fj[0];
-                const bool fj_ok = (a.F > 0) && (fj0 == fj0);
-                const int kend = (int)kn;
-                // Four pairs per step.  Every pair updates one histogram slot; pairs
-                // that are not counted (out of range, outside this launch's slots,
-                // NaN) go to the scratch row NH, so values and counts need no
-                // selects.  The four slots are read together; a later pair in the
-                // same slot as an earlier one adds onto that pair's new value
-                // (the latest earlier match), and the writes go out in pair order,
-                // so the last write to a slot holds every pair's contribution.
-                // CLEAN: every coordinate and field value of this wave's points and
-                // of the staged tile is finite, so no pair has a NaN distance or a
-                // NaN field value.
-                auto run = [&](auto uni, auto clean) {
-                    constexpr bool UNI = decltype(uni)::value;
-                    constexpr bool CLEAN = decltype(clean)::value;
-                    // eight pairs per iteration: their bins are found together (the
-                    // threshold reads overlap), then two updates of four slots each,
-                    // in order (the second group's reads see the first group's writes)
-                    for (int k8 = kstart; k8 < kend; k8 += 8) {
-                        int slot[8];
-                        double val[8];
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) {
-                            // past kend (at most 7 entries) the reads see staged values,
-                            // zeros or the pad, all finite when CLEAN; such pairs go to
-                            // the scratch row
-                            const int kk = k8 + u;
-                            const bool live = kk < kend;
-                            double d2 = 0.0;
-#pragma unroll
-                            for (int c = 0; c < DIM; ++c) {
-                                const double dd = s_pos[c * kVT + kk] - xj[c];
-                                d2 += dd * dd;
-                            }
-                            const double fk = s_f[kk];
-                            const double x = fk - fj0;
-                            const double v = CRESSIE ? sqrt(fabs(x)) : x * x;
-                            bool ok = live;
-                            if constexpr (!CLEAN) {
-                                ok = ok && fj_ok && (fk == fk);
-                                const bool dnan = d2 != d2;  // in every bin by the reference's comparisons
-                                nan_sum += (dnan && ok) ? v : 0.0;
-                                nan_cnt += (dnan && ok) ? 1u : 0u;
-                                ok = ok && !dnan;
-                            }
-                            int g;
-                            if constexpr (UNI) {
-                                // guess from an FP32 distance, within 0.1 bin of (d - e0) / w
-                                // for the edges `uniform` admits (every edge within w/4 of
-                                // uniform), so the truncated guess is within one bin of the
-                                // true one and one threshold step is exact; thresholds are
-                                // non-decreasing, so at most one of dec / inc holds
-                                float q = __builtin_fmaf(__builtin_amdgcn_sqrtf((float)d2), inv_wf, qoff);
-                                if constexpr (!CLEAN) q = (d2 == d2) ? q : -1.0f;
-                                q = __builtin_amdgcn_fmed3f(q, -1.0f, (float)Bi);
-                                const int g0 = (int)q;  // -1 .. B
-                                const double tdown = s_thp[g0 + 1], tup = s_thp[g0 + 2];  // T(e_g0), T(e_g0+1)
-                                g = g0 - (tdown > d2 ? 1 : 0) + (tup <= d2 ? 1 : 0);
-                            } else {
-                                g = (int)upper_edge(s_thr, a.B, d2);
-                            }
-                            // g is made opaque so the search stays unconditional: otherwise
-                            // the compiler moves it, loads included, under a branch on `ok`
-                            // and the four pairs' threshold reads no longer overlap
-                            asm volatile("" : "+v"(g));
-                            // launch slots lie in [0, B): one unsigned test covers the bin range
-                            const unsigned sl = (unsigned)(g - h0i);
-                            slot[u] = (ok && sl < (unsigned)NHi) ? (int)sl : NHi;
-                            val[u] = v;
-                        }
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) hist_add(h_sum, h_cnt, slot[u] * kVT + t, val[u]);
-                    }
-                };
-                const bool clean = !tile_nan && !__any((xj_nan || !__builtin_isfinite(fj0) || a.F < 1) ? 1 : 0);
-                if (uniform) {
-                    if (clean)
-                        run(std::integral_constant<bool, true>{}, std::integral_constant<bool, true>{});
-                    else
-                        run(std::integral_constant<bool, true>{}, std::integral_constant<bool, false>{});
-                } else {
-                    if (clean)
-                        run(std::integral_constant<bool, false>{}, std::integral_constant<bool, true>{});
-                    else
-                        run(std::integral_constant<bool, false>{}, std::integral_constant<bool, false>{});
-                }
-                continue;
-            }
-        }
         if constexpr (DIRF) {
             const double fj0 = fj[0];
             const bool clean = !tile_nan && !__any((xj_nan || !__builtin_isfinite(fj0) || a.F != 1) ? 1 : 0);
@@ -495,63 +360,82 @@ __global__ __launch_bounds__(kVT) void k_vario_pairs(VarioArgs a, const double* 
             }
         }
     }
-    if (nan_cnt) {
-        for (int h = 0; h < NHi; ++h) {
-            const int b = h + h0i;
-            if (b < Bi) {
-                h_sum[h * kVT + t] += nan_sum;
-                h_cnt[h * kVT + t] += nan_cnt;
-            }
-        }
-    }
     __syncthreads();
-    // block partials: slot h summed over the threads in order
+    // block partials: slot h summed over the threads in turn, each slot starting at
+    // its own thread's column (no bank conflicts)
     for (int64_t h = t; h < NH; h += kVT) {
         double s = 0.0;
         unsigned long long c = 0;
         for (int i = 0; i < kVT; ++i) {
-            s += h_sum[h * kVT + i];
-            c += h_cnt[h * kVT + i];
+            s += h_sum[h * kVT + ((i + t) & (kVT - 1))];
+            c += h_cnt[h * kVT + ((i + t) & (kVT - 1))];
         }
-        part_sum[(int64_t)blockIdx.x * NH + h] = s;
-        part_cnt[(int64_t)blockIdx.x * NH + h] = c;
+        part_sum[h * gridDim.x + blockIdx.x] = s;
+        part_cnt[h * gridDim.x + blockIdx.x] = c;
     }
 }
 
-// Sum the block partials of slot h in block order; accumulate into the totals.
-__global__ void k_vario_collect(int64_t blocks, int64_t NH, int64_t h0, const double* __restrict__ part_sum,
-                                const unsigned long long* __restrict__ part_cnt, double* __restrict__ tot_sum,
-                                long long* __restrict__ tot_cnt, int accumulate) {
-    const int64_t h = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= NH) return;
+// Estimate from a sum and a count (Matheron or Cressie), N = max(count, 1)
+__device__ __forceinline__ double vario_gamma(double s, long long count, int cressie) {
+    const double cnt = (double)(count > 0 ? count : 1);
+    if (cressie) {
+        const double q = s / cnt;
+        return 0.5 * (q * q * (q * q)) / (0.457 + 0.494 / cnt + 0.045 / (cnt * cnt));
+    }
+    return s / (2.0 * cnt);
+}
+
+// One block per slot: its partials ([slot][block]) in a fixed order (thread t adds
+// partials t, t + 256, ..., then the threads as a tree); then into the totals, or
+// the estimate from them.  One thread per slot walking 2048 blocks took 0.53 ms.
+__global__ __launch_bounds__(256) void k_vario_collect(int64_t blocks, int64_t h0,
+                                                       const double* __restrict__ part_sum,
+                                                       const unsigned long long* __restrict__ part_cnt,
+                                                       double* __restrict__ gamma, long long* __restrict__ counts,
+                                                       int accumulate, int finish, int cressie) {
+    __shared__ double rs[4];
+    __shared__ unsigned long long rc[4];
+    const int64_t h = blockIdx.x;
     double s = 0.0;
     unsigned long long c = 0;
-    for (int64_t b = 0; b < blocks; ++b) {
-        s += part_sum[b * NH + h];
-        c += part_cnt[b * NH + h];
+#pragma unroll 8
+    for (int64_t b = threadIdx.x; b < blocks; b += 256) {
+        s += part_sum[h * blocks + b];
+        c += part_cnt[h * blocks + b];
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o);
+        c += __shfl_xor(c, o);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        rs[threadIdx.x >> 6] = s;
+        rc[threadIdx.x >> 6] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    s = (rs[0] + rs[1]) + (rs[2] + rs[3]);
+    long long n = (long long)(rc[0] + rc[1] + rc[2] + rc[3]);
     if (accumulate) {
-        tot_sum[h0 + h] += s;
-        tot_cnt[h0 + h] += (long long)c;
-    } else {
-        tot_sum[h0 + h] = s;
-        tot_cnt[h0 + h] = (long long)c;
+        s += gamma[h0 + h];
+        n += counts[h0 + h];
     }
+    counts[h0 + h] = n;
+    gamma[h0 + h] = finish ? vario_gamma(s, n, cressie) : s;
 }
 
-// gamma from sums and counts (Matheron or Cressie), N = max(count, 1)
+int vario_collect(int64_t blocks, int64_t NH, int64_t h0, const double* part_sum, const unsigned long long* part_cnt,
+                  double* gamma, int64_t* counts, bool accumulate, bool finish, int cressie, hipStream_t s) {
+    hipLaunchKernelGGL(k_vario_collect, dim3((unsigned)NH), dim3(256), 0, s, blocks, h0, part_sum, part_cnt, gamma,
+                       reinterpret_cast<long long*>(counts), accumulate ? 1 : 0, finish ? 1 : 0, cressie);
+    return launch_status();
+}
+
+// gamma from sums and counts of the axis lags
 __global__ void k_vario_normalize(int64_t n, int cressie, double* __restrict__ gamma,
                                   const long long* __restrict__ counts) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double cnt = (double)(counts[i] > 0 ? counts[i] : 1);
-    const double s = gamma[i];
-    if (cressie) {
-        const double q = s / cnt;
-        gamma[i] = 0.5 * (q * q * (q * q)) / (0.457 + 0.494 / cnt + 0.045 / (cnt * cnt));
-    } else {
-        gamma[i] = s / (2.0 * cnt);
-    }
+    if (i < n) gamma[i] = vario_gamma(gamma[i], counts[i], cressie);
 }
 
 // structured lags: block b takes lag k = b / tiles and column tile b % tiles.
@@ -786,16 +670,16 @@ inline int64_t vario_slots_per_launch(size_t limit, int64_t B, int64_t D, int di
     return (int64_t)((limit - fixed) / ((sizeof(double) + sizeof(unsigned)) * kVT));
 }
 
-template <int DIM, bool FAST, bool CRESSIE, bool HAV = false, bool DIRF = false>
+template <int DIM, bool CRESSIE, bool HAV = false, bool DIRF = false>
 int launch_pairs_t(const VarioArgs& a, size_t lds, int64_t blocks, hipStream_t s, const double* f,
                    const double* edges, const double* pos, const double* dirs, double* part_sum,
                    unsigned long long* part_cnt) {
     if (lds > 65536 &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_vario_pairs<DIM, FAST, CRESSIE, HAV, DIRF>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&k_vario_pairs<DIM, CRESSIE, HAV, DIRF>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return GSX_E_LAUNCH;
-    hipLaunchKernelGGL((k_vario_pairs<DIM, FAST, CRESSIE, HAV, DIRF>), dim3((unsigned)blocks), dim3(kVT), lds, s, a,
-                       f, edges, pos, dirs, part_sum, part_cnt);
+    hipLaunchKernelGGL((k_vario_pairs<DIM, CRESSIE, HAV, DIRF>), dim3((unsigned)blocks), dim3(kVT), lds, s, a, f, edges,
+                       pos, dirs, part_sum, part_cnt);
     return launch_status();
 }
 
@@ -803,25 +687,25 @@ template <int DIM>
 int launch_pairs(const VarioArgs& a, size_t lds, int64_t blocks, hipStream_t s, const double* f,
                  const double* edges, const double* pos, const double* dirs, double* part_sum,
                  unsigned long long* part_cnt) {
-    if (!a.directional && a.F <= 1) {
-        if (a.cressie)
-            return launch_pairs_t<DIM, true, true>(a, lds, blocks, s, f, edges, pos, dirs, part_sum, part_cnt);
-        return launch_pairs_t<DIM, true, false>(a, lds, blocks, s, f, edges, pos, dirs, part_sum, part_cnt);
-    }
     if (a.directional && a.F == 1) {
         if (a.cressie)
-            return launch_pairs_t<DIM, false, true, false, true>(a, lds, blocks, s, f, edges, pos, dirs, part_sum,
-                                                                 part_cnt);
-        return launch_pairs_t<DIM, false, false, false, true>(a, lds, blocks, s, f, edges, pos, dirs, part_sum,
-                                                              part_cnt);
+            return launch_pairs_t<DIM, true, false, true>(a, lds, blocks, s, f, edges, pos, dirs, part_sum, part_cnt);
+        return launch_pairs_t<DIM, false, false, true>(a, lds, blocks, s, f, edges, pos, dirs, part_sum, part_cnt);
     }
-    return launch_pairs_t<DIM, false, false>(a, lds, blocks, s, f, edges, pos, dirs, part_sum, part_cnt);
+    return launch_pairs_t<DIM, false>(a, lds, blocks, s, f, edges, pos, dirs, part_sum, part_cnt);
 }
 
 inline int64_t vario_pair_blocks(int64_t P) {
     const int64_t nt = ceil_div(P, (int64_t)kVT);
     const int64_t ntri = nt * (nt + 1) / 2;
     return ntri < kVBlocks ? (ntri > 0 ? ntri : 1) : kVBlocks;
+}
+
+// One field, all directions, Euclidean distances: the one-wavefront pair kernel
+// (gsx_vario_iso.hip).  Several fields share a pair's distance and bin, which
+// k_vario_pairs computes once for up to 8 of them.
+inline bool vario_iso_route(int64_t F, int64_t P, bool directional, bool haversine) {
+    return F == 1 && P > 1 && !directional && !haversine;
 }
 
 int vario_pairs(int64_t F, int64_t P, int64_t dim, int64_t B, int64_t D, const double* f, const double* edges,
@@ -852,9 +736,12 @@ int vario_pairs(int64_t F, int64_t P, int64_t dim, int64_t B, int64_t D, const d
     const int64_t tiles_per_block = ceil_div(nt * nt, blocks);
     if ((double)tiles_per_block * kVT * (double)(F > 0 ? F : 1) > 4.0e9) return GSX_E_UNSUPPORTED;
     hipStream_t s = as_stream(stream);
+    if (vario_iso_route(F, P, directional != 0, haversine)) {
+        if (ws_bytes < vario_iso_ws(P, dim, B)) return GSX_E_WORKSPACE;
+        return vario_iso(P, dim, B, f, edges, pos, estimator, gamma, counts, ws, s);
+    }
     double* part_sum = static_cast<double*>(ws);
     unsigned long long* part_cnt = reinterpret_cast<unsigned long long*>(part_sum + blocks * chunk_slots);
-    long long* tot_cnt = reinterpret_cast<long long*>(counts);
     for (int64_t h0 = 0; h0 < NHall; h0 += chunk_slots) {
         const int64_t h1 = (h0 + chunk_slots < NHall) ? h0 + chunk_slots : NHall;
         for (int64_t m0 = 0; m0 < (F > 0 ? F : 1); m0 += kVFields) {
@@ -876,8 +763,7 @@ int vario_pairs(int64_t F, int64_t P, int64_t dim, int64_t B, int64_t D, const d
             if (P > 1) {
                 const double* fm = F > 0 ? f + m0 * P : nullptr;
                 if (haversine)
-                    st = launch_pairs_t<2, false, false, true>(a, lds, blocks, s, fm, edges, pos, dirs, part_sum,
-                                                               part_cnt);
+                    st = launch_pairs_t<2, false, true>(a, lds, blocks, s, fm, edges, pos, dirs, part_sum, part_cnt);
                 else if (dim == 1)
                     st = launch_pairs<1>(a, lds, blocks, s, fm, edges, pos, dirs, part_sum, part_cnt);
                 else if (dim == 2)
@@ -885,19 +771,14 @@ int vario_pairs(int64_t F, int64_t P, int64_t dim, int64_t B, int64_t D, const d
                 else
                     st = launch_pairs<3>(a, lds, blocks, s, fm, edges, pos, dirs, part_sum, part_cnt);
                 if (st != GSX_OK) return st;
-                hipLaunchKernelGGL(k_vario_collect, dim3((unsigned)ceil_div(h1 - h0, (int64_t)256)), dim3(256), 0,
-                                   s, blocks, h1 - h0, h0, part_sum, part_cnt, gamma, tot_cnt, m0 > 0 ? 1 : 0);
-            } else {
-                hipLaunchKernelGGL(k_vario_collect, dim3((unsigned)ceil_div(h1 - h0, (int64_t)256)), dim3(256), 0,
-                                   s, (int64_t)0, h1 - h0, h0, part_sum, part_cnt, gamma, tot_cnt, 0);
             }
-            st = launch_status();
+            // (a single point has no pairs: no partials to add)
+            st = vario_collect(P > 1 ? blocks : 0, h1 - h0, h0, part_sum, part_cnt, gamma, counts, m0 > 0,
+                               m0 + kVFields >= F, estimator, s);
             if (st != GSX_OK) return st;
         }
     }
-    hipLaunchKernelGGL(k_vario_normalize, dim3((unsigned)ceil_div(NHall, (int64_t)256)), dim3(256), 0, s, NHall,
-                       estimator, gamma, tot_cnt);
-    return launch_status();
+    return GSX_OK;
 }
 
 // structured lags of an (n0, n1 >= 64) array with the register-window kernel
@@ -958,7 +839,9 @@ int64_t gsx_vario_workspace(int64_t kind, int64_t P_or_n0, int64_t dim_or_n1, in
     if (P_or_n0 < 0 || dim_or_n1 < 1 || dim_or_n1 > gsx::kVMaxDim || B < 0 || D < 1) return GSX_E_INVALID;
     // per-block partials of every (direction, bin) slot: enough for any split into launches
     const int64_t slots = (kind == 1 ? D : 1) * B;
-    return gsx::vario_pair_blocks(P_or_n0) * (slots > 0 ? slots : 1) * 16;
+    const int64_t ws = gsx::vario_pair_blocks(P_or_n0) * (slots > 0 ? slots : 1) * 16;
+    const int64_t iso = kind == 1 || P_or_n0 < 2 ? 0 : gsx::vario_iso_ws(P_or_n0, dim_or_n1, B);
+    return ws > iso ? ws : iso;
 }
 
 int gsx_vario_unstructured_f64(int64_t F, int64_t P, int64_t dim, int64_t B, const double* f, const double* edges,

@@ -234,3 +234,43 @@ def test_reference_fields_from_srf():
     cases.direction_axis(gs, field)
     cases.direction_angle(gs, field)
     cases.latlon_auto_binning(gs, field)
+
+
+def _iso_points(kind, dim, p, rs):
+    if kind == "lattice":  # every distance between neighbours lies on an edge
+        side = int(np.ceil(p ** (1.0 / dim)))
+        grid = np.stack(np.meshgrid(*[np.arange(side, dtype=float)] * dim, indexing="ij")).reshape(dim, -1)
+        return grid[:, rs.permutation(grid.shape[1])[:p]]
+    pos = rs.uniform(-50.0, 50.0, size=(dim, p))
+    if kind == "crowded":  # most points in one cell of the bounding box
+        pos[:, p // 3:] *= 1e-4
+    if kind == "odd":
+        pos[0, p // 2] = np.nan
+        pos[-1, p // 3] = np.inf
+    return pos
+
+
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "crowded", "odd"])
+@pytest.mark.parametrize("dim,p", [(1, 65), (2, 64), (3, 127), (2, 129), (1, 4097), (3, 12287), (2, 12289),
+                                   (3, 13000)])
+def test_one_field_pairs_at_tile_and_sorting_edges(kind, dim, p):
+    """One field, all directions: whole and partial 64-point tiles, below and from the size where
+    the points are sorted; edges that the FP32 form decides, edges on the distances, edges of
+    uneven width, more bins than one launch holds, and NaN values."""
+    _say(f"vario one field {kind} dim={dim} P={p}")
+    rs = np.random.RandomState(p)
+    pos = _iso_points(kind, dim, p, rs)
+    f = rs.normal(size=p)
+    f[rs.choice(p, p // 20, replace=False)] = np.nan
+    reach = 9.0 if kind == "lattice" else 40.0
+    edge_sets = [np.linspace(0.0, reach, 10), np.array([0.5, 1.0, 4.0, 4.0, 7.5])]
+    if p < 5000:
+        edge_sets += [np.linspace(1.0, reach, 102), np.array([0.0, reach])]
+    for edges in edge_sets:
+        for est in ("m", "c"):
+            g, c = v.unstructured(f, edges, pos, est)
+            g_ref, c_ref = oracle.vario_unstructured_c(f[None], edges, pos, est)
+            assert np.array_equal(c, c_ref), (edges.size, est)
+            assert np.allclose(g, g_ref, rtol=1e-12, atol=1e-300, equal_nan=True)
+            g2, c2 = v.unstructured(f, edges, pos, est)
+            assert np.array_equal(g, g2, equal_nan=True) and np.array_equal(c, c2)
