@@ -52,6 +52,26 @@ def test_kernel_matches_oracle(k, p):
     assert np.array_equal(f, f3) and np.array_equal(e, e3)  # fixed reduction order
 
 
+@pytest.mark.parametrize("k", [1, 15, 17, 31, 33, 48, 97, 128, 129, 161, 257, 400])
+def test_field_and_variance_at_block_edges(k):
+    """Systems that end inside a 16-row fragment, a 32-row diagonal block or a 128-row tile:
+    the oracle's sums within 1e-13 of the sum of absolute terms, and the same field bits with
+    and without the variance, and from an odd, an even and a cut number of points."""
+    _say(f"krige edges K={k}")
+    rs = np.random.RandomState(k)
+    m, v, c = rs.normal(size=(k, k)), rs.normal(size=(k, 391)), rs.normal(size=k)
+    f_ref, e_ref = oracle.krige_c(m, v, c)
+    bf, be = _bounds(m, v, c)
+    f, e = calc_field_krige_and_variance(m, v, c)
+    assert np.all(np.abs(f - f_ref) <= 1e-13 * bf) and np.all(np.abs(e - e_ref) <= 1e-13 * be)
+    assert np.array_equal(calc_field_krige(m, v, c), f)
+    for p in (390, 130, 1):
+        vp = np.ascontiguousarray(v[:, :p])
+        fp, ep = calc_field_krige_and_variance(m, vp, c)
+        assert np.array_equal(fp, f[:p]) and np.array_equal(ep, e[:p])
+        assert np.array_equal(calc_field_krige(m, vp, c), f[:p])
+
+
 def test_empty_conditions_and_errors():
     _say("krige empty / errors")
     f, e = calc_field_krige_and_variance(np.zeros((0, 0)), np.zeros((0, 6)), np.zeros(0))
