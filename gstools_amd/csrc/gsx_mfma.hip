@@ -20,6 +20,8 @@
 // accumulated in FP32.
 //
 // Kernels:
+//  * k_mfma_axes: whether the row axis is its own mirror image (k_mfma_grid3 then sums
+//    cosine and sine halves, half the matrix instructions), and a 2D grid's virtual axes.
 //  * k_mfma_tables: phase factors in FP64 (sincos of the FP64 phase), A split
 //    into hi/lo 16-bit rows [i0][2Np], E1/E2 as complex FP32 rows [i][Np].
 //  * k_mfma_grid: block = 4 waves, tile = 128 rows x 256 columns; the A tile
@@ -29,6 +31,8 @@
 //    + hi/lo split), so B never touches memory.  Block -> tile mapping is
 //    XCD-aware: the blocks resident on one XCD work on one row tile of A,
 //    so that XCD's L2 holds the A rows its blocks stream.
+//  * k_mfma_grid3: the same for grids with two column axes of 16 points or more, E1 / E2
+//    staged through LDS as well.
 //
 // MFMA operand layouts (v_mfma_f32_16x16x32, 64 lanes, g = lane / 16):
 //   A: lane holds row (lane % 16), K elements 8g .. 8g+7
@@ -70,12 +74,13 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
     g.n1 = d == 3 ? shape[1] : 1;
     g.n2 = d == 3 ? shape[2] : shape[1];
     g.n0p = ceil_div(g.n0, kMBM) * kMBM;
-    g.Np = ceil_div(N, kMKM) * kMKM;
+    g.g2 = (g.n1 >= 16 && g.n2 >= 16) ? 1 : 16;
+    // k_mfma_grid3 may step 32 modes at a time
+    g.Np = g.g2 == 1 ? ceil_div(N, 2 * kMKM) * 2 * kMKM : ceil_div(N, kMKM) * kMKM;
     g.ncols = g.n1 * g.n2;
     g.out_cols = g.ncols;
     g.rs = g.ncols;
     g.c1s = g.n2;
-    g.g2 = (g.n1 >= 16 && g.n2 >= 16) ? 1 : 16;
     g.t1 = g.g2 == 1 ? ceil_div(g.n1, (int64_t)16) : 1;
     g.t2 = g.g2 == 1 ? ceil_div(g.n2, (int64_t)16) : ceil_div(g.ncols, (int64_t)256);
     g.row_tiles = g.n0p / kMBM;
@@ -102,7 +107,8 @@ inline int64_t mfma_steps_per_split(const MfmaGeom& g, int64_t comps, int64_t fi
     int64_t k = blocks >= fill ? 1 : fill / blocks;
     if (k > steps / 8) k = steps / 8;
     if (k < 1) k = 1;
-    return ceil_div(steps, k);
+    const int64_t per = ceil_div(steps, k);
+    return g.g2 == 1 ? ceil_div(per, (int64_t)2) * 2 : per;  // whole 32-mode steps
 }
 
 inline int64_t mfma_ksplit(const MfmaGeom& g, int64_t comps, int64_t fill = kMFillBlocks) {
@@ -115,11 +121,14 @@ inline int64_t mfma_table_bytes(const MfmaGeom& g, int64_t comps) {
     return 2 * g.a_elems * 2 + (g.e1_elems + comps * g.e2_elems) * 8;
 }
 
-// tables, then (K split) the FP32 partial sums, 256-byte aligned
+// the mirror flag (kMFlagBytes), tables, then (K split) the FP32 partial sums, 256-byte
+// aligned
+constexpr int64_t kMFlagBytes = 256;
+
 inline int64_t mfma_ws_bytes(const MfmaGeom& g, int64_t comps = 1, int64_t fill = kMFillBlocks) {
     const int64_t ks = mfma_ksplit(g, comps, fill);
     const int64_t tables = ceil_div(mfma_table_bytes(g, comps), (int64_t)256) * 256;
-    return ks > 1 ? tables + ks * comps * g.n0 * g.out_cols * 4 : mfma_table_bytes(g, comps);
+    return kMFlagBytes + (ks > 1 ? tables + ks * comps * g.n0 * g.out_cols * 4 : mfma_table_bytes(g, comps));
 }
 
 // A uniformly spaced last axis of a 2D grid, y_j = y_0 + j h, factorises:
@@ -153,7 +162,7 @@ inline int64_t mfma_split_ws_bytes(const MfmaGeom& gv, int64_t fill = kMFillBloc
 // about 2.2 k_mfma_grid3 tiles (512x512x8 against 512^3 per mode-point).
 struct MfmaPlan {
     MfmaGeom g;
-    bool split;    // 2D grid, uniform last axis factorised (k_split_axis)
+    bool split;    // 2D grid, uniform last axis factorised (k_mfma_axes)
     bool swapped;  // 3D grid run with axes 0 and 1 swapped
     int64_t fill;  // K-split fill target (resident blocks)
 };
@@ -225,6 +234,11 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
 // ka_row, k1_row, kz_row: the rows of cov holding the wave-vector components of A, E1
 // and E2 (0, 1, d - 1; 1, 1 for a split axis's two virtual axes; 1, 0, 2 with axes 0
 // and 1 swapped).  The projector weight always uses cov's own rows.
+//
+// *mirror != 0 (the row axis is its own mirror image, k_mfma_axes): the A entries are
+// cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, 64 of them per tile of 128
+// table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
+// thread per mode pair); E2 takes the phase of the axis's centre.
 template <bool FP16>
 __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int64_t N, int64_t comps,
                                                      int64_t ka_row, int64_t k1_row, int64_t kz_row,
@@ -235,13 +249,42 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                                                      const double* __restrict__ z1,
                                                      const double* __restrict__ z2,
                                                      const double* __restrict__ fac,
+                                                     const int* __restrict__ mirror,
                                                      uint32_t* __restrict__ a_hi,
                                                      uint32_t* __restrict__ a_lo,
                                                      float2* __restrict__ e1,
                                                      float2* __restrict__ e2) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t na = g.n0p * g.Np, n1 = g.e1_elems, n2 = comps * g.e2_elems;
-    if (t < na) {
+    const bool mir = mirror && *mirror;
+    const int64_t na = mir ? (g.n0p / 2) * (g.Np / 2) : g.n0p * g.Np;
+    const int64_t n1 = g.e1_elems, n2 = comps * g.e2_elems;
+    if (mir && t < na) {
+        const int64_t pitch = g.Np / 2;
+        const int64_t r = t / pitch, jp = t - r * pitch;
+        float c2[2] = {0.0f, 0.0f}, s2[2] = {0.0f, 0.0f};
+        if (2 * r < g.n0) {
+            const double h = 0.5 * (ax0[g.n0 - 1 - r] - ax0[r]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int64_t j = 2 * jp + e;
+                if (j < N) {
+                    double sn, cs;
+                    const double th = cov[ka_row * N + j] * h;
+                    if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &sn, &cs); else sincos(th, &sn, &cs);
+                    c2[e] = (float)cs;
+                    s2[e] = (float)sn;
+                }
+            }
+        }
+        const int64_t at = ((r / (kMBM / 2)) * kMBM + r % (kMBM / 2)) * pitch + jp;
+        uint32_t hi, lo;
+        split2<FP16>(c2[0], c2[1], hi, lo);
+        a_hi[at] = hi;
+        a_lo[at] = lo;
+        split2<FP16>(s2[0], s2[1], hi, lo);
+        a_hi[at + (kMBM / 2) * pitch] = hi;
+        a_lo[at + (kMBM / 2) * pitch] = lo;
+    } else if (t < na) {
         const int64_t row = t / g.Np, j = t - row * g.Np;
         float re = 0.0f, im = 0.0f;
         if (row < g.n0 && j < N) {
@@ -278,7 +321,8 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
         if (j < N) {
             double s, c;
             const double kz = cov[kz_row * N + j];
-            const double th = kz * (d == 3 ? ax2[i2] : ax1[i2]);
+            double th = kz * (d == 3 ? ax2[i2] : ax1[i2]);
+            if (mir) th += cov[ka_row * N + j] * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
             if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
             double f = fac ? fac[j] : 1.0;
             if (comps > 1) {
@@ -507,24 +551,35 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
 struct alignas(16) Stage3 {
     uint32_t ah[kMBM * 16];
     uint32_t al[kMBM * 16];
-    float e1[16 * 32];
-    float e2[16 * 32];
+    float e1[16 * 64];  // 16 modes per step: the first 16 * 32
+    float e2[16 * 64];
 };
 
-template <bool FP16, bool SPLIT>
-__global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, double alpha,
-                                                                const uint32_t* __restrict__ a_hi,
-                                                                const uint32_t* __restrict__ a_lo,
-                                                                const float2* __restrict__ e1,
-                                                                const float2* __restrict__ e2,
-                                                                float* __restrict__ out, int64_t out_stride,
-                                                                int64_t comps, int64_t steps_per,
-                                                                float* __restrict__ partial) {
-    // two stages as separate LDS objects, the step loop unrolled by two: the compiler
-    // then sees that a step's LDS reads and the next step's global -> LDS loads touch
-    // different objects and does not wait for those loads before the reads
-    __shared__ Stage3 st0;
-    __shared__ Stage3 st1;
+// MIRROR: the row axis is its own mirror image about x_c (every regular axis), so with
+// h_r = x_(n0-1-r) - x_c >= 0 and c'_j the centre-shifted column factors
+//   u(x_c + h_r) = C - S,  u(x_c - h_r) = C + S,
+//   C = sum_j Re c'_j cos k_j h_r,  S = sum_j Im c'_j sin k_j h_r:
+// one real product of K = N for each of C and S over half the rows, instead of one of
+// K = 2N over all: half the matrix instructions.  The tile's first 64 A rows are the
+// cosines (times the real parts of B), its last 64 the sines (times the imaginary parts);
+// a K step is 32 modes, so A stage, accumulators and instructions per step stay as they are
+// and only the B fragments double (two of 32 modes in place of one of 16).
+// 512^3, N = 4096, bf16: 4.40 -> 2.77 ms a call; 3 x 128^3, N = 4096: 336 -> 259 us.
+// What bounds it now: a stream of matrix instructions leaves the SIMD's other wave hardly any
+// vector issue slots, so the 320 vector instructions that build the B fragments of a step
+// add to its 96 matrix instructions (1604 of 2288 cycles per wave and step).  Building half of
+// them between the products, priorities and v_dot2 for the remainders gained nothing or lost.
+template <bool FP16, bool SPLIT, bool MIRROR>
+__device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const MfmaGeom& g, double alpha,
+                                                const uint32_t* __restrict__ a_hi,
+                                                const uint32_t* __restrict__ a_lo,
+                                                const float2* __restrict__ e1, const float2* __restrict__ e2,
+                                                float* __restrict__ out, int64_t out_stride, int64_t comps,
+                                                int64_t steps_per, float* __restrict__ partial) {
+    constexpr int kStep = MIRROR ? 2 * kMKM : kMKM;  // modes per K step
+    constexpr int kEP = kStep * 2;                   // floats per E row of a stage
+    constexpr int kECh = kEP / 4;                    // 16-byte chunks per E row
+    const int64_t apitch = MIRROR ? g.Np / 2 : g.Np;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -556,11 +611,11 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
 
     // each K step, each thread fills two 16-byte LDS slots of the A tile (hi and lo: slots
     // tid and tid + 256, row q >> 2) and one of E: threads 0..127 -> E1, 128..255 -> E2
-    // (row (tid & 127) >> 3)
-    const int erow = (tid & 127) >> 3;
+    // (row (tid & 127) >> 3); 32 modes per step: one of E1 and one of E2 (row tid >> 4)
+    const int erow = MIRROR ? tid >> 4 : (tid & 127) >> 3;
     const bool is_e1 = tid < 128;
-    const int64_t eidx = is_e1 ? (i1b + erow < g.n1 ? i1b + erow : g.n1 - 1)
-                               : (i2b + erow < g.n2 ? i2b + erow : g.n2 - 1);
+    const int64_t i1e = i1b + erow < g.n1 ? i1b + erow : g.n1 - 1;
+    const int64_t i2e = i2b + erow < g.n2 ? i2b + erow : g.n2 - 1;
     // global -> LDS loads: lane l of an instruction writes 16 B at the wave's LDS base + 16 l,
     // so each lane fetches the global chunk that the swizzled layout puts at its LDS slot
     const int wv = __builtin_amdgcn_readfirstlane(wave);
@@ -569,9 +624,11 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
     for (int h = 0; h < 2; ++h) {
         const int q = h * 256 + wv * 64 + lane;
         const int r = q >> 2;
-        aoff[h] = (row0 + r) * g.Np + (((q & 3) ^ ((r >> 1) & 3)) * 4);
+        aoff[h] = (row0 + r) * apitch + (((q & 3) ^ ((r >> 1) & 3)) * 4);
     }
-    const float2* ebase = (is_e1 ? e1 : e2) + eidx * g.Np + (((tid & 7) ^ (erow & 7)) * 2);
+    const int echunk = ((tid & (kECh - 1)) ^ (erow & 7)) * 2;
+    const float2* ebase = (MIRROR || is_e1) ? e1 + i1e * g.Np + echunk : e2 + i2e * g.Np + echunk;
+    const float2* ebase2 = e2 + i2e * g.Np + echunk;  // MIRROR only
     auto load = [&](int64_t step, Stage3& S) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -581,9 +638,12 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
             __builtin_amdgcn_global_load_lds((const void*)(a_lo + aoff[h] + step * kMKM),
                                              (__attribute__((address_space(3))) void*)&S.al[slot], 16, 0, 0);
         }
-        float* es = (wv < 2 ? S.e1 : S.e2) + (wv & 1) * 256;
-        __builtin_amdgcn_global_load_lds((const void*)(ebase + step * kMKM),
+        float* es = MIRROR ? S.e1 + wv * 256 : (wv < 2 ? S.e1 : S.e2) + (wv & 1) * 256;
+        __builtin_amdgcn_global_load_lds((const void*)(ebase + step * kStep),
                                          (__attribute__((address_space(3))) void*)es, 16, 0, 0);
+        if constexpr (MIRROR)
+            __builtin_amdgcn_global_load_lds((const void*)(ebase2 + step * kStep),
+                                             (__attribute__((address_space(3))) void*)(S.e2 + wv * 256), 16, 0, 0);
     };
 
     f32x4 acc[kMRF][kMCF];
@@ -592,9 +652,10 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
 #pragma unroll
         for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int64_t steps = g.Np / kMKM;
-    const int64_t s0 = SPLIT ? split * steps_per : 0;
-    const int64_t s1 = SPLIT ? (s0 + steps_per < steps ? s0 + steps_per : steps) : steps;
+    const int64_t steps = g.Np / kStep;
+    const int64_t per = MIRROR ? steps_per / 2 : steps_per;  // steps_per: even, in steps of 16 modes
+    const int64_t s0 = SPLIT ? split * per : 0;
+    const int64_t s1 = SPLIT ? (s0 + per < steps ? s0 + per : steps) : steps;
     load(s0, st0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -602,48 +663,86 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
     // one K step on stage C while stage Nx receives the next step's tiles
     auto step = [&](const Stage3& C, Stage3& Nx, int64_t s) {
         if (s + 1 < s1) load(s + 1, Nx);
-        // B fragments: E2 of this lane's i2 (row l16) times E1 of each fragment's i1
-        float2 zf[4];
-        {
-            const float* zr = C.e2 + l16 * 32;
-            const float4 q0 = *reinterpret_cast<const float4*>(zr + (((2 * grp) ^ zsw) * 4));
-            const float4 q1 = *reinterpret_cast<const float4*>(zr + (((2 * grp + 1) ^ zsw) * 4));
-            zf[0] = {q0.x, q0.y};
-            zf[1] = {q0.z, q0.w};
-            zf[2] = {q1.x, q1.y};
-            zf[3] = {q1.z, q1.w};
+        // B fragments: E2 of this lane's i2 (row l16) times E1 of each fragment's i1; lane
+        // group grp takes modes kQ grp ... of the step (a fragment's K elements 8 grp ...: the
+        // re / im pairs of 4 modes, or one part of 8)
+        constexpr int kQ = kStep / 4;
+        // A fragments of row fragment rf, read one row fragment ahead of their use (the first
+        // before the B fragments are built), so that no product waits for LDS
+        const int asw = (l16 >> 1) & 3;
+        u32x4 ah[2], al[2];
+        auto read_a = [&](int rf) {
+            const int pos = (rf * 16 + l16) * 16 + ((grp ^ asw) * 4);
+            ah[rf & 1] = *reinterpret_cast<const u32x4*>(&C.ah[pos]);
+            al[rf & 1] = *reinterpret_cast<const u32x4*>(&C.al[pos]);
+        };
+        // chunk kQ/2 grp + q of a row sits at slot kECh/4 (grp ^ hi) + (q ^ lo), hi and lo the
+        // high and low bits of the row's swizzle: the E1 rows of a wave differ in constants only.
+        // E1 is read two column fragments ahead of its use.
+        constexpr int kLoBits = MIRROR ? 2 : 1;
+        const float* zr = C.e2 + l16 * kEP + (grp ^ (zsw >> kLoBits)) * (2 * kQ);
+        const int zlo = zsw & ((1 << kLoBits) - 1);
+        float2 zf[kQ], yf[kMCF][kQ];
+#pragma unroll
+        for (int q = 0; q < kQ / 2; ++q) {
+            const float4 v = *reinterpret_cast<const float4*>(zr + ((q ^ zlo) * 4));
+            zf[2 * q] = {v.x, v.y};
+            zf[2 * q + 1] = {v.z, v.w};
         }
-        u32x4 bh[kMCF], bl[kMCF];
+        auto read_y = [&](int cf) {
+            // row er = 4 wave + cf, swizzle er & 7 = 4 (wave & 1) + cf
+            const float* yr = C.e1 + (wave * kMCF + cf) * kEP +
+                              (MIRROR ? (grp ^ (wave & 1)) : (grp ^ ((wave & 1) * 2 + (cf >> 1)))) * (2 * kQ);
+#pragma unroll
+            for (int q = 0; q < kQ / 2; ++q) {
+                const float4 v = *reinterpret_cast<const float4*>(yr + ((q ^ (cf & ((1 << kLoBits) - 1))) * 4));
+                yf[cf][2 * q] = {v.x, v.y};
+                yf[cf][2 * q + 1] = {v.z, v.w};
+            }
+        };
+        read_y(0);
+        read_y(1);
+
+        // fragments [real, imaginary parts][column fragment]; without MIRROR one of the pairs
+        constexpr int kParts = MIRROR ? 2 : 1;
+        u32x4 bh[kParts][kMCF], bl[kParts][kMCF];
 #pragma unroll
         for (int cf = 0; cf < kMCF; ++cf) {
-            const int er = wave * kMCF + cf;
-            const int ysw = er & 7;
-            const float* yr = C.e1 + er * 32;
-            const float4 q0 = *reinterpret_cast<const float4*>(yr + (((2 * grp) ^ ysw) * 4));
-            const float4 q1 = *reinterpret_cast<const float4*>(yr + (((2 * grp + 1) ^ ysw) * 4));
-            const float2 yf[4] = {{q0.x, q0.y}, {q0.z, q0.w}, {q1.x, q1.y}, {q1.z, q1.w}};
-            uint32_t h4[4], l4[4];
+            __builtin_amdgcn_sched_barrier(0);
+            if (cf + 2 < kMCF) read_y(cf + 2);
+            if (cf + 2 == kMCF) read_a(0);
+            uint32_t h, l;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const float2 v = cmul(yf[t], zf[t]);
-                split2<FP16>(v.x, v.y, h4[t], l4[t]);
+                if constexpr (MIRROR) {
+                    const float2 v = cmul(yf[cf][2 * t], zf[2 * t]), w = cmul(yf[cf][2 * t + 1], zf[2 * t + 1]);
+                    split2<FP16>(v.x, w.x, h, l);
+                    bh[0][cf][t] = h;
+                    bl[0][cf][t] = l;
+                    split2<FP16>(v.y, w.y, h, l);
+                    bh[1][cf][t] = h;
+                    bl[1][cf][t] = l;
+                } else {
+                    const float2 v = cmul(yf[cf][t], zf[t]);
+                    split2<FP16>(v.x, v.y, h, l);
+                    bh[0][cf][t] = h;
+                    bl[0][cf][t] = l;
+                }
             }
-            bh[cf] = u32x4{h4[0], h4[1], h4[2], h4[3]};
-            bl[cf] = u32x4{l4[0], l4[1], l4[2], l4[3]};
         }
 
-        const int asw = (l16 >> 1) & 3;
 #pragma unroll
         for (int rf = 0; rf < kMRF; ++rf) {
-            const int pos = (rf * 16 + l16) * 16 + ((grp ^ asw) * 4);
-            const u32x4 ah = *reinterpret_cast<const u32x4*>(&C.ah[pos]);
-            const u32x4 al = *reinterpret_cast<const u32x4*>(&C.al[pos]);
+            const int part = MIRROR && rf >= kMRF / 2 ? 1 : 0;
+            if (rf + 1 < kMRF) read_a(rf + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            // the products of one accumulator lie kMCF instructions apart
 #pragma unroll
-            for (int cf = 0; cf < kMCF; ++cf) {
-                acc[rf][cf] = mfma<FP16>(ah, bh[cf], acc[rf][cf]);
-                acc[rf][cf] = mfma<FP16>(ah, bl[cf], acc[rf][cf]);
-                acc[rf][cf] = mfma<FP16>(al, bh[cf], acc[rf][cf]);
-            }
+            for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = mfma<FP16>(ah[rf & 1], bh[part][cf], acc[rf][cf]);
+#pragma unroll
+            for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = mfma<FP16>(ah[rf & 1], bl[part][cf], acc[rf][cf]);
+#pragma unroll
+            for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = mfma<FP16>(al[rf & 1], bh[part][cf], acc[rf][cf]);
         }
         // the next step's LDS loads have landed (the barrier's own wait covers LDS, not them)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -662,15 +761,51 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
         if (i1 >= g.n1 || i2 >= g.n2) continue;
         if (i1 * g.n2 + i2 >= g.out_cols) continue;  // past the end of a split axis
         const int64_t col = i1 * g.c1s + i2;
+        if constexpr (MIRROR) {
 #pragma unroll
-        for (int rf = 0; rf < kMRF; ++rf) {
+            for (int rf = 0; rf < kMRF / 2; ++rf) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int64_t row = row0 + rf * 16 + grp * 4 + i;
-                if (row < g.n0) out[row * g.rs + col] = fa * acc[rf][cf][i];
+                for (int i = 0; i < 4; ++i) {
+                    const int64_t row = rt * (kMBM / 2) + rf * 16 + grp * 4 + i;
+                    const float c = acc[rf][cf][i], sn = acc[rf + kMRF / 2][cf][i];
+                    if (2 * row < g.n0) out[row * g.rs + col] = fa * (c + sn);
+                    if (2 * row + 1 < g.n0) out[(g.n0 - 1 - row) * g.rs + col] = fa * (c - sn);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int rf = 0; rf < kMRF; ++rf) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int64_t row = row0 + rf * 16 + grp * 4 + i;
+                    if (row < g.n0) out[row * g.rs + col] = fa * acc[rf][cf][i];
+                }
             }
         }
     }
+}
+
+template <bool FP16, bool SPLIT>
+__global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, double alpha,
+                                                                const int* __restrict__ mirror,
+                                                                const uint32_t* __restrict__ a_hi,
+                                                                const uint32_t* __restrict__ a_lo,
+                                                                const float2* __restrict__ e1,
+                                                                const float2* __restrict__ e2,
+                                                                float* __restrict__ out, int64_t out_stride,
+                                                                int64_t comps, int64_t steps_per,
+                                                                float* __restrict__ partial) {
+    // two stages as separate LDS objects, the step loop unrolled by two: the compiler
+    // then sees that a step's LDS reads and the next step's global -> LDS loads touch
+    // different objects and does not wait for those loads before the reads
+    __shared__ Stage3 st0;
+    __shared__ Stage3 st1;
+    if (*mirror)  // one value for the launch
+        mfma_grid3_tile<FP16, SPLIT, true>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
+                                           steps_per, partial);
+    else
+        mfma_grid3_tile<FP16, SPLIT, false>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
+                                            steps_per, partial);
 }
 
 // out[i] = alpha * sum_k partial[k * n + i], k in order (K-split partial sums)
@@ -688,35 +823,60 @@ __global__ void k_fill_zero_f32(float* __restrict__ p, int64_t n) {
     if (i < n) p[i] = 0.0f;
 }
 
-// Virtual axes of a split last axis (one block): vy[a] = y[16a], vz[b] = y[b] - y[0].
+// What the grid's axes allow (one block).
+//
+// *mirror: whether the row axis x (n0 points) is its own mirror image, x_r + x_(n0-1-r) ==
+// x_0 + x_(n0-1) to 4 ulp of max(|x_0|, |x_(n0-1)|) for every r (a NaN or infinity: no).
+// Half the matrix work of k_mfma_grid3 hangs on it, so it is looked up here, on the
+// device, for every caller; past kMMirrorMax points the look itself would take longer than
+// some of the grids, and the axis counts as not mirrored (n0 = 0 from the host).
+//
+// Virtual axes of a split last axis y (n > 0 points): vy[a] = y[16a], vz[b] = y[b] - y[0].
 // Checks y[j] == y[16 floor(j/16)] + (y[j mod 16] - y[0]) to 4 ulp of max|y| for every
 // j (the same FP64 operations as the host's check); any miss (or a NaN) makes every vy
 // NaN, so the whole output is NaN rather than a wrong field.
-__global__ __launch_bounds__(256) void k_split_axis(const double* __restrict__ y, int64_t n,
-                                                    double* __restrict__ vy, double* __restrict__ vz) {
-    __shared__ double s_max[256];
-    __shared__ int s_bad;
+constexpr int64_t kMMirrorMax = 32768;
+constexpr int kMAxesThreads = 512;
+
+__global__ __launch_bounds__(kMAxesThreads) void k_mfma_axes(const double* __restrict__ x, int64_t n0,
+                                                             int* __restrict__ mirror,
+                                                             const double* __restrict__ y, int64_t n,
+                                                             double* __restrict__ vy, double* __restrict__ vz) {
+    __shared__ double s_max[kMAxesThreads];
+    __shared__ int s_bad, s_odd;
     const int t = threadIdx.x;
     double m = 0.0;
-    for (int64_t j = t; j < n; j += 256) m = fmax(m, fabs(y[j]));
+    for (int64_t j = t; j < n; j += kMAxesThreads) m = fmax(m, fabs(y[j]));
     s_max[t] = m;
-    if (t == 0) s_bad = 0;
+    if (t == 0) {
+        s_bad = 0;
+        s_odd = n0 > 0 ? 0 : 1;
+    }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
+    if (n0 > 0) {
+        const double ends = x[0] + x[n0 - 1], tol = 0x1p-50 * fmax(fabs(x[0]), fabs(x[n0 - 1]));
+        bool odd = false;
+        for (int64_t r = t; 2 * r < n0; r += kMAxesThreads)
+            if (!(fabs((x[r] + x[n0 - 1 - r]) - ends) <= tol)) odd = true;
+        if (odd) s_odd = 1;
+    }
+    for (int w = kMAxesThreads / 2; w > 0; w >>= 1) {
         if (t < w) s_max[t] = fmax(s_max[t], s_max[t + w]);
         __syncthreads();
     }
+    if (t == 0) *mirror = s_odd ? 0 : 1;
+    if (n == 0) return;  // whole block
     const double tol = 0x1p-50 * s_max[0];
     const double y0 = y[0];
     bool bad = false;
-    for (int64_t j = t; j < n; j += 256) {
+    for (int64_t j = t; j < n; j += kMAxesThreads) {
         const double r = y[j & ~(int64_t)15] + (y[j & 15] - y0);
         if (!(fabs(y[j] - r) <= tol)) bad = true;
     }
     if (bad) s_bad = 1;
     __syncthreads();
     const double poison = s_bad ? __builtin_nan("") : 0.0;
-    for (int64_t a = t; a < (n + 15) / 16; a += 256) vy[a] = y[16 * a] + poison;
+    for (int64_t a = t; a < (n + 15) / 16; a += kMAxesThreads) vy[a] = y[16 * a] + poison;
     if (t < 16) vz[t] = y[t] - y0;
 }
 
@@ -724,14 +884,15 @@ template <bool FP16>
 int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t comps, int64_t ka_row, int64_t k1_row,
                 int64_t kz_row, const double* ax0,
                 const double* ax1, const double* ax2, const double* cov, const double* z1, const double* z2,
-                const double* fac, double alpha, float* out, void* ws, hipStream_t s) {
+                const double* fac, double alpha, float* out, const int* mirror, void* ws, hipStream_t s) {
     uint32_t* a_hi = static_cast<uint32_t*>(ws);
     uint32_t* a_lo = a_hi + g.a_elems / 2;
     float2* e1 = reinterpret_cast<float2*>(a_lo + g.a_elems / 2);
     float2* e2 = e1 + g.e1_elems;
     const int64_t entries = g.n0p * g.Np + g.e1_elems + comps * g.e2_elems;
     hipLaunchKernelGGL((k_mfma_tables<FP16>), dim3((unsigned)ceil_div(entries, 256)), dim3(256), 0, s, g, d,
-                       N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, a_hi, a_lo, e1, e2);
+                       N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, mirror, a_hi, a_lo, e1,
+                       e2);
     int st = launch_status();
     if (st != GSX_OK) return st;
     const int64_t steps_per = mfma_steps_per_split(g, comps, fill);
@@ -745,11 +906,11 @@ int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t c
     const dim3 grid((unsigned)blocks), block(kMWaves * 64);
     if (g.g2 == 1) {
         if (ksplit > 1)
-            hipLaunchKernelGGL((k_mfma_grid3<FP16, true>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2, out,
+            hipLaunchKernelGGL((k_mfma_grid3<FP16, true>), grid, block, 0, s, g, alpha, mirror, a_hi, a_lo, e1, e2, out,
                                stride, comps, steps_per, partial);
         else
-            hipLaunchKernelGGL((k_mfma_grid3<FP16, false>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2, out,
-                               stride, comps, steps_per, partial);
+            hipLaunchKernelGGL((k_mfma_grid3<FP16, false>), grid, block, 0, s, g, alpha, mirror, a_hi, a_lo, e1, e2,
+                               out, stride, comps, steps_per, partial);
     } else if (d == 2) {
         if (ksplit > 1)
             hipLaunchKernelGGL((k_mfma_grid<FP16, true, true>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2,
@@ -816,23 +977,32 @@ int mfma_entry(int64_t d, int64_t N, const int64_t* shape, const double* axes, c
         ka_row = 1;
         k1_row = 0;
     }
-    if (split) {
-        double* vy = reinterpret_cast<double*>(static_cast<char*>(workspace) +
-                                               ceil_div(mfma_ws_bytes(g, 1, fill), (int64_t)256) * 256);
-        double* vz = vy + g.n1;
-        hipLaunchKernelGGL(k_split_axis, dim3(1), dim3(256), 0, s, ax1, shape[1], vy, vz);
+    int* mirror = nullptr;
+    if (g.g2 == 1) {  // k_mfma_grid3
+        mirror = static_cast<int*>(workspace);
+        double *vy = nullptr, *vz = nullptr;
+        if (split) {
+            vy = reinterpret_cast<double*>(static_cast<char*>(workspace) +
+                                           ceil_div(mfma_ws_bytes(g, 1, fill), (int64_t)256) * 256);
+            vz = vy + g.n1;
+        }
+        hipLaunchKernelGGL(k_mfma_axes, dim3(1), dim3(kMAxesThreads), 0, s, ax0, g.n0 <= kMMirrorMax ? g.n0 : 0,
+                           mirror, ax1, split ? shape[1] : (int64_t)0, vy, vz);
         const int st = launch_status();
         if (st != GSX_OK) return st;
-        ax1 = vy;
-        ax2 = vz;
-        dk = 3;      // tables of the 3D form
-        kz_row = 1;  // both virtual axes carry the mode's k_1
+        if (split) {
+            ax1 = vy;
+            ax2 = vz;
+            dk = 3;      // tables of the 3D form
+            kz_row = 1;  // both virtual axes carry the mode's k_1
+        }
     }
+    void* tables = static_cast<char*>(workspace) + kMFlagBytes;
     if (variant == GSX_MFMA_FP16X3)
         return mfma_launch<true>(g, fill, dk, N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac,
-                                 alpha, out, workspace, s);
+                                 alpha, out, mirror, tables, s);
     return mfma_launch<false>(g, fill, dk, N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac,
-                              alpha, out, workspace, s);
+                              alpha, out, mirror, tables, s);
 }
 
 }  // namespace gsx

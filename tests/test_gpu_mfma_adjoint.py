@@ -27,7 +27,7 @@ from gstools_amd import (Gaussian, Matern, RandMeth, _native, summate_adjoint_de
                          summate_grid_device)
 from gstools_amd.autograd import RandMethSum, randmeth_field
 from gstools_amd.geometry import generate_grid
-from gstools_amd.summate import uniform_axis
+from gstools_amd.summate import summate_incompr_grid_device, uniform_axis
 
 pytestmark = pytest.mark.gpu
 
@@ -127,6 +127,38 @@ def test_mfma_uniform_last_axis(shape, n):
             else:
                 assert rel_rms <= 1e-5 and rel_max <= 5e-5
         assert not np.array_equal(split, plain)  # the two forms round differently
+
+
+@pytest.mark.parametrize("shape,n,comps", [
+    ((1, 17, 16), 31, 1), ((2, 16, 33), 32, 1), ((3, 16, 16), 33, 3), ((64, 18, 20), 100, 1), ((65, 16, 17), 65, 1),
+    ((127, 16, 16), 64, 3), ((128, 17, 16), 40, 1), ((129, 16, 19), 300, 1), ((33, 260), 70, 1), ((258, 257), 129, 1),
+])
+def test_mfma_mirrored_row_axis(shape, n, comps):
+    """A row axis that is its own mirror image is summed over half its rows (cosine and sine
+    halves); moved off by 1e-9 at one point it takes the general form, as do NaN axes.  Both
+    within the split precision's bars of the FP64 sum, at row counts around the 64-row half
+    tiles, odd and even, and mode counts around the 32-mode steps."""
+    _say(f"mfma mirror shape={shape} N={n} comps={comps}")
+    d = len(shape)
+    cov, z1, z2 = _modes(d, n, 300 + n, kscale=0.6)
+    axes = [np.arange(s) * 0.25 - 2.0 * i - 3.0 for i, s in enumerate(shape)]
+    odd = [axes[0].copy()] + axes[1:]
+    odd[0][len(odd[0]) // 3] += 1e-9
+    fn = summate_incompr_grid_device if comps > 1 else summate_grid_device
+    for precision in ("fp16x3", "bf16x3"):
+        outs = []
+        for ax in (axes, odd):
+            ref = fn(cov, z1, z2, ax, "fp64").cpu().numpy().ravel()
+            got = fn(cov, z1, z2, ax, precision).cpu().numpy().astype(np.float64).ravel()
+            rel_max, rel_rms = oracle.rel_errors(got, ref)
+            _say(f"  {precision} rel_max={rel_max:.3e} rel_rms={rel_rms:.3e}")
+            assert rel_rms <= 1e-5 and rel_max <= (1e-5 if precision == "fp16x3" else 5e-5)
+            outs.append(got)
+        if shape[0] > 2:  # shorter axes are mirrored whatever their points
+            assert not np.array_equal(outs[0], outs[1])
+    bad = [axes[0].copy()] + axes[1:]
+    bad[0][0] = np.nan
+    assert np.isnan(fn(cov, z1, z2, bad, "bf16x3").cpu().numpy().reshape(comps, -1)[:, 0]).all()
 
 
 def test_mfma_uniform_flag_checked_and_ignored():
