@@ -20,8 +20,6 @@
 // accumulated in FP32.
 //
 // Kernels:
-//  * k_mfma_axes: whether the row axis is its own mirror image (k_mfma_grid3 then sums
-//    cosine and sine halves, half the matrix instructions), and a 2D grid's virtual axes.
 //  * k_mfma_tables: phase factors in FP64 (sincos of the FP64 phase), A split
 //    into hi/lo 16-bit rows [i0][2Np], E1/E2 as complex FP32 rows [i][Np].
 //  * k_mfma_grid: block = 4 waves, tile = 128 rows x 256 columns; the A tile
@@ -32,7 +30,8 @@
 //    XCD-aware: the blocks resident on one XCD work on one row tile of A,
 //    so that XCD's L2 holds the A rows its blocks stream.
 //  * k_mfma_grid3: the same for grids with two column axes of 16 points or more, E1 / E2
-//    staged through LDS as well.
+//    staged through LDS as well, and half the matrix instructions where the row axis is its
+//    own mirror image.
 //
 // MFMA operand layouts (v_mfma_f32_16x16x32, 64 lanes, g = lane / 16):
 //   A: lane holds row (lane % 16), K elements 8g .. 8g+7
@@ -121,14 +120,11 @@ inline int64_t mfma_table_bytes(const MfmaGeom& g, int64_t comps) {
     return 2 * g.a_elems * 2 + (g.e1_elems + comps * g.e2_elems) * 8;
 }
 
-// the mirror flag (kMFlagBytes), tables, then (K split) the FP32 partial sums, 256-byte
-// aligned
-constexpr int64_t kMFlagBytes = 256;
-
+// tables, then (K split) the FP32 partial sums, 256-byte aligned
 inline int64_t mfma_ws_bytes(const MfmaGeom& g, int64_t comps = 1, int64_t fill = kMFillBlocks) {
     const int64_t ks = mfma_ksplit(g, comps, fill);
     const int64_t tables = ceil_div(mfma_table_bytes(g, comps), (int64_t)256) * 256;
-    return kMFlagBytes + (ks > 1 ? tables + ks * comps * g.n0 * g.out_cols * 4 : mfma_table_bytes(g, comps));
+    return ks > 1 ? tables + ks * comps * g.n0 * g.out_cols * 4 : mfma_table_bytes(g, comps);
 }
 
 // A uniformly spaced last axis of a 2D grid, y_j = y_0 + j h, factorises:
@@ -162,7 +158,7 @@ inline int64_t mfma_split_ws_bytes(const MfmaGeom& gv, int64_t fill = kMFillBloc
 // about 2.2 k_mfma_grid3 tiles (512x512x8 against 512^3 per mode-point).
 struct MfmaPlan {
     MfmaGeom g;
-    bool split;    // 2D grid, uniform last axis factorised (k_mfma_axes)
+    bool split;    // 2D grid, uniform last axis factorised (k_split_axis)
     bool swapped;  // 3D grid run with axes 0 and 1 swapped
     int64_t fill;  // K-split fill target (resident blocks)
 };
@@ -226,6 +222,26 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
     }
 }
 
+// ---------------------------------------------------------------- mirror ---
+// Whether the row axis x (n0 points) is its own mirror image, x_r + x_(n0-1-r) == x_0 +
+// x_(n0-1) to 4 ulp of max(|x_0|, |x_(n0-1)|) for every r (a NaN or infinity: no).  Every
+// block of the tables and of k_mfma_grid3 looks for itself (about a microsecond for 512
+// points, less than a launch to look once); longer axes than kMMirrorMax count as not
+// mirrored.  Called by the whole block.
+constexpr int64_t kMMirrorMax = 4096;
+
+__device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int64_t n0) {
+    if (n0 > kMMirrorMax) return false;
+    // the ends and the first pair are read together (one round trip for up to 512 points)
+    const int64_t r0 = 2 * (int64_t)threadIdx.x < n0 ? threadIdx.x : 0;
+    const double first = x[0], last = x[n0 - 1], a = x[r0], b = x[n0 - 1 - r0];
+    const double ends = first + last, tol = 0x1p-50 * fmax(fabs(first), fabs(last));
+    int odd = !(fabs((a + b) - ends) <= tol);
+    for (int64_t r = r0 + blockDim.x; 2 * r < n0; r += blockDim.x)
+        if (!(fabs((x[r] + x[n0 - 1 - r]) - ends) <= tol)) odd = 1;
+    return !__syncthreads_or(odd);
+}
+
 // --------------------------------------------------------------- tables ----
 // One thread per table entry: A (n0p x Np), E1 (n1 x Np), E2 (comps x n2 x Np).
 // comps > 1 (incompressible fields): E2 of component c carries the projector
@@ -235,10 +251,13 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
 // and E2 (0, 1, d - 1; 1, 1 for a split axis's two virtual axes; 1, 0, 2 with axes 0
 // and 1 swapped).  The projector weight always uses cov's own rows.
 //
-// *mirror != 0 (the row axis is its own mirror image, k_mfma_axes): the A entries are
+// The row axis its own mirror image (and k_mfma_grid3 to follow): the A entries are
 // cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, 64 of them per tile of 128
 // table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
-// thread per mode pair); E2 takes the phase of the axis's centre.
+// thread per mode pair); E2 takes the phase of the axis's centre.  At most kMTableBlocks
+// blocks, so that the look at the axis is not repeated for every 256 entries.
+constexpr int64_t kMTableBlocks = 4096;
+
 template <bool FP16>
 __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int64_t N, int64_t comps,
                                                      int64_t ka_row, int64_t k1_row, int64_t kz_row,
@@ -249,92 +268,92 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                                                      const double* __restrict__ z1,
                                                      const double* __restrict__ z2,
                                                      const double* __restrict__ fac,
-                                                     const int* __restrict__ mirror,
                                                      uint32_t* __restrict__ a_hi,
                                                      uint32_t* __restrict__ a_lo,
                                                      float2* __restrict__ e1,
                                                      float2* __restrict__ e2) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool mir = mirror && *mirror;
+    const bool mir = g.g2 == 1 && mirrored_axis(ax0, g.n0);
     const int64_t na = mir ? (g.n0p / 2) * (g.Np / 2) : g.n0p * g.Np;
     const int64_t n1 = g.e1_elems, n2 = comps * g.e2_elems;
-    if (mir && t < na) {
-        const int64_t pitch = g.Np / 2;
-        const int64_t r = t / pitch, jp = t - r * pitch;
-        float c2[2] = {0.0f, 0.0f}, s2[2] = {0.0f, 0.0f};
-        if (2 * r < g.n0) {
-            const double h = 0.5 * (ax0[g.n0 - 1 - r] - ax0[r]);
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < na + n1 + n2; t += (int64_t)gridDim.x * 256) {
+        if (mir && t < na) {
+            const int64_t pitch = g.Np / 2;
+            const int64_t r = t / pitch, jp = t - r * pitch;
+            float c2[2] = {0.0f, 0.0f}, s2[2] = {0.0f, 0.0f};
+            if (2 * r < g.n0) {
+                const double h = 0.5 * (ax0[g.n0 - 1 - r] - ax0[r]);
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int64_t j = 2 * jp + e;
-                if (j < N) {
-                    double sn, cs;
-                    const double th = cov[ka_row * N + j] * h;
-                    if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &sn, &cs); else sincos(th, &sn, &cs);
-                    c2[e] = (float)cs;
-                    s2[e] = (float)sn;
+                for (int e = 0; e < 2; ++e) {
+                    const int64_t j = 2 * jp + e;
+                    if (j < N) {
+                        double sn, cs;
+                        const double th = cov[ka_row * N + j] * h;
+                        if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &sn, &cs); else sincos(th, &sn, &cs);
+                        c2[e] = (float)cs;
+                        s2[e] = (float)sn;
+                    }
                 }
             }
-        }
-        const int64_t at = ((r / (kMBM / 2)) * kMBM + r % (kMBM / 2)) * pitch + jp;
-        uint32_t hi, lo;
-        split2<FP16>(c2[0], c2[1], hi, lo);
-        a_hi[at] = hi;
-        a_lo[at] = lo;
-        split2<FP16>(s2[0], s2[1], hi, lo);
-        a_hi[at + (kMBM / 2) * pitch] = hi;
-        a_lo[at + (kMBM / 2) * pitch] = lo;
-    } else if (t < na) {
-        const int64_t row = t / g.Np, j = t - row * g.Np;
-        float re = 0.0f, im = 0.0f;
-        if (row < g.n0 && j < N) {
-            double s, c;
-            const double th = cov[ka_row * N + j] * ax0[row];
-            if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
-            re = (float)c;
-            im = (float)(-s);
-        }
-        uint32_t hi, lo;
-        split2<FP16>(re, im, hi, lo);
-        a_hi[t] = hi;  // element pair (2j, 2j+1) of row `row`
-        a_lo[t] = lo;
-    } else if (t < na + n1) {
-        const int64_t u = t - na;
-        const int64_t i1 = u / g.Np, j = u - i1 * g.Np;
-        float2 v = {0.0f, 0.0f};
-        if (j < N) {
-            if (d == 3) {
+            const int64_t at = ((r / (kMBM / 2)) * kMBM + r % (kMBM / 2)) * pitch + jp;
+            uint32_t hi, lo;
+            split2<FP16>(c2[0], c2[1], hi, lo);
+            a_hi[at] = hi;
+            a_lo[at] = lo;
+            split2<FP16>(s2[0], s2[1], hi, lo);
+            a_hi[at + (kMBM / 2) * pitch] = hi;
+            a_lo[at + (kMBM / 2) * pitch] = lo;
+        } else if (t < na) {
+            const int64_t row = t / g.Np, j = t - row * g.Np;
+            float re = 0.0f, im = 0.0f;
+            if (row < g.n0 && j < N) {
                 double s, c;
-                const double th = cov[k1_row * N + j] * ax1[i1];
+                const double th = cov[ka_row * N + j] * ax0[row];
                 if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
-                v = {(float)c, (float)s};
-            } else {
-                v = {1.0f, 0.0f};
+                re = (float)c;
+                im = (float)(-s);
             }
-        }
-        e1[u] = v;
-    } else if (t < na + n1 + n2) {
-        const int64_t u = t - na - n1;
-        const int64_t comp = u / g.e2_elems, uc = u - comp * g.e2_elems;
-        const int64_t i2 = uc / g.Np, j = uc - i2 * g.Np;
-        float2 v = {0.0f, 0.0f};
-        if (j < N) {
-            double s, c;
-            const double kz = cov[kz_row * N + j];
-            double th = kz * (d == 3 ? ax2[i2] : ax1[i2]);
-            if (mir) th += cov[ka_row * N + j] * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
-            if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
-            double f = fac ? fac[j] : 1.0;
-            if (comps > 1) {
-                double k2 = 0.0;
-                for (int64_t e = 0; e < d; ++e) k2 += cov[e * N + j] * cov[e * N + j];
-                f = (comp == 0 ? 1.0 : 0.0) - cov[comp * N + j] * cov[j] / k2;
+            uint32_t hi, lo;
+            split2<FP16>(re, im, hi, lo);
+            a_hi[t] = hi;  // element pair (2j, 2j+1) of row `row`
+            a_lo[t] = lo;
+        } else if (t < na + n1) {
+            const int64_t u = t - na;
+            const int64_t i1 = u / g.Np, j = u - i1 * g.Np;
+            float2 v = {0.0f, 0.0f};
+            if (j < N) {
+                if (d == 3) {
+                    double s, c;
+                    const double th = cov[k1_row * N + j] * ax1[i1];
+                    if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
+                    v = {(float)c, (float)s};
+                } else {
+                    v = {1.0f, 0.0f};
+                }
             }
-            const double a = f * z1[j], b = f * z2[j];
-            // (a - i b)(c + i s)
-            v = {(float)(a * c + b * s), (float)(a * s - b * c)};
+            e1[u] = v;
+        } else if (t < na + n1 + n2) {
+            const int64_t u = t - na - n1;
+            const int64_t comp = u / g.e2_elems, uc = u - comp * g.e2_elems;
+            const int64_t i2 = uc / g.Np, j = uc - i2 * g.Np;
+            float2 v = {0.0f, 0.0f};
+            if (j < N) {
+                double s, c;
+                const double kz = cov[kz_row * N + j];
+                double th = kz * (d == 3 ? ax2[i2] : ax1[i2]);
+                if (mir) th += cov[ka_row * N + j] * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
+                if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
+                double f = fac ? fac[j] : 1.0;
+                if (comps > 1) {
+                    double k2 = 0.0;
+                    for (int64_t e = 0; e < d; ++e) k2 += cov[e * N + j] * cov[e * N + j];
+                    f = (comp == 0 ? 1.0 : 0.0) - cov[comp * N + j] * cov[j] / k2;
+                }
+                const double a = f * z1[j], b = f * z2[j];
+                // (a - i b)(c + i s)
+                v = {(float)(a * c + b * s), (float)(a * s - b * c)};
+            }
+            e2[u] = v;
         }
-        e2[u] = v;
     }
 }
 
@@ -564,7 +583,7 @@ struct alignas(16) Stage3 {
 // cosines (times the real parts of B), its last 64 the sines (times the imaginary parts);
 // a K step is 32 modes, so A stage, accumulators and instructions per step stay as they are
 // and only the B fragments double (two of 32 modes in place of one of 16).
-// 512^3, N = 4096, bf16: 4.40 -> 2.77 ms a call; 3 x 128^3, N = 4096: 336 -> 259 us.
+// 512^3, N = 4096, bf16: 4.36 -> 2.69 ms; 3 x 128^3, N = 4096: 242 -> 161 us.
 // What bounds it now: a stream of matrix instructions leaves the SIMD's other wave hardly any
 // vector issue slots, so the 320 vector instructions that build the B fragments of a step
 // add to its 96 matrix instructions (1604 of 2288 cycles per wave and step).  Building half of
@@ -787,7 +806,7 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
 
 template <bool FP16, bool SPLIT>
 __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, double alpha,
-                                                                const int* __restrict__ mirror,
+                                                                const double* __restrict__ ax0,
                                                                 const uint32_t* __restrict__ a_hi,
                                                                 const uint32_t* __restrict__ a_lo,
                                                                 const float2* __restrict__ e1,
@@ -800,7 +819,7 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
     // different objects and does not wait for those loads before the reads
     __shared__ Stage3 st0;
     __shared__ Stage3 st1;
-    if (*mirror)  // one value for the launch
+    if (mirrored_axis(ax0, g.n0))  // one value for the launch, and that of its tables
         mfma_grid3_tile<FP16, SPLIT, true>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
                                            steps_per, partial);
     else
@@ -823,60 +842,35 @@ __global__ void k_fill_zero_f32(float* __restrict__ p, int64_t n) {
     if (i < n) p[i] = 0.0f;
 }
 
-// What the grid's axes allow (one block).
-//
-// *mirror: whether the row axis x (n0 points) is its own mirror image, x_r + x_(n0-1-r) ==
-// x_0 + x_(n0-1) to 4 ulp of max(|x_0|, |x_(n0-1)|) for every r (a NaN or infinity: no).
-// Half the matrix work of k_mfma_grid3 hangs on it, so it is looked up here, on the
-// device, for every caller; past kMMirrorMax points the look itself would take longer than
-// some of the grids, and the axis counts as not mirrored (n0 = 0 from the host).
-//
-// Virtual axes of a split last axis y (n > 0 points): vy[a] = y[16a], vz[b] = y[b] - y[0].
+// Virtual axes of a split last axis (one block): vy[a] = y[16a], vz[b] = y[b] - y[0].
 // Checks y[j] == y[16 floor(j/16)] + (y[j mod 16] - y[0]) to 4 ulp of max|y| for every
 // j (the same FP64 operations as the host's check); any miss (or a NaN) makes every vy
 // NaN, so the whole output is NaN rather than a wrong field.
-constexpr int64_t kMMirrorMax = 32768;
-constexpr int kMAxesThreads = 512;
-
-__global__ __launch_bounds__(kMAxesThreads) void k_mfma_axes(const double* __restrict__ x, int64_t n0,
-                                                             int* __restrict__ mirror,
-                                                             const double* __restrict__ y, int64_t n,
-                                                             double* __restrict__ vy, double* __restrict__ vz) {
-    __shared__ double s_max[kMAxesThreads];
-    __shared__ int s_bad, s_odd;
+__global__ __launch_bounds__(256) void k_split_axis(const double* __restrict__ y, int64_t n,
+                                                    double* __restrict__ vy, double* __restrict__ vz) {
+    __shared__ double s_max[256];
+    __shared__ int s_bad;
     const int t = threadIdx.x;
     double m = 0.0;
-    for (int64_t j = t; j < n; j += kMAxesThreads) m = fmax(m, fabs(y[j]));
+    for (int64_t j = t; j < n; j += 256) m = fmax(m, fabs(y[j]));
     s_max[t] = m;
-    if (t == 0) {
-        s_bad = 0;
-        s_odd = n0 > 0 ? 0 : 1;
-    }
+    if (t == 0) s_bad = 0;
     __syncthreads();
-    if (n0 > 0) {
-        const double ends = x[0] + x[n0 - 1], tol = 0x1p-50 * fmax(fabs(x[0]), fabs(x[n0 - 1]));
-        bool odd = false;
-        for (int64_t r = t; 2 * r < n0; r += kMAxesThreads)
-            if (!(fabs((x[r] + x[n0 - 1 - r]) - ends) <= tol)) odd = true;
-        if (odd) s_odd = 1;
-    }
-    for (int w = kMAxesThreads / 2; w > 0; w >>= 1) {
+    for (int w = 128; w > 0; w >>= 1) {
         if (t < w) s_max[t] = fmax(s_max[t], s_max[t + w]);
         __syncthreads();
     }
-    if (t == 0) *mirror = s_odd ? 0 : 1;
-    if (n == 0) return;  // whole block
     const double tol = 0x1p-50 * s_max[0];
     const double y0 = y[0];
     bool bad = false;
-    for (int64_t j = t; j < n; j += kMAxesThreads) {
+    for (int64_t j = t; j < n; j += 256) {
         const double r = y[j & ~(int64_t)15] + (y[j & 15] - y0);
         if (!(fabs(y[j] - r) <= tol)) bad = true;
     }
     if (bad) s_bad = 1;
     __syncthreads();
     const double poison = s_bad ? __builtin_nan("") : 0.0;
-    for (int64_t a = t; a < (n + 15) / 16; a += kMAxesThreads) vy[a] = y[16 * a] + poison;
+    for (int64_t a = t; a < (n + 15) / 16; a += 256) vy[a] = y[16 * a] + poison;
     if (t < 16) vz[t] = y[t] - y0;
 }
 
@@ -884,15 +878,15 @@ template <bool FP16>
 int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t comps, int64_t ka_row, int64_t k1_row,
                 int64_t kz_row, const double* ax0,
                 const double* ax1, const double* ax2, const double* cov, const double* z1, const double* z2,
-                const double* fac, double alpha, float* out, const int* mirror, void* ws, hipStream_t s) {
+                const double* fac, double alpha, float* out, void* ws, hipStream_t s) {
     uint32_t* a_hi = static_cast<uint32_t*>(ws);
     uint32_t* a_lo = a_hi + g.a_elems / 2;
     float2* e1 = reinterpret_cast<float2*>(a_lo + g.a_elems / 2);
     float2* e2 = e1 + g.e1_elems;
     const int64_t entries = g.n0p * g.Np + g.e1_elems + comps * g.e2_elems;
-    hipLaunchKernelGGL((k_mfma_tables<FP16>), dim3((unsigned)ceil_div(entries, 256)), dim3(256), 0, s, g, d,
-                       N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, mirror, a_hi, a_lo, e1,
-                       e2);
+    const int64_t tblocks = ceil_div(entries, (int64_t)256) < kMTableBlocks ? ceil_div(entries, (int64_t)256) : kMTableBlocks;
+    hipLaunchKernelGGL((k_mfma_tables<FP16>), dim3((unsigned)tblocks), dim3(256), 0, s, g, d,
+                       N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, a_hi, a_lo, e1, e2);
     int st = launch_status();
     if (st != GSX_OK) return st;
     const int64_t steps_per = mfma_steps_per_split(g, comps, fill);
@@ -906,10 +900,10 @@ int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t c
     const dim3 grid((unsigned)blocks), block(kMWaves * 64);
     if (g.g2 == 1) {
         if (ksplit > 1)
-            hipLaunchKernelGGL((k_mfma_grid3<FP16, true>), grid, block, 0, s, g, alpha, mirror, a_hi, a_lo, e1, e2, out,
+            hipLaunchKernelGGL((k_mfma_grid3<FP16, true>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2, out,
                                stride, comps, steps_per, partial);
         else
-            hipLaunchKernelGGL((k_mfma_grid3<FP16, false>), grid, block, 0, s, g, alpha, mirror, a_hi, a_lo, e1, e2,
+            hipLaunchKernelGGL((k_mfma_grid3<FP16, false>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2,
                                out, stride, comps, steps_per, partial);
     } else if (d == 2) {
         if (ksplit > 1)
@@ -977,32 +971,23 @@ int mfma_entry(int64_t d, int64_t N, const int64_t* shape, const double* axes, c
         ka_row = 1;
         k1_row = 0;
     }
-    int* mirror = nullptr;
-    if (g.g2 == 1) {  // k_mfma_grid3
-        mirror = static_cast<int*>(workspace);
-        double *vy = nullptr, *vz = nullptr;
-        if (split) {
-            vy = reinterpret_cast<double*>(static_cast<char*>(workspace) +
-                                           ceil_div(mfma_ws_bytes(g, 1, fill), (int64_t)256) * 256);
-            vz = vy + g.n1;
-        }
-        hipLaunchKernelGGL(k_mfma_axes, dim3(1), dim3(kMAxesThreads), 0, s, ax0, g.n0 <= kMMirrorMax ? g.n0 : 0,
-                           mirror, ax1, split ? shape[1] : (int64_t)0, vy, vz);
+    if (split) {
+        double* vy = reinterpret_cast<double*>(static_cast<char*>(workspace) +
+                                               ceil_div(mfma_ws_bytes(g, 1, fill), (int64_t)256) * 256);
+        double* vz = vy + g.n1;
+        hipLaunchKernelGGL(k_split_axis, dim3(1), dim3(256), 0, s, ax1, shape[1], vy, vz);
         const int st = launch_status();
         if (st != GSX_OK) return st;
-        if (split) {
-            ax1 = vy;
-            ax2 = vz;
-            dk = 3;      // tables of the 3D form
-            kz_row = 1;  // both virtual axes carry the mode's k_1
-        }
+        ax1 = vy;
+        ax2 = vz;
+        dk = 3;      // tables of the 3D form
+        kz_row = 1;  // both virtual axes carry the mode's k_1
     }
-    void* tables = static_cast<char*>(workspace) + kMFlagBytes;
     if (variant == GSX_MFMA_FP16X3)
         return mfma_launch<true>(g, fill, dk, N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac,
-                                 alpha, out, mirror, tables, s);
+                                 alpha, out, workspace, s);
     return mfma_launch<false>(g, fill, dk, N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac,
-                              alpha, out, mirror, tables, s);
+                              alpha, out, workspace, s);
 }
 
 }  // namespace gsx
