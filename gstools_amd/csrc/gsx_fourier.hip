@@ -40,30 +40,42 @@ typedef __attribute__((ext_vector_type(4))) double f64x4;
 
 constexpr int kFR = 128;     // C rows per block
 constexpr int kFK = 16;      // K per LDS stage
-constexpr int kFApad = kFK + 1;
+constexpr int kFApad = kFK + 2;  // 16-byte aligned rows, operand reads over all banks
 
 // Batched real FP64 GEMM, row-major: C_b = A_b B_b, A_b (M x K, lda), B_b (K x N,
 // ldb), C_b (M x N, ldc), operand b at A + b sA, B + b sB, C + b sC.  Block =
-// (batch, row tile, column tile) of 128 x 64 WC: 4 waves in (4 / WC) x WC, each
-// (128 WC / 4) rows x 64 columns of 16 x 16 MFMA tiles (WC = 2: 4 x 4; WC = 1,
+// (batch, row tile, column tile) of kFR x 64 WC: 4 waves in (4 / WC) x WC, each
+// (kFR WC / 4) rows x 64 columns of 16 x 16 MFMA tiles (WC = 2: 4 x 4; WC = 1,
 // for launches with few tiles or N <= 64: 2 x 4); A and B tiles staged through
-// LDS with the next stage prefetched into registers; out-of-range operand
-// entries are zero.
+// LDS with the next stage prefetched into registers.  Rows and columns past the end
+// are read from clamped addresses and not stored; K entries past the end are zero.
+// kPair: N, lda, ldb, sA, sB even and A, B 16-byte aligned, so whole stages are read as
+// 16-byte pairs without a check (N even, so a pair of columns is whole or past the
+// end).
+//
+// Bound by the FP64 matrix cores, which share the vector unit's issue: a vector
+// instruction in the loop costs its time, so the loop carries as few as it can.
+// 4096^2 points, 256^2 modes: the last stage (4096 x 4096 x 512) 307 -> 290 us, the first
+// (8192 x 256 x 512, 64-column tiles) 56 -> 52, from reads of 8 bytes with a check each;
+// the matrix cores are then busy 80% of the time at 2.17 GHz.  A second LDS buffer (one
+// barrier a stage) changed neither.
 // v_mfma_f64_16x16x4 layouts (g = lane / 16): A: lane holds row lane % 16, K
 // element g; B: column lane % 16, K element g; C: column lane % 16, register r
 // holds row g + 4 r.
-template <int WC>
+template <int WC, bool kPair>
 __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, int64_t K,
                                                           const double* __restrict__ A, int64_t lda, int64_t sA,
                                                           const double* __restrict__ B, int64_t ldb, int64_t sB,
                                                           double* __restrict__ C, int64_t ldc, int64_t sC,
                                                           int64_t row_tiles, int64_t col_tiles) {
+    typedef __attribute__((ext_vector_type(2))) double f64x2;
     constexpr int kBC = 64 * WC;            // block columns
     constexpr int kBpad = kBC + 16;
     constexpr int kRF = kFR * WC / 4 / 16;  // 16-row MFMA tiles per wave
-    constexpr int kBT = 256 / kBC;          // B rows staged per pass
-    __shared__ double As[kFR * kFApad];
-    __shared__ double Bs[kFK * kBpad];
+    constexpr int kBW = kPair ? 2 : 1;      // columns per staging thread
+    constexpr int kBT = 256 * kBW / kBC;    // B rows staged per pass
+    __shared__ __align__(16) double As[kFR * kFApad];
+    __shared__ __align__(16) double Bs[kFK * kBpad];
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
     const int wr = wave / WC, wc = wave % WC;
@@ -77,30 +89,61 @@ __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, 
     C += bt * sC;
     const int64_t i0 = rt * kFR, p0 = ct * kBC;
 
-    // staging: A 128 x 16 (two threads per row, 8 consecutive each); B 16 x kBC
-    // (column t % kBC of rows t / kBC + kBT u: unit-stride loads and LDS stores)
+    // staging: A kFR x 16 (two threads per row, 8 consecutive each); B 16 x kBC (kBW
+    // columns of rows t / (kBC / kBW) + kBT u)
     const int ar = t >> 1, ac = (t & 1) * 8;
-    const int br = t / kBC, bc = t % kBC;
-    double pa[8], pb[kFK / kBT];
+    const int br = t / (kBC / kBW), bc = t % (kBC / kBW) * kBW;
+    const double* arow = A + (i0 + ar < M ? i0 + ar : M - 1) * lda + ac;
+    const int64_t pc = p0 + bc < N ? p0 + bc : (kPair ? (N - 1) / 2 * 2 : N - 1);
+    const double* brow = B + br * ldb + pc;
+    double pa[8], pb[kBW * kFK / kBT];
+    auto load_whole = [&](int64_t j0) {
+        if constexpr (kPair) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const f64x2 v = *reinterpret_cast<const f64x2*>(arow + j0 + 2 * u);
+                pa[2 * u] = v.x;
+                pa[2 * u + 1] = v.y;
+            }
+#pragma unroll
+            for (int u = 0; u < kFK / kBT; ++u) {
+                const f64x2 v = *reinterpret_cast<const f64x2*>(brow + (j0 + kBT * u) * ldb);
+                pb[2 * u] = v.x;
+                pb[2 * u + 1] = v.y;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) pa[u] = arow[j0 + u];
+#pragma unroll
+            for (int u = 0; u < kFK / kBT; ++u) pb[u] = brow[(j0 + kBT * u) * ldb];
+        }
+    };
+    auto load_tail = [&](int64_t j0) {  // the last stage when K is no multiple of 16
+#pragma unroll
+        for (int u = 0; u < 8; ++u) pa[u] = j0 + ac + u < K ? arow[j0 + u] : 0.0;
+#pragma unroll
+        for (int u = 0; u < kFK / kBT; ++u)
+#pragma unroll
+            for (int e = 0; e < kBW; ++e)
+                pb[kBW * u + e] = j0 + br + kBT * u < K && pc + e < N ? brow[(j0 + kBT * u) * ldb + e] : 0.0;
+    };
     auto load = [&](int64_t j0) {
-        const int64_t row = i0 + ar;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int64_t col = j0 + ac + u;
-            pa[u] = (row < M && col < K) ? A[row * lda + col] : 0.0;
-        }
-        const int64_t p = p0 + bc;
-#pragma unroll
-        for (int u = 0; u < kFK / kBT; ++u) {
-            const int64_t j = j0 + br + kBT * u;
-            pb[u] = (j < K && p < N) ? B[j * ldb + p] : 0.0;
-        }
+        if (j0 + kFK <= K)
+            load_whole(j0);
+        else
+            load_tail(j0);
     };
     auto store = [&]() {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) As[ar * kFApad + ac + u] = pa[u];
+        for (int u = 0; u < 4; ++u)
+            *reinterpret_cast<f64x2*>(&As[ar * kFApad + ac + 2 * u]) = f64x2{pa[2 * u], pa[2 * u + 1]};
 #pragma unroll
-        for (int u = 0; u < kFK / kBT; ++u) Bs[(br + kBT * u) * kBpad + bc] = pb[u];
+        for (int u = 0; u < kFK / kBT; ++u) {
+            if constexpr (kPair)
+                *reinterpret_cast<f64x2*>(&Bs[(br + kBT * u) * kBpad + bc]) = f64x2{pb[2 * u], pb[2 * u + 1]};
+            else
+                Bs[(br + kBT * u) * kBpad + bc] = pb[u];
+        }
     };
 
     f64x4 acc[kRF][4];
@@ -152,42 +195,58 @@ __device__ __forceinline__ void phase_sincos(double th, double* s, double* c) {
     if (fabs(th) <= kFastPhaseMax) sincos_fast(th, s, c); else sincos(th, s, c);
 }
 
-// c = f (z1 - i z2) as [cr; ci]: 2 x N doubles (N = all modes, C order)
-__global__ void k_fourier_coeff(int64_t N, const double* __restrict__ fac, const double* __restrict__ z1,
-                                const double* __restrict__ z2, double* __restrict__ c) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N) return;
-    c[j] = fac[j] * z1[j];
-    c[N + j] = -(fac[j] * z2[j]);
-}
+// Everything the contractions read, in one launch (five launches of 2 to 9 us for 4096^2
+// points with 256^2 modes were three preparations and two contractions), one thread per
+// entry, in this order:
+//  * c = f (z1 - i z2) as [cr; ci]: 2 x N doubles (N = all modes, C order);
+//  * the last axis's table [cos(k_m x_i); -sin(k_m x_i)] as rows (part, m) x columns i
+//    (2 M x n);
+//  * the other axes' tables in rotation form, rows (point, part) x columns (part', m):
+//    row (i, 0) = [cos(k_m x_i), -sin(k_m x_i)], row (i, 1) = [sin, cos] (2 n x 2 M).
+struct FourierPrep {
+    int64_t N, d;
+    int64_t M[3], n[3];
+    const double *fac, *z1, *z2, *x[3], *k[3];
+    double *c, *tab[3];
+};
 
-// Rotation-form table of one axis, rows (point, part) x columns (part', m):
-// row (i, 0) = [cos(k_m x_i), -sin(k_m x_i)], row (i, 1) = [sin, cos] (2 n x 2 M)
-__global__ void k_fourier_rot_table(int64_t n, int64_t M, const double* __restrict__ x,
-                                    const double* __restrict__ k, double* __restrict__ out) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * M) return;
-    const int64_t i = e / M, m = e - i * M;
-    double s, c;
-    phase_sincos(k[m] * x[i], &s, &c);
-    double* r0 = out + (2 * i) * (2 * M);
-    double* r1 = r0 + 2 * M;
-    r0[m] = c;
-    r0[M + m] = -s;
-    r1[m] = s;
-    r1[M + m] = c;
-}
-
-// Last-stage table [cos(k_m x_i); -sin(k_m x_i)] as rows (part, m) x columns i (2 M x n)
-__global__ void k_fourier_last_table(int64_t n, int64_t M, const double* __restrict__ x,
-                                     const double* __restrict__ k, double* __restrict__ out) {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n * M) return;
-    const int64_t m = e / n, i = e - m * n;
-    double s, c;
-    phase_sincos(k[m] * x[i], &s, &c);
-    out[m * n + i] = c;
-    out[(M + m) * n + i] = -s;
+__global__ __launch_bounds__(256) void k_fourier_prepare(FourierPrep f) {
+    int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e < f.N) {
+        f.c[e] = f.fac[e] * f.z1[e];
+        f.c[f.N + e] = -(f.fac[e] * f.z2[e]);
+        return;
+    }
+    e -= f.N;
+    const int64_t last = f.d - 1;
+    {
+        const int64_t n = f.n[last], M = f.M[last];
+        if (e < n * M) {
+            const int64_t m = e / n, i = e - m * n;
+            double s, c;
+            phase_sincos(f.k[last][m] * f.x[last][i], &s, &c);
+            f.tab[last][m * n + i] = c;
+            f.tab[last][(M + m) * n + i] = -s;
+            return;
+        }
+        e -= n * M;
+    }
+    for (int64_t a = 0; a < last; ++a) {
+        const int64_t n = f.n[a], M = f.M[a];
+        if (e < n * M) {
+            const int64_t i = e / M, m = e - i * M;
+            double s, c;
+            phase_sincos(f.k[a][m] * f.x[a][i], &s, &c);
+            double* r0 = f.tab[a] + (2 * i) * (2 * M);
+            double* r1 = r0 + 2 * M;
+            r0[m] = c;
+            r0[M + m] = -s;
+            r1[m] = s;
+            r1[M + m] = c;
+            return;
+        }
+        e -= n * M;
+    }
 }
 
 struct FourierTensorPlan {
@@ -235,12 +294,16 @@ inline int dgemm(int64_t M, int64_t N, int64_t K, int64_t batch, const double* A
     const bool narrow = N <= 64 || batch * rt * ct2 < 256;
     const int64_t ct = narrow ? ct1 : ct2;
     if (batch * rt * ct > 0x7fffffffLL) return GSX_E_INVALID;
+    const bool pair = lda % 2 == 0 && ldb % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 && N % 2 == 0 &&
+                      reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0;
+    const dim3 grid((unsigned)(batch * rt * ct));
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, rt, ct);
+    };
     if (narrow)
-        hipLaunchKernelGGL(k_fourier_dgemm<1>, dim3((unsigned)(batch * rt * ct)), dim3(256), 0, s, M, N, K, A, lda,
-                           sA, B, ldb, sB, C, ldc, sC, rt, ct);
+        pair ? go(k_fourier_dgemm<1, true>) : go(k_fourier_dgemm<1, false>);
     else
-        hipLaunchKernelGGL(k_fourier_dgemm<2>, dim3((unsigned)(batch * rt * ct)), dim3(256), 0, s, M, N, K, A, lda,
-                           sA, B, ldb, sB, C, ldc, sC, rt, ct);
+        pair ? go(k_fourier_dgemm<2, true>) : go(k_fourier_dgemm<2, false>);
     return launch_status();
 }
 
@@ -274,27 +337,29 @@ int gsx_summate_fourier_tensor_f64(int64_t d, const int64_t* mode_no, const doub
     const double* ax[3] = {axes, axes + p.n[0], axes + p.n[0] + p.n[1]};
     const double* ka[3] = {kaxes, kaxes + p.M[0], kaxes + p.M[0] + p.M[1]};
     double* c = ws + p.off_c;
-    auto blocks = [](int64_t n) { return dim3((unsigned)gsx::ceil_div(n, (int64_t)256)); };
-    if (gsx::ceil_div(p.N, (int64_t)256) > 0x7fffffffLL) return GSX_E_INVALID;
-    for (int i = 0; i < d; ++i)
-        if (gsx::ceil_div(p.n[i] * p.M[i], (int64_t)256) > 0x7fffffffLL) return GSX_E_INVALID;
-    hipLaunchKernelGGL(gsx::k_fourier_coeff, blocks(p.N), dim3(256), 0, s, p.N, spectrum_factor, z1, z2, c);
+    gsx::FourierPrep f{p.N, d, {}, {}, spectrum_factor, z1, z2, {}, {}, c, {}};
+    int64_t entries = p.N;
+    for (int i = 0; i < d; ++i) {
+        f.M[i] = p.M[i];
+        f.n[i] = p.n[i];
+        f.x[i] = ax[i];
+        f.k[i] = ka[i];
+        f.tab[i] = ws + (i == d - 1 ? p.off_last : i == 0 ? p.off_e1 : p.off_e2);
+        entries += p.n[i] * p.M[i];
+    }
+    if (gsx::ceil_div(entries, (int64_t)256) > 0x7fffffffLL) return GSX_E_INVALID;
+    hipLaunchKernelGGL(gsx::k_fourier_prepare, dim3((unsigned)gsx::ceil_div(entries, (int64_t)256)), dim3(256), 0, s,
+                       f);
     int st = gsx::launch_status();
     if (st != GSX_OK) return st;
     const int64_t Md = p.M[d - 1], nd = p.n[d - 1];
     double* last = ws + p.off_last;
-    hipLaunchKernelGGL(gsx::k_fourier_last_table, blocks(nd * Md), dim3(256), 0, s, nd, Md, ax[d - 1], ka[d - 1],
-                       last);
-    if ((st = gsx::launch_status()) != GSX_OK) return st;
     if (d == 1)  // u (1 x n1) = [cr, ci] (1 x 2 M1) . [cos; -sin] (2 M1 x n1)
         return gsx::dgemm(1, nd, 2 * Md, 1, c, 2 * Md, 0, last, nd, 0, out, nd, 0, s);
     // first stage: T1 (2 n1 x R) = E1rot (2 n1 x 2 M1) . [cr; ci] (2 M1 x R), R = M2 ... Md
     const int64_t R = p.M[1] * p.M[2];
     double* e1 = ws + p.off_e1;
     double* t1 = ws + p.off_t1;
-    hipLaunchKernelGGL(gsx::k_fourier_rot_table, blocks(p.n[0] * p.M[0]), dim3(256), 0, s, p.n[0], p.M[0], ax[0],
-                       ka[0], e1);
-    if ((st = gsx::launch_status()) != GSX_OK) return st;
     // [cr; ci] (2 M1 x R): c holds all cr then all ci, mode index (m1, rest) in C order
     st = gsx::dgemm(2 * p.n[0], R, 2 * p.M[0], 1, e1, 2 * p.M[0], 0, c, R, 0, t1, R, 0, s);
     if (st != GSX_OK) return st;
@@ -303,9 +368,6 @@ int gsx_summate_fourier_tensor_f64(int64_t d, const int64_t* mode_no, const doub
     // middle stage, batched over x: T2(x) (2 n2 x M3) = E2rot (2 n2 x 2 M2) . T1(x) (2 M2 x M3)
     double* e2 = ws + p.off_e2;
     double* t2 = ws + p.off_t2;
-    hipLaunchKernelGGL(gsx::k_fourier_rot_table, blocks(p.n[1] * p.M[1]), dim3(256), 0, s, p.n[1], p.M[1], ax[1],
-                       ka[1], e2);
-    if ((st = gsx::launch_status()) != GSX_OK) return st;
     st = gsx::dgemm(2 * p.n[1], p.M[2], 2 * p.M[1], p.n[0], e2, 2 * p.M[1], 0, t1, p.M[2], 2 * R, t2, p.M[2],
                     2 * p.n[1] * p.M[2], s);
     if (st != GSX_OK) return st;
