@@ -60,17 +60,41 @@ def host_array(t):
     return a
 
 
-def _as_f64(x, name, dev):
-    if isinstance(x, torch.Tensor):
-        if x.dtype != torch.float64:
-            raise ValueError(f"{name}: expected float64, got {x.dtype}")
-        return x.to(dev).contiguous()
+def _host_f64(x, name):
     arr = np.asarray(x)
     if arr.dtype != np.float64:
         if not np.issubdtype(arr.dtype, np.number):
             raise ValueError(f"{name}: expected a float64 array, got {arr.dtype}")
         arr = arr.astype(np.float64)
-    return torch.from_numpy(np.ascontiguousarray(arr)).to(dev)
+    return np.ascontiguousarray(arr)
+
+
+def _as_f64(x, name, dev):
+    if isinstance(x, torch.Tensor):
+        if x.dtype != torch.float64:
+            raise ValueError(f"{name}: expected float64, got {x.dtype}")
+        return x.to(dev).contiguous()
+    return torch.from_numpy(_host_f64(x, name)).to(dev)
+
+
+def _axes(axes, name, dev):
+    """The axes one after the other in one device tensor, and their lengths.  Host axes go
+    through a page-locked buffer in one asynchronous copy (torch's host allocator keeps the
+    buffer until the copy is done): a pageable copy per axis waits for the work queued
+    before it, 40 to 50 us of an idle GPU per call.  While the stream is being captured they
+    are copied the plain way, which a capture refuses: a recorded copy would read the buffer
+    again at every replay."""
+    if any(isinstance(a, torch.Tensor) for a in axes) or torch.cuda.is_current_stream_capturing():
+        parts = [_as_f64(a, name, dev).reshape(-1) for a in axes]
+        flat = torch.cat(parts) if parts else torch.empty(0, dtype=torch.float64, device=dev)
+        return flat, [int(a.numel()) for a in parts]
+    parts = [_host_f64(a, name).reshape(-1) for a in axes]
+    shape = [a.size for a in parts]
+    if sum(shape) == 0:
+        return torch.empty(0, dtype=torch.float64, device=dev), shape
+    host = torch.empty(sum(shape), dtype=torch.float64, pin_memory=True)
+    np.concatenate(parts, out=host.numpy())
+    return host.to(dev, non_blocking=True), shape
 
 
 def _modes(cov_samples, z_1, z_2, dev):
@@ -203,12 +227,10 @@ def summate_grid_device(cov_samples, z_1, z_2, axes, precision="fp64", alpha=1.0
     d, n = cov.shape
     fac = _factor(spectrum_factor, n, dev)
     uniform_last = len(axes) == 2 and precision in ("bf16x3", "fp16x3") and uniform_axis(axes[1])
-    axes = [_as_f64(a, "axes", dev).reshape(-1) for a in axes]
+    flat, shape = _axes(axes, "axes", dev)
     if len(axes) != d:
         raise ValueError(f"expected {d} axes, got {len(axes)}")
-    shape = [int(a.numel()) for a in axes]
     npts = int(np.prod(shape))
-    flat = torch.cat(axes) if axes else torch.empty(0, dtype=torch.float64, device=dev)
     shape_c = (ctypes.c_int64 * 3)(*(shape + [1] * (3 - d)))
     if precision not in GRID_PRECISIONS:
         raise ValueError(f"precision must be one of {GRID_PRECISIONS}")
@@ -280,12 +302,10 @@ def summate_incompr_grid_device(cov_samples, z_1, z_2, axes, precision="fp64", a
     d, n = cov.shape
     if d < 2:
         raise ValueError(f"summate_incompr: incompressible sums need d = 2 or 3, got d = {d}")
-    axes = [_as_f64(a, "axes", dev).reshape(-1) for a in axes]
+    flat, shape = _axes(axes, "axes", dev)
     if len(axes) != d:
         raise ValueError(f"expected {d} axes, got {len(axes)}")
-    shape = [int(a.numel()) for a in axes]
     npts = int(np.prod(shape))
-    flat = torch.cat(axes)
     shape_c = (ctypes.c_int64 * 3)(*(shape + [1] * (3 - d)))
     if precision not in INCOMPR_GRID_PRECISIONS:
         raise ValueError(f"precision must be one of {INCOMPR_GRID_PRECISIONS}")
@@ -344,19 +364,17 @@ def summate_fourier_tensor_device(spectrum_factor, kaxes, z_1, z_2, axes, out=No
     axis on the matrix cores (``gsx_summate_fourier_tensor_f64``); returns the flat
     float64 sum in C order."""
     dev = _device()
-    kax = [_as_f64(k, "kaxes", dev).reshape(-1) for k in kaxes]
-    axs = [_as_f64(a, "axes", dev).reshape(-1) for a in axes]
-    d = len(axs)
-    if not 1 <= d <= 3 or len(kax) != d:
+    flat_k, mode_no = _axes(kaxes, "kaxes", dev)
+    flat_x, shape = _axes(axes, "axes", dev)
+    d = len(shape)
+    if not 1 <= d <= 3 or len(mode_no) != d:
         raise ValueError("one wavenumber axis per grid axis, 1 to 3 axes")
-    mode_no = [int(k.numel()) for k in kax]
     n = int(np.prod(mode_no))
     fac = _as_f64(spectrum_factor, "spectrum_factor", dev).reshape(-1)
     z1 = _as_f64(z_1, "z_1", dev).reshape(-1)
     z2 = _as_f64(z_2, "z_2", dev).reshape(-1)
     if fac.numel() != n or z1.numel() != n or z2.numel() != n:
         raise ValueError(f"spectrum_factor, z_1, z_2 must have prod(mode_no) = {n} entries")
-    shape = [int(a.numel()) for a in axs]
     npts = int(np.prod(shape))
     if out is None:
         out = torch.empty(npts, dtype=torch.float64, device=dev)
@@ -369,8 +387,6 @@ def summate_fourier_tensor_device(spectrum_factor, kaxes, z_1, z_2, axes, out=No
     if ws_bytes < 0:
         _native.check(ws_bytes, "summate_fourier_tensor")
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    flat_k = torch.cat(kax) if n else torch.zeros(1, dtype=torch.float64, device=dev)
-    flat_x = torch.cat(axs)
     _native.check(lib.gsx_summate_fourier_tensor_f64(d, m_c, _ptr(flat_k), s_c, _ptr(flat_x), _ptr(fac), _ptr(z1),
                                                       _ptr(z2), _ptr(out), _ptr(ws), ws_bytes, _stream()),
                   "summate_fourier_tensor")
