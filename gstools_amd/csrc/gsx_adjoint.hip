@@ -13,8 +13,12 @@
 // walks the chunk's points, which are staged through LDS with g_i x_id
 // precomputed (every lane reads the same point: LDS broadcast).  It writes
 // the 2 + 2D partial sums of its (chunk, mode) to the workspace.  Stage 2
-// sums the chunks of each mode in a fixed order, so results are bitwise
-// reproducible run to run (no atomics).
+// sums the chunks of each mode in a fixed order (64 threads of every 64th chunk, the
+// threads in order), so results are bitwise reproducible run to run (no atomics).
+//
+// 2D, 2048 modes, FP32, 1e6 points: stage 1 719 -> 694 us (bound by the vector unit),
+// stage 2 70 -> 8 us (245 chunks were added by 8 blocks).  FP64, 2000 points: both 45 ->
+// 22 us; FP32, 100 modes in 3D, 1e6 points: 782 -> 140.
 //
 // FP64: exact reference phase and sincos_fast (two-term reduction) with a
 // library fallback for waves whose phases may exceed 2^46.  FP32: phase in
@@ -36,26 +40,36 @@
 namespace gsx {
 
 constexpr int kAdjPts = 256;         // points per LDS stage
+// A chunk is a whole number of units: in FP32 the stages whose points form one FP32
+// partial sum, in FP64 as few points as outweigh a block's start
+template <bool F64>
+constexpr int64_t adj_unit() {
+    return F64 ? 64 : kAdjPts;
+}
 constexpr int64_t kAdjTargetBlocks = 2048;
-constexpr int kAdjModesF32 = 2;        // modes per thread of the FP32 stage 1
+// modes per thread of the FP32 stage 1 (adj_modes: one where two would leave half of
+// the only mode tile's threads idle, or the launch short of two blocks per CU)
+constexpr int kAdjModesF32 = 2;
 
 struct AdjPlan {
-    int64_t mode_tiles, chunks, chunk_pts;
+    int64_t chunks, units;  // chunk c: units [c units / chunks, (c + 1) units / chunks)
 };
 
 // Point chunks of the stage-1 grid.  max_chunks_cap (> 0) bounds the number
 // of chunks, and with it the partial sums (chunks x (2 + 2D) x N doubles).
+template <bool F64>
 inline AdjPlan adj_plan(int64_t N, int64_t P, int64_t max_chunks_cap = 0) {
     AdjPlan pl;
-    pl.mode_tiles = ceil_div(N, kThreads);
-    const int64_t max_chunks = ceil_div(P, kAdjPts);
-    int64_t chunks = ceil_div(kAdjTargetBlocks, pl.mode_tiles);
-    if (chunks > max_chunks) chunks = max_chunks;
-    if (max_chunks_cap > 0 && chunks > max_chunks_cap) chunks = max_chunks_cap;
-    if (chunks < 1) chunks = 1;
-    pl.chunk_pts = ceil_div(ceil_div(P, chunks), kAdjPts) * kAdjPts;
-    pl.chunks = ceil_div(P, pl.chunk_pts);
+    pl.units = ceil_div(P, adj_unit<F64>());
+    pl.chunks = ceil_div(kAdjTargetBlocks, ceil_div(N, (int64_t)kThreads));
+    if (pl.chunks > pl.units) pl.chunks = pl.units;
+    if (max_chunks_cap > 0 && pl.chunks > max_chunks_cap) pl.chunks = max_chunks_cap;
+    if (pl.chunks < 1) pl.chunks = 1;
     return pl;
+}
+
+inline int adj_modes(const AdjPlan& pl, int64_t N) {
+    return N > kThreads && ceil_div(N, (int64_t)kThreads * kAdjModesF32) * pl.chunks >= 512 ? kAdjModesF32 : 1;
 }
 
 // sin / cos at any |x|: the fast reduction where it is exact, else the library.
@@ -117,7 +131,7 @@ __device__ __forceinline__ void adj_stage_f32(int cnt, const double* s_x, const 
 }
 
 template <int D, typename GT, int MPT>
-__global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t P, int64_t chunk_pts,
+__global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t P, int64_t units,
                                                              const double* __restrict__ cov,
                                                              const double* __restrict__ z1,
                                                              const double* __restrict__ z2,
@@ -155,8 +169,10 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
 #pragma unroll
         for (int q = 0; q < Q; ++q) acc[u][q] = 0.0;
 
-    const int64_t p0 = (int64_t)blockIdx.y * chunk_pts;
-    const int64_t p1 = (p0 + chunk_pts < P) ? p0 + chunk_pts : P;
+    constexpr int64_t kUnit = adj_unit<F64>();
+    const int64_t p0 = blockIdx.y * units / gridDim.y * kUnit;
+    const int64_t pe = (blockIdx.y + 1) * units / gridDim.y * kUnit;
+    const int64_t p1 = pe < P ? pe : P;
     for (int64_t s0 = p0; s0 < p1; s0 += kAdjPts) {
         const int cnt = (int)((p1 - s0) < kAdjPts ? (p1 - s0) : kAdjPts);
         __syncthreads();
@@ -241,25 +257,46 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
     }
 }
 
+// modes per stage-2 block (16 doubles: one 128-byte line) and threads per mode
+constexpr int kAdj2Modes = 16, kAdj2Slices = 64;
+
 template <int D, bool F64>
-__global__ __launch_bounds__(kThreads) void k_adjoint_stage2(int64_t N, int64_t chunks,
-                                                             const double* __restrict__ z1,
-                                                             const double* __restrict__ z2,
-                                                             const double* __restrict__ part,
-                                                             double* __restrict__ gz1,
-                                                             double* __restrict__ gz2,
-                                                             double* __restrict__ gk) {
+__global__ __launch_bounds__(kAdj2Modes * kAdj2Slices) void k_adjoint_stage2(int64_t N, int64_t chunks,
+                                                                             const double* __restrict__ z1,
+                                                                             const double* __restrict__ z2,
+                                                                             const double* __restrict__ part,
+                                                                             double* __restrict__ gz1,
+                                                                             double* __restrict__ gz2,
+                                                                             double* __restrict__ gk) {
     constexpr int Q = adj_sums<D, F64>();
-    const int64_t j = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (j >= N) return;
+    static_assert(Q <= kAdj2Slices, "one slice adds the slices' sums of one quantity");
+    __shared__ double red[kAdj2Slices][Q][kAdj2Modes];
+    const int m = threadIdx.x % kAdj2Modes, w = threadIdx.x / kAdj2Modes;
+    const int64_t j = (int64_t)blockIdx.x * kAdj2Modes + m;
     double acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) acc[q] = 0.0;
-    for (int64_t c = 0; c < chunks; ++c) {
-        const double* src = part + c * Q * N;
+    if (j < N) {
+#pragma unroll 4
+        for (int64_t c = w; c < chunks; c += kAdj2Slices) {
+            const double* src = part + c * Q * N;
 #pragma unroll
-        for (int q = 0; q < Q; ++q) acc[q] += src[q * N + j];
+            for (int q = 0; q < Q; ++q) acc[q] += src[q * N + j];
+        }
     }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) red[w][q][m] = acc[q];
+    __syncthreads();
+    if (w < Q) {
+        double r = 0.0;
+#pragma unroll 16
+        for (int v = 0; v < kAdj2Slices; ++v) r += red[v][w][m];
+        red[0][w][m] = r;  // read by this thread only until the barrier
+    }
+    __syncthreads();
+    if (w != 0 || j >= N) return;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc[q] = red[0][q][m];
     const double a1 = z1[j], a2 = z2[j];
     if constexpr (F64) {
         gz1[j] = acc[0];
@@ -282,14 +319,22 @@ int adjoint_launch(const AdjPlan& pl, int64_t N, int64_t P, const double* cov, c
                    const double* z2, const double* pos, const GT* g, double* gz1, double* gz2,
                    double* gk, void* ws, hipStream_t s) {
     double* part = static_cast<double*>(ws);
-    constexpr int mpt = sizeof(GT) == 8 ? 1 : kAdjModesF32;
-    hipLaunchKernelGGL((k_adjoint_stage1<D, GT, mpt>), dim3((unsigned)ceil_div(N, (int64_t)kThreads * mpt),
-                                                          (unsigned)pl.chunks),
-                       dim3(kThreads), 0, s, N, P, pl.chunk_pts, cov, z1, z2, pos, g, part);
+    auto stage1 = [&](auto kernel, int mpt) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(N, (int64_t)kThreads * mpt), (unsigned)pl.chunks),
+                           dim3(kThreads), 0, s, N, P, pl.units, cov, z1, z2, pos, g, part);
+    };
+    if constexpr (sizeof(GT) == 8) {
+        stage1(k_adjoint_stage1<D, GT, 1>, 1);
+    } else {
+        if (adj_modes(pl, N) == 1)
+            stage1(k_adjoint_stage1<D, GT, 1>, 1);
+        else
+            stage1(k_adjoint_stage1<D, GT, kAdjModesF32>, kAdjModesF32);
+    }
     int st = launch_status();
     if (st != GSX_OK) return st;
-    hipLaunchKernelGGL((k_adjoint_stage2<D, sizeof(GT) == 8>), dim3((unsigned)pl.mode_tiles), dim3(kThreads), 0, s,
-                       N, pl.chunks, z1, z2, part, gz1, gz2, gk);
+    hipLaunchKernelGGL((k_adjoint_stage2<D, sizeof(GT) == 8>), dim3((unsigned)ceil_div(N, (int64_t)kAdj2Modes)),
+                       dim3(kAdj2Modes * kAdj2Slices), 0, s, N, pl.chunks, z1, z2, part, gz1, gz2, gk);
     return launch_status();
 }
 
@@ -343,7 +388,7 @@ int adjoint_entry(int64_t d, int64_t N, int64_t P, const double* cov, const doub
     if (done) return st;
     const int64_t need = gsx_summate_adjoint_workspace(d, N, P);
     if (!ws || ws_bytes < need) return GSX_E_WORKSPACE;
-    return adjoint_run<GT>(adj_plan(N, P), d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
+    return adjoint_run<GT>(adj_plan<sizeof(GT) == 8>(N, P), d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -397,7 +442,7 @@ int adjoint_noalloc_entry(int64_t d, int64_t N, int64_t P, const double* cov, co
     // the workspace entry point's plan whenever its partial sums fit, else
     // as many point chunks as fit (the sums then differ in rounding only)
     const int64_t per_chunk = (2 + 2 * d) * N * (int64_t)sizeof(double);
-    const AdjPlan pl = adj_plan(N, P, kScratchBytes / per_chunk);
+    const AdjPlan pl = adj_plan<sizeof(GT) == 8>(N, P, kScratchBytes / per_chunk);
     return adjoint_run<GT>(pl, d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
 }
 
@@ -408,7 +453,7 @@ extern "C" {
 int64_t gsx_summate_adjoint_workspace(int64_t d, int64_t N, int64_t P) {
     if (d < 1 || d > 3 || N < 0 || P < 0) return GSX_E_INVALID;
     if (N == 0 || P == 0) return 0;
-    const gsx::AdjPlan pl = gsx::adj_plan(N, P);
+    const gsx::AdjPlan pl = gsx::adj_plan<true>(N, P);  // FP32: fewer chunks
     return pl.chunks * (2 + 2 * d) * N * (int64_t)sizeof(double);
 }
 
@@ -417,7 +462,7 @@ int gsx_summate_adjoint_f64(int64_t d, int64_t N, int64_t P, const double* cov, 
                             double* gz2, double* gk, void* workspace, int64_t workspace_bytes,
                             void* stream) {
     return gsx::adjoint_entry<double>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, workspace,
-                                      workspace_bytes, stream);
+                                   workspace_bytes, stream);
 }
 
 int gsx_summate_adjoint_f32(int64_t d, int64_t N, int64_t P, const double* cov, const double* z1,
@@ -425,7 +470,7 @@ int gsx_summate_adjoint_f32(int64_t d, int64_t N, int64_t P, const double* cov, 
                             double* gz2, double* gk, void* workspace, int64_t workspace_bytes,
                             void* stream) {
     return gsx::adjoint_entry<float>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, workspace,
-                                     workspace_bytes, stream);
+                                   workspace_bytes, stream);
 }
 
 int gsx_summate_adjoint_f32_noalloc(int64_t d, int64_t N, int64_t P, const double* cov,

@@ -255,6 +255,27 @@ def test_adjoint_fp64_matches_oracle(d):
     assert np.max(np.abs(bk - rk)) <= 1e-5 * scale * 4
 
 
+@pytest.mark.parametrize("n,p", [(1, 1), (100, 63), (256, 65), (257, 256), (300, 257), (520, 4099), (64, 70000)])
+def test_adjoint_chunks_and_mode_tiles(n, p):
+    """Point counts around the chunk units (64 in FP64, 256 in FP32) and mode counts around
+    the tiles of one and two modes per thread, against float64 sums of the same formula."""
+    _say(f"adjoint chunks N={n} P={p}")
+    cov, z1, z2 = _modes(3, n, n + p, kscale=0.3)
+    rs = np.random.RandomState(p)
+    pos, g = rs.uniform(-20, 20, size=(3, p)), rs.normal(size=p)
+    t = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (cov, z1, z2, pos, g)]
+    ph = t[0].T @ t[3]
+    c, s = torch.cos(ph), torch.sin(ph)
+    r1, r2 = c @ t[4], s @ t[4]
+    rk = torch.stack([t[2] * (c @ (t[4] * x)) - t[1] * (s @ (t[4] * x)) for x in t[3]])
+    amp = torch.hypot(t[1], t[2])
+    for precision, tol in (("fp64", 1e-12), ("fp32", 1e-5)):
+        a1, a2, ak = summate_adjoint_device(*t[:4], t[4], precision)
+        total = float(t[4].abs().sum())
+        assert float((a1 - r1).abs().max()) <= tol * total and float((a2 - r2).abs().max()) <= tol * total
+        assert bool(torch.all((ak - rk).abs() <= tol * 20.0 * total * 2.0 * (1.0 + amp)[None, :]))
+
+
 def test_adjoint_empty_points():
     cov, z1, z2 = _modes(2, 33, 3)
     a1, a2, ak = summate_adjoint_device(cov, z1, z2, np.zeros((2, 0)), np.zeros(0), "fp64")
