@@ -432,13 +432,36 @@ __global__ __launch_bounds__(kSplitModes) void k_forward_f32_split(
 }
 
 // ------------------------------------------------------------ launchers -----
-constexpr int kPptF64 = 2;
-// FP32 points per thread: 8 for the scalar sum (the per-block mode tables and
-// LDS reads spread over twice the terms: 1.5-2% faster than 4 on the 4e6-point
-// 3D sum, at 152 VGPRs); 4 for the incompressible sum, whose d accumulators
-// per point would take 8 points to 228 VGPRs (2 waves per SIMD)
-template <bool INCOMPR>
-constexpr int ppt_f32() { return INCOMPR ? 4 : 8; }
+// Points per thread of a plain launch.  Its blocks (256 threads) spread over the 256 CUs in
+// whole rounds, so a launch of 600000 points in blocks of 2048 (293 of them) took as long as
+// one of 1e6.  Cycles of a CU per round, measured over 1.4e5 to 2.1e6 points and 150 to 2000
+// modes in 2D and 3D (a block's mode table and LDS reads spread over its points; the smaller
+// FP32 blocks look through the whole segment's coordinates, too):
+//   FP32  PPT 8 244 N + 1600, 4 126 N + 2500, 2 67 N + 3300
+//   FP64  PPT 4 405 N + 16000, 2 210 N + 5300, 1 117 N + 4000
+// a tenth more (FP64: a twentieth) for the largest in a single round, one wave per SIMD,
+// and the choice is the least rounds times cost, of equals the largest.  3D, N = 2000, cycles
+// of a SIMD per 64 terms: FP32 600000 points 57 -> 41 (PPT 2), 1.3e6 38 -> 32 (4), 4e6 31 (8);
+// FP64 140000 points 223 -> 185 (1), 1.3e6 108 -> 104 (4).
+// The incompressible sums, d accumulators to a point, start at 4 and 2 points (8 and 4
+// would leave 2 waves per SIMD).
+template <bool F64, bool INCOMPR>
+inline int plain_ppt(int64_t N, int64_t P) {
+    constexpr int kTop = (F64 ? 4 : 8) / (INCOMPR ? 2 : 1);
+    const double n = (double)N;
+    auto cost = [&](int ppt) {
+        const double rounds = (double)ceil_div(ceil_div(P, (int64_t)kThreads * ppt), (int64_t)256);
+        const double alone = rounds > 1.0 || ppt < (F64 ? 4 : 8) ? 1.0 : (F64 ? 1.05 : 1.1);
+        if (F64)
+            return alone * rounds *
+                   (ppt == 4 ? 405.0 * n + 16000.0 : ppt == 2 ? 210.0 * n + 5300.0 : 117.0 * n + 4000.0);
+        return alone * rounds * (ppt == 8 ? 244.0 * n + 1600.0 : ppt == 4 ? 126.0 * n + 2500.0 : 67.0 * n + 3300.0);
+    };
+    int best = kTop;
+    for (int ppt = kTop / 2; ppt >= (F64 ? 1 : 2); ppt /= 2)
+        if (cost(ppt) < cost(best)) best = ppt;
+    return best;
+}
 
 template <int D, int PPT, int L, bool INCOMPR, class Pts>
 int launch_f64_split(Pts pts, int64_t N, int64_t P, const double* cov, const double* z1, const double* z2,
@@ -458,22 +481,22 @@ int launch_f32_split(Pts pts, int64_t N, int64_t P, const double* cov, const dou
     return launch_status();
 }
 
-// Whether the split kernels serve (N, P).  A plain block walks all N modes for
-// its 512 (FP64) or 2048 / 1024 (FP32 scalar / incompressible) points, so up to
-// one block per CU a launch takes the time of one block whatever P is (10^4
+// Whether the split kernels serve (N, P).  A plain block of 512 (FP64) or 2048 / 1024
+// (FP32 scalar / incompressible) points walks all N modes for them, so up to one block per CU a launch takes the time of one block whatever P is (10^4
 // points, 1000 modes, 2D: FP64 130 us, FP32 119 us); a split launch takes rounds
 // of 256 blocks (24 and 14 us).  Fits of the measured times (us; 2D and 3D, 64 to
 // 4096 modes, 1 to 10^6 points; C chunks of 1024 modes, R rounds):
 //   FP64  plain N / 7.7      split R (8 C + N / 46)
-//   FP32  plain 5 + N / 8.9  split R (12 C + N / 56)
+//   FP32  plain 5 + N / 8.9  split R (12 C + N / 56), in 1D 5 + N / 10.5 and R (8 C + N / 66)
 // The plain fits hold up to 131072 (FP64), 524288 (FP32) and 262144 (FP32
 // incompressible) points; the rounds that the inequalities allow end before.
-template <bool F64>
+template <bool F64, int D>
 inline bool split_pays(int64_t N, int64_t P, int64_t round_points) {
     const double R = (double)ceil_div(P, round_points), C = (double)ceil_div(N, (int64_t)kSplitModes);
     const double n = (double)N;
     if (R > 4.0) return false;
-    return F64 ? R * (8.0 * C + n / 46.0) <= n / 7.7 : R * (12.0 * C + n / 56.0) <= 5.0 + n / 8.9;
+    if (F64) return R * (8.0 * C + n / 46.0) <= n / 7.7;
+    return D == 1 ? R * (8.0 * C + n / 66.0) <= 5.0 + n / 10.5 : R * (12.0 * C + n / 56.0) <= 5.0 + n / 8.9;
 }
 
 template <int D, bool INCOMPR, class Pts, class OutT>
@@ -481,26 +504,49 @@ int launch_forward(Pts pts, int64_t N, int64_t P, const double* cov, const doubl
                    const double* z2, const double* fac, OutT* out, hipStream_t s) {
     if constexpr (sizeof(OutT) == 8) {
         // the smallest blocks that keep the launch within one round of 256
-        if (split_pays<true>(N, P, 256 * 128)) {
+        if (split_pays<true, D>(N, P, 256 * 128)) {
             if (P <= 256 * 32) return launch_f64_split<D, 1, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             if (P <= 256 * 64) return launch_f64_split<D, 2, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             return launch_f64_split<D, 2, 1, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
         }
-        const int64_t blocks = ceil_div(P, (int64_t)kThreads * kPptF64);
-        hipLaunchKernelGGL((k_forward_f64<D, kPptF64, INCOMPR, Pts>), dim3((unsigned)blocks),
-                           dim3(kThreads), 0, s, pts, N, P, cov, z1, z2, fac, out);
+        const int ppt = plain_ppt<true, INCOMPR>(N, P);
+        auto plain = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(P, (int64_t)kThreads * ppt)), dim3(kThreads), 0, s, pts,
+                               N, P, cov, z1, z2, fac, out);
+        };
+        if constexpr (!INCOMPR) {
+            if (ppt == 4) {
+                plain(k_forward_f64<D, 4, INCOMPR, Pts>);
+                return launch_status();
+            }
+        }
+        if (ppt == 2)
+            plain(k_forward_f64<D, 2, INCOMPR, Pts>);
+        else
+            plain(k_forward_f64<D, 1, INCOMPR, Pts>);
     } else {
         constexpr int big = INCOMPR ? 4 : 8;  // points per thread of the largest split block
-        if (split_pays<false>(N, P, 256 * 64 * big)) {
+        if (split_pays<false, D>(N, P, 256 * 64 * big)) {
             if (P <= 256 * 64) return launch_f32_split<D, 1, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             if (P <= 256 * 128) return launch_f32_split<D, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             if (P <= 256 * 256) return launch_f32_split<D, 4, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             return launch_f32_split<D, big, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
         }
-        constexpr int ppt = ppt_f32<INCOMPR>();
-        const int64_t blocks = ceil_div(P, (int64_t)kThreads * ppt);
-        hipLaunchKernelGGL((k_forward_f32<D, ppt, INCOMPR, Pts>), dim3((unsigned)blocks),
-                           dim3(kThreads), 0, s, pts, N, P, cov, z1, z2, fac, out);
+        const int ppt = plain_ppt<false, INCOMPR>(N, P);
+        auto plain = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(P, (int64_t)kThreads * ppt)), dim3(kThreads), 0, s, pts,
+                               N, P, cov, z1, z2, fac, out);
+        };
+        if constexpr (!INCOMPR) {
+            if (ppt == 8) {
+                plain(k_forward_f32<D, 8, INCOMPR, Pts>);
+                return launch_status();
+            }
+        }
+        if (ppt == 4)
+            plain(k_forward_f32<D, 4, INCOMPR, Pts>);
+        else
+            plain(k_forward_f32<D, 2, INCOMPR, Pts>);
     }
     return launch_status();
 }

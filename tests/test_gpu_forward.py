@@ -243,3 +243,25 @@ def test_split_launches_equal_plain_launch(d, n, precision, incompr):
     for p in (1, 31, 33, 64, 65, 127, 129, 8192, 8193, 16385, 32769, 65537, 131073):
         got = fn(cov, z1, z2, pos[:, :p].contiguous(), precision).reshape(-1, p)
         assert torch.equal(got, want[:, :p]), (p, precision)
+
+
+@pytest.mark.parametrize("incompr", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("d", [2, 3])
+def test_plain_launches_agree_whatever_their_blocks(d, precision, incompr):
+    """The points per thread of a plain launch follow its size; a point's value does not:
+    launches of 1.4e5 to 1.1e6 points, which take each of the block shapes, give the bits of
+    the first.  One far point per 2048-point segment puts some modes of every group on the
+    other phase reduction and keeps the segments' bounds the same."""
+    n, big = 300, 1_050_001
+    rs = np.random.RandomState(d)
+    cov = torch.from_numpy(rs.standard_cauchy(size=(d, n))).cuda()
+    z1, z2 = torch.from_numpy(rs.normal(size=(2, n))).cuda()
+    pos = torch.from_numpy(rs.uniform(-200.0, 200.0, size=(d, big))).cuda()
+    pos[:, ::2048] *= 5e3
+    fn = summate_incompr_device if incompr else summate_device
+    want = fn(cov, z1, z2, pos, precision).reshape(-1, big)
+    assert bool(torch.isfinite(want).all())
+    for p in (140_003, 262_145, 393_217, 524_289, 600_000, 700_001, 800_000, 1_048_576):
+        got = fn(cov, z1, z2, pos[:, :p].contiguous(), precision).reshape(-1, p)
+        assert torch.equal(got, want[:, :p]), (p, precision)
