@@ -33,8 +33,9 @@
 //
 // Bound by the FP64 matrix cores, and on few points by the last round of blocks.
 // Field and variance term of 40000 points, K = 301: 299 us with 128 x 128 diagonal
-// blocks, pairs of row tiles per block and the field as a pass of its own, now 135;
-// K = 1001 onto 400000: 9.17 -> 8.00 ms.  Field alone, K = 301 onto 40000: 97 -> 23 us.
+// blocks, pairs of row tiles per block and the field as a pass of its own, 135 without,
+// and 117 with staging reads that check nothing (but in the first stage) and the
+// epilogue's reads of V in batches; K = 1001 onto 400000: 9.17 -> 8.00 -> 7.11 ms.  Field alone, K = 301 onto 40000: 97 -> 23 us.
 //
 // Right-hand sides: k_krige_cov writes the covariance rows of V,
 // C(|c_i - x_p|) for conditioning points c_i and targets x_p, for models
@@ -58,7 +59,7 @@ constexpr int kKrRows = 128;  // W rows per block
 constexpr int kKrRF = kKrRows / 32;  // 16-row MFMA tiles per wave (two row waves)
 constexpr int kKrPts = 128;   // points per block
 constexpr int kKrK = 16;      // reduction depth per LDS stage
-constexpr int kKrApad = kKrK + 1;
+constexpr int kKrApad = kKrK + 2;  // 16-byte aligned rows, operand reads over all banks
 // B rows padded by 16 doubles: the operand reads of K groups g and g + 1
 // (rows 144 doubles apart) fall in disjoint LDS banks
 constexpr int kKrBpad = kKrPts + 16;
@@ -130,8 +131,8 @@ __global__ __launch_bounds__(256, 2) void k_krige_gemm(int64_t K, int64_t Kp, in
                                                     const double* __restrict__ wgt,
                                                     double* __restrict__ part_e, double* __restrict__ field) {
     typedef __attribute__((ext_vector_type(2))) double f64x2;
-    __shared__ double As[kKrRows * kKrApad];
-    __shared__ double Bs[kKrK * kKrBpad];
+    __shared__ __align__(16) double As[kKrRows * kKrApad];
+    __shared__ __align__(16) double Bs[kKrK * kKrBpad];
     __shared__ double red[4][kKrPts];  // [row wave][point], or [row class][point] of the field
 
     const int t = threadIdx.x;
@@ -156,38 +157,32 @@ __global__ __launch_bounds__(256, 2) void k_krige_gemm(int64_t K, int64_t Kp, in
     const f64x2* arow = reinterpret_cast<const f64x2*>(M + (i0 + ar) * Kp + ac);
     const int br = __builtin_amdgcn_readfirstlane(kPairB ? t >> 6 : t >> 7);
     const int bc = kPairB ? (t & 63) * 2 : t & 127;
+    // columns past P are read from a clamped address and not stored; rows past K, in the first
+    // stage only, are zero
+    const double* vcol = V + (p0 + bc < P ? p0 + bc : (kPairB ? P - 2 : P - 1)) + br * P;
     f64x2 pa[4];
-    f64x2 pb2[4];    // point pairs: loads from clamped (valid) addresses, zeroed at the store (bit u of mb)
-    double pb1[8];   // single points
-    unsigned mb = 0;
-    auto load = [&](int64_t j0) {
+    f64x2 pb2[4];   // point pairs (P even: a pair is whole or out of range)
+    double pb1[8];  // single points
+    auto load = [&](int64_t j0, bool whole) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) pa[v] = arow[(j0 >> 1) + v];
-        const int64_t p = p0 + bc;
-        if constexpr (kPairB) {
-            const int64_t pc = p < P ? p : P - 2;  // P even: a pair is whole or out of range
-            mb = 0;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int64_t j = j0 + br + 4 * u;
-                pb2[u] = *reinterpret_cast<const f64x2*>(V + (j < K ? j : K - 1) * P + pc);
-                mb |= (j < K && p < P) ? (1u << u) : 0u;
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int64_t j = j0 + br + 2 * u;
-                pb1[u] = (j < K && p < P) ? V[j * P + p] : 0.0;
-            }
+        for (int u = 0; u < (kPairB ? 4 : 8); ++u) {
+            const int64_t j = j0 + (kPairB ? 4 : 2) * u;  // row less br
+            const bool in = whole || j + br < K;
+            if constexpr (kPairB)
+                pb2[u] = in ? *reinterpret_cast<const f64x2*>(vcol + j * P) : f64x2{0.0, 0.0};
+            else
+                pb1[u] = in ? vcol[j * P] : 0.0;
         }
     };
     // the field's terms of the staged rows: class br (pairs), classes br and br + 2
     double f0 = 0.0, f1 = 0.0;
-    auto field_terms = [&](int64_t j0) {
+    auto field_terms = [&](int64_t j0, bool whole) {
 #pragma unroll
         for (int u = 0; u < (kPairB ? 4 : 8); ++u) {
             const int64_t j = j0 + br + (kPairB ? 4 : 2) * u;
-            if (j < K) {
+            if (whole || j < K) {
                 const double aj = wgt[j];
                 if constexpr (kPairB) {
                     f0 = fma_(aj, pb2[u].x, f0);
@@ -202,18 +197,13 @@ __global__ __launch_bounds__(256, 2) void k_krige_gemm(int64_t K, int64_t Kp, in
     };
     auto store = [&]() {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            As[ar * kKrApad + ac + 2 * v] = pa[v].x;
-            As[ar * kKrApad + ac + 2 * v + 1] = pa[v].y;
-        }
-        if constexpr (kPairB) {
+        for (int v = 0; v < 4; ++v) *reinterpret_cast<f64x2*>(&As[ar * kKrApad + ac + 2 * v]) = pa[v];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                *reinterpret_cast<f64x2*>(&Bs[(br + 4 * u) * kKrBpad + bc]) =
-                    ((mb >> u) & 1u) ? pb2[u] : f64x2{0.0, 0.0};
-        } else {
-#pragma unroll
-            for (int u = 0; u < 8; ++u) Bs[(br + 2 * u) * kKrBpad + bc] = pb1[u];
+        for (int u = 0; u < (kPairB ? 4 : 8); ++u) {
+            if constexpr (kPairB)
+                *reinterpret_cast<f64x2*>(&Bs[(br + 4 * u) * kKrBpad + bc]) = pb2[u];
+            else
+                Bs[(br + 2 * u) * kKrBpad + bc] = pb1[u];
         }
     };
 
@@ -228,15 +218,7 @@ __global__ __launch_bounds__(256, 2) void k_krige_gemm(int64_t K, int64_t Kp, in
     // same rows of V, so the row tiles of one column tile (resident together on
     // one XCD) read each V row at about the same time and share it through L2.
     const int64_t jlast = ((K - 1) / kKrK) * kKrK;
-    load(jlast);
-    for (int64_t j0 = jlast; j0 >= i0; j0 -= kKrK) {
-        __syncthreads();
-        store();
-        if (rt_idx == 0) field_terms(j0);
-        __syncthreads();
-        if (j0 - kKrK >= i0) load(j0 - kKrK);
-        const int64_t rows_in = K - i0 - wr * 16 > j0 - i0 + 1 ? j0 - i0 + 1 : K - i0 - wr * 16;
-        const int rt_end = (int)(rows_in >= kKrRows ? kKrRF : (rows_in + 31) >> 5);
+    auto products = [&](int rt_end) {
 #pragma unroll
         for (int kk = 0; kk < kKrK; kk += 4) {
             double a[kKrRF], b[4];
@@ -244,7 +226,6 @@ __global__ __launch_bounds__(256, 2) void k_krige_gemm(int64_t K, int64_t Kp, in
             for (int rt = 0; rt < kKrRF; ++rt) a[rt] = As[(rt * 32 + wr * 16 + l16) * kKrApad + kk + g];
 #pragma unroll
             for (int ct = 0; ct < 4; ++ct) b[ct] = Bs[(kk + g) * kKrBpad + wc * 64 + ct * 16 + l16];
-            // fragments left of their diagonal block or past row K add nothing
 #pragma unroll
             for (int rt = 0; rt < kKrRF; ++rt)
                 if (rt < rt_end)
@@ -252,26 +233,66 @@ __global__ __launch_bounds__(256, 2) void k_krige_gemm(int64_t K, int64_t Kp, in
                     for (int ct = 0; ct < 4; ++ct)
                         acc[rt][ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[rt], b[ct], acc[rt][ct], 0, 0, 0);
         }
+    };
+    // row fragments with rows below K (this wave's: 16 of every 32 rows)
+    const int64_t rows_left = K - i0 - wr * 16;
+    const int rt_rows = rows_left >= kKrRows ? kKrRF : (rows_left > 0 ? (int)((rows_left + 31) >> 5) : 0);
+    auto stage = [&](int64_t j0) {
+        __syncthreads();
+        store();
+        if (rt_idx == 0) field_terms(j0, j0 + kKrK <= K);
+        __syncthreads();
+        if (j0 - kKrK >= i0) load(j0 - kKrK, true);
+    };
+    load(jlast, jlast + kKrK <= K);
+    int64_t j0 = jlast;
+    if (i0 + kKrRows <= K)  // every fragment has rows: a straight line of products down to the diagonal
+        for (; j0 >= i0 + kKrRows - 32; j0 -= kKrK) {
+            stage(j0);
+            products(kKrRF);
+        }
+    for (; j0 >= i0; j0 -= kKrK) {
+        // fragments left of their diagonal block or past row K add nothing
+        stage(j0);
+        const int rt_diag = (int)((j0 - i0) >> 5) + 1;
+        products(rt_diag < rt_rows ? rt_diag : rt_rows);
     }
 
-    // epilogue: per column, sum over this wave's kKrRows / 2 rows of V o W (fragments
-    // past row K hold zeros)
+    // epilogue: per column, sum over this wave's kKrRows / 2 rows of V o W (fragments past row
+    // K hold zeros).  V is read in two batches of 32 values per lane from clamped addresses:
+    // a checked read at a time left 23 us of latency on a block whose loop takes 65.
     double se[4];
 #pragma unroll
-    for (int ct = 0; ct < 4; ++ct) {
-        const int64_t p = p0 + wc * 64 + ct * 16 + l16;
-        double e = 0.0;
+    for (int c2 = 0; c2 < 4; c2 += 2) {
+        double v[2][kKrRF][4];
 #pragma unroll
-        for (int rt = 0; rt < kKrRF; ++rt)
+        for (int h = 0; h < 2; ++h) {
+            const int64_t p = p0 + wc * 64 + (c2 + h) * 16 + l16;
+            const double* vp = V + (p < P ? p : P - 1);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t i = i0 + rt * 32 + wr * 16 + g + 4 * r;
-                if (i < K && p < P) e += V[i * P + p] * acc[rt][ct][r];
-            }
-        // the four lane groups holding this column, in a fixed order
-        e += __shfl_xor(e, 16);
-        e += __shfl_xor(e, 32);
-        se[ct] = e;
+            for (int rt = 0; rt < kKrRF; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t i = i0 + rt * 32 + wr * 16 + g + 4 * r;
+                    v[h][rt][r] = vp[(i < K ? i : K - 1) * P];
+                }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            double e = 0.0;
+#pragma unroll
+            for (int rt = 0; rt < kKrRF; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t i = i0 + rt * 32 + wr * 16 + g + 4 * r;
+                    e += (i < K ? v[h][rt][r] : 0.0) * acc[rt][c2 + h][r];
+                }
+            // the four lane groups holding this column, in a fixed order
+            e += __shfl_xor(e, 16);
+            e += __shfl_xor(e, 32);
+            se[c2 + h] = e;
+        }
     }
     if (g == 0) {
 #pragma unroll
@@ -351,49 +372,96 @@ struct CovModelArgs {
     double sill_at_0;   // >= 0: value where r <= 1e-8 (cov_nugget); < 0: none
 };
 
-__device__ __forceinline__ double cov_of(const CovModelArgs& m, double r) {
-    if (m.sill_at_0 >= 0.0 && r <= 1e-8) return m.sill_at_0;
-    const double h = r / m.len;
-    double c;
-    switch (m.kind) {
-        case 0: c = exp(-(h * h)); break;
-        case 1: c = exp(-h); break;
-        case 2: c = exp(-pow(h, m.alpha)); break;
-        default: {
-            const double g = fmin(h, 1.0);
-            c = 1.0 - 1.5 * g + 0.5 * (g * g * g);
-        }
+// C(r).  kDiv: h = r / m.len by division; else by inv = 1 / m.len rounded: the product
+// corrected by its remainder, the rounded quotient again (for lengths that krige_cov_launch
+// passes; a product out of range stays as it is, infinite or NaN like the quotient).
+template <int KIND, bool kDiv>
+__device__ __forceinline__ double cov_of(const CovModelArgs& m, double inv, double r) {
+    double h;
+    if constexpr (kDiv) {
+        h = r / m.len;
+    } else {
+        const double q = r * inv;
+        h = q < 0x1p+900 ? fma_(fma_(-q, m.len, r), inv, q) : q;
     }
-    return m.var * c;
+    double c;
+    if constexpr (KIND == 0) {
+        c = exp(-(h * h));
+    } else if constexpr (KIND == 1) {
+        c = exp(-h);
+    } else if constexpr (KIND == 2) {
+        c = exp(-pow(h, m.alpha));
+    } else {
+        const double g = fmin(h, 1.0);
+        c = 1.0 - 1.5 * g + 0.5 * (g * g * g);
+    }
+    return (m.sill_at_0 >= 0.0 && r <= 1e-8) ? m.sill_at_0 : m.var * c;
 }
 
 // out[i * ld + p] = C(|c_i - x_p|), i < K, p < P.  A thread keeps its target in
 // registers and writes kCovRows rows (conditioning points i0 .. i0 + kCovRows - 1,
-// read as wave-uniform values), so the targets are read once per kCovRows rows.
+// read as wave-uniform values), so the targets are read once per kCovRows rows.  Bound by
+// the vector unit (square root and exponential) and by stores of 512 bytes per wave: a pair
+// of points per thread where P and ld are even and out is 16-byte aligned, the model a template
+// argument, the quotient by a reciprocal.  Exponential, 300 x 40000 in 2D: 39 -> 30 us.
 constexpr int kCovRows = 16;
 
-template <int DIM>
+template <int DIM, int KIND, bool kPair, bool kDiv>
 __global__ __launch_bounds__(256) void k_krige_cov(CovModelArgs m, int64_t K, int64_t P,
                                                    const double* __restrict__ cpos,
                                                    const double* __restrict__ pos, double* __restrict__ out,
                                                    int64_t ld) {
 #pragma clang fp contract(off)
-    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    typedef __attribute__((ext_vector_type(2))) double f64x2;
+    constexpr int kPts = kPair ? 2 : 1;
+    const int64_t p = ((int64_t)blockIdx.x * 256 + threadIdx.x) * kPts;
     const int64_t i0 = (int64_t)blockIdx.y * kCovRows;
     if (p >= P) return;
-    double x[DIM];
+    double x[kPts][DIM];
 #pragma unroll
-    for (int d = 0; d < DIM; ++d) x[d] = pos[d * P + p];
-    const int rows = (int)(K - i0 < kCovRows ? K - i0 : kCovRows);
-    for (int r = 0; r < rows; ++r) {
-        const int64_t i = i0 + r;
-        double d2 = 0.0;
+    for (int e = 0; e < kPts; ++e)
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            const double t = cpos[d * K + i] - x[d];
-            d2 += t * t;
+        for (int d = 0; d < DIM; ++d) x[e][d] = pos[d * P + p + e];
+    const double inv = 1.0 / m.len;
+    const int64_t ie = K - i0 < kCovRows ? K : i0 + kCovRows;
+#pragma unroll 2
+    for (int64_t i = i0; i < ie; ++i) {
+        double c[kPts];
+#pragma unroll
+        for (int e = 0; e < kPts; ++e) {
+            double d2 = 0.0;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                const double t = cpos[d * K + i] - x[e][d];
+                d2 += t * t;
+            }
+            c[e] = cov_of<KIND, kDiv>(m, inv, sqrt(d2));
         }
-        out[i * ld + p] = cov_of(m, sqrt(d2));
+        if constexpr (kPair)
+            *reinterpret_cast<f64x2*>(out + i * ld + p) = f64x2{c[0], c[1]};
+        else
+            out[i * ld + p] = c[0];
+    }
+}
+
+template <int DIM>
+void krige_cov_launch(const CovModelArgs& m, int64_t K, int64_t P, const double* cpos, const double* pos,
+                      double* out, int64_t ld, hipStream_t s) {
+    // lengths whose reciprocal and remainders are exact enough: far from the exponent's limits
+    const bool div = !(m.len >= 0x1p-400 && m.len <= 0x1p+400);
+    const bool pair = !div && P % 2 == 0 && ld % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    const dim3 grid((unsigned)ceil_div(P, (int64_t)(pair ? 512 : 256)), (unsigned)ceil_div(K, (int64_t)kCovRows));
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, m, K, P, cpos, pos, out, ld); };
+    auto form = [&](auto pairs, auto singles, auto division) { pair ? go(pairs) : div ? go(division) : go(singles); };
+    switch (m.kind) {
+        case 0: form(k_krige_cov<DIM, 0, true, false>, k_krige_cov<DIM, 0, false, false>,
+                     k_krige_cov<DIM, 0, false, true>); break;
+        case 1: form(k_krige_cov<DIM, 1, true, false>, k_krige_cov<DIM, 1, false, false>,
+                     k_krige_cov<DIM, 1, false, true>); break;
+        case 2: form(k_krige_cov<DIM, 2, true, false>, k_krige_cov<DIM, 2, false, false>,
+                     k_krige_cov<DIM, 2, false, true>); break;
+        default: form(k_krige_cov<DIM, 3, true, false>, k_krige_cov<DIM, 3, false, false>,
+                      k_krige_cov<DIM, 3, false, true>);
     }
 }
 
@@ -490,11 +558,10 @@ int gsx_krige_cov_f64(int model_kind, double var, double len_rescaled, double al
     if (!cond_pos || !pos || !out) return GSX_E_INVALID;
     gsx::CovModelArgs m{model_kind, var, len_rescaled, alpha, sill_at_zero};
     hipStream_t s = gsx::as_stream(stream);
-    const dim3 grid((unsigned)gsx::ceil_div(P, (int64_t)256), (unsigned)gsx::ceil_div(K, (int64_t)gsx::kCovRows));
     switch (dim) {
-        case 1: hipLaunchKernelGGL((gsx::k_krige_cov<1>), grid, dim3(256), 0, s, m, K, P, cond_pos, pos, out, ld_out); break;
-        case 2: hipLaunchKernelGGL((gsx::k_krige_cov<2>), grid, dim3(256), 0, s, m, K, P, cond_pos, pos, out, ld_out); break;
-        default: hipLaunchKernelGGL((gsx::k_krige_cov<3>), grid, dim3(256), 0, s, m, K, P, cond_pos, pos, out, ld_out);
+        case 1: gsx::krige_cov_launch<1>(m, K, P, cond_pos, pos, out, ld_out, s); break;
+        case 2: gsx::krige_cov_launch<2>(m, K, P, cond_pos, pos, out, ld_out, s); break;
+        default: gsx::krige_cov_launch<3>(m, K, P, cond_pos, pos, out, ld_out, s);
     }
     return gsx::launch_status();
 }

@@ -72,6 +72,23 @@ def test_field_and_variance_at_block_edges(k):
         assert np.array_equal(calc_field_krige(m, vp, c), f[:p])
 
 
+@pytest.mark.parametrize("length", [7.0, 1e-130, 3e150])
+@pytest.mark.parametrize("p", [1, 511, 512, 1030])
+def test_covariance_rows_forms(p, length):
+    """Pairs of points (even counts), single points (odd ones) and lengths far out, where the
+    quotient is a division, against the model's covariance to 4e-15 of the variance."""
+    from scipy.spatial.distance import cdist
+
+    from gstools_amd.krige import krige_cov_device
+
+    rs = np.random.RandomState(p)
+    cpos, pos = rs.uniform(0, 3 * length, size=(2, 19)), rs.uniform(0, 3 * length, size=(2, p))
+    for model in (gs.Gaussian(dim=2, var=1.7, len_scale=length), gs.Exponential(dim=2, var=1.7, len_scale=length),
+                  gs.Spherical(dim=2, var=1.7, len_scale=length)):
+        got = krige_cov_device(model, cpos, pos).cpu().numpy()
+        assert np.max(np.abs(got - model.covariance(cdist(cpos.T, pos.T)))) <= 4e-15 * 1.7
+
+
 def test_empty_conditions_and_errors():
     _say("krige empty / errors")
     f, e = calc_field_krige_and_variance(np.zeros((0, 0)), np.zeros((0, 6)), np.zeros(0))
