@@ -64,6 +64,8 @@ struct MfmaGeom {
     int g2;               // 1: k_mfma_grid3 (16 i1 x 16 i2 column tiles); 16: k_mfma_grid
     int64_t t1, t2;       // column tiles along i1 / i2 (k_mfma_grid: 1 x tiles of 256 flat columns)
     int64_t row_tiles, col_tiles;
+    // mirrored row axis (k_mfma_grid3): half rows per tile, row tiles, column tiles along i1
+    int64_t mhalf, mrow_tiles, mt1;
     int64_t a_elems, e1_elems, e2_elems;
 };
 
@@ -84,6 +86,11 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
     g.t2 = g.g2 == 1 ? ceil_div(g.n2, (int64_t)16) : ceil_div(g.ncols, (int64_t)256);
     g.row_tiles = g.n0p / kMBM;
     g.col_tiles = g.t1 * g.t2;
+    // 128 half rows per tile where that pads the rows hardly more than 64 do
+    const int64_t half = (g.n0 + 1) / 2, narrow = ceil_div(half, (int64_t)64), wide = ceil_div(half, (int64_t)128);
+    g.mhalf = wide * 128 * 7 <= narrow * 64 * 8 ? 128 : 64;
+    g.mrow_tiles = g.mhalf == 128 ? wide : narrow;
+    g.mt1 = g.mhalf == 128 ? ceil_div(g.n1, (int64_t)8) : g.t1;
     g.a_elems = g.n0p * 2 * g.Np;  // 16-bit elements, hi and lo tables each
     g.e1_elems = g.n1 * g.Np;      // complex float
     g.e2_elems = g.n2 * g.Np;
@@ -252,8 +259,8 @@ __device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int6
 // and 1 swapped).  The projector weight always uses cov's own rows.
 //
 // The row axis its own mirror image (and k_mfma_grid3 to follow): the A entries are
-// cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, 64 of them per tile of 128
-// table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
+// cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, g.mhalf of them per tile
+// of twice as many table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
 // thread per mode pair); E2 takes the phase of the axis's centre.  At most kMTableBlocks
 // blocks, so that the look at the axis is not repeated for every 256 entries.
 constexpr int64_t kMTableBlocks = 4096;
@@ -273,7 +280,7 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                                                      float2* __restrict__ e1,
                                                      float2* __restrict__ e2) {
     const bool mir = g.g2 == 1 && mirrored_axis(ax0, g.n0);
-    const int64_t na = mir ? (g.n0p / 2) * (g.Np / 2) : g.n0p * g.Np;
+    const int64_t na = mir ? g.mrow_tiles * g.mhalf * (g.Np / 2) : g.n0p * g.Np;
     const int64_t n1 = g.e1_elems, n2 = comps * g.e2_elems;
     for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < na + n1 + n2; t += (int64_t)gridDim.x * 256) {
         if (mir && t < na) {
@@ -294,14 +301,14 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                     }
                 }
             }
-            const int64_t at = ((r / (kMBM / 2)) * kMBM + r % (kMBM / 2)) * pitch + jp;
+            const int64_t at = ((r / g.mhalf) * 2 * g.mhalf + r % g.mhalf) * pitch + jp;
             uint32_t hi, lo;
             split2<FP16>(c2[0], c2[1], hi, lo);
             a_hi[at] = hi;
             a_lo[at] = lo;
             split2<FP16>(s2[0], s2[1], hi, lo);
-            a_hi[at + (kMBM / 2) * pitch] = hi;
-            a_lo[at + (kMBM / 2) * pitch] = lo;
+            a_hi[at + g.mhalf * pitch] = hi;
+            a_lo[at + g.mhalf * pitch] = lo;
         } else if (t < na) {
             const int64_t row = t / g.Np, j = t - row * g.Np;
             float re = 0.0f, im = 0.0f;
@@ -567,11 +574,12 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
 // 16 B) hit 8 distinct groups, for the reads (8 rows) and the stores:
 //   A row r (64 B = 4 chunks, two rows per 128 B):  chunk c stored at c ^ ((r >> 1) & 3)
 //   E row r (128 B = 8 chunks):                      chunk c stored at c ^ (r & 7)
+template <bool WIDE>
 struct alignas(16) Stage3 {
-    uint32_t ah[kMBM * 16];
-    uint32_t al[kMBM * 16];
-    float e1[16 * 64];  // 16 modes per step: the first 16 * 32
-    float e2[16 * 64];
+    uint32_t ah[(WIDE ? 2 : 1) * kMBM * 16];
+    uint32_t al[(WIDE ? 2 : 1) * kMBM * 16];
+    float e1[16 * (WIDE ? 32 : 64)];  // 16 rows of 16 modes or 8 of 32; 16 of 32
+    float e2[16 * 64];                 // 16 rows, 16 modes per step: the first 16 * 32
 };
 
 // MIRROR: the row axis is its own mirror image about x_c (every regular axis), so with
@@ -583,22 +591,34 @@ struct alignas(16) Stage3 {
 // cosines (times the real parts of B), its last 64 the sines (times the imaginary parts);
 // a K step is 32 modes, so A stage, accumulators and instructions per step stay as they are
 // and only the B fragments double (two of 32 modes in place of one of 16).
-// 512^3, N = 4096, bf16: 4.36 -> 2.69 ms; 3 x 128^3, N = 4096: 242 -> 161 us.
-// What bounds it now: a stream of matrix instructions leaves the SIMD's other wave hardly any
-// vector issue slots, so the 320 vector instructions that build the B fragments of a step
-// add to its 96 matrix instructions (1604 of 2288 cycles per wave and step).  Building half of
-// them between the products, priorities and v_dot2 for the remainders gained nothing or lost.
-template <bool FP16, bool SPLIT, bool MIRROR>
-__device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const MfmaGeom& g, double alpha,
+// WIDE: 128 half rows x 8 i1 x 16 i2 per block instead of 64 x 16 x 16: a wave then has 256 A
+// rows to 2 column fragments, half the B fragments for the same products, and reads the A
+// tile twice as often (36 -> 44 LDS reads per step).  Taken where 128-row padding costs at most
+// an eighth more than 64 (mfma_geom).
+// 512^3, N = 4096, bf16 4.36 -> 2.69 (64) -> 2.42 ms (128), fp16 4.9 -> 3.3 -> 2.8; 3 x 128^3, N =
+// 4096 (64): 242 -> 161 us.
+// What bounds it: a stream of matrix instructions leaves the SIMD's other wave hardly any
+// vector issue slots, so the vector instructions that build the B fragments of a step (320,
+// WIDE 160) add to its 96 matrix instructions (64: 1604 of 2288 cycles per wave and step).
+// Building half of them between the products, priorities, v_dot2 for the remainders and A reads
+// two fragments ahead gained nothing or lost.
+template <bool FP16, bool SPLIT, bool MIRROR, bool WIDE>
+__device__ __forceinline__ void mfma_grid3_tile(Stage3<WIDE>& st0, Stage3<WIDE>& st1,
+                                                const MfmaGeom& g, double alpha,
                                                 const uint32_t* __restrict__ a_hi,
                                                 const uint32_t* __restrict__ a_lo,
                                                 const float2* __restrict__ e1, const float2* __restrict__ e2,
                                                 float* __restrict__ out, int64_t out_stride, int64_t comps,
-                                                int64_t steps_per, float* __restrict__ partial) {
+                                                int64_t parts, int64_t steps_per, float* __restrict__ partial) {
     constexpr int kStep = MIRROR ? 2 * kMKM : kMKM;  // modes per K step
     constexpr int kEP = kStep * 2;                   // floats per E row of a stage
     constexpr int kECh = kEP / 4;                    // 16-byte chunks per E row
     const int64_t apitch = MIRROR ? g.Np / 2 : g.Np;
+    constexpr bool kWide = MIRROR && WIDE;
+    constexpr int kRows = kWide ? 2 * kMBM : kMBM;  // A rows of the tile
+    constexpr int kRF = kRows / 16;                 // and their 16-row fragments
+    constexpr int kCF = kWide ? 2 : kMCF;           // 16-column fragments per wave: E1 rows
+    constexpr int kE1 = kMWaves * kCF;              // E1 rows of the block
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -606,8 +626,11 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
     const int l16 = lane & 15;
 
     // block index = (K split, component, tile), as in k_mfma_grid
-    const int64_t ntile = g.row_tiles * g.col_tiles;
+    const int64_t row_tiles = MIRROR ? g.mrow_tiles : g.row_tiles;
+    const int64_t col_tiles = MIRROR ? g.mt1 * g.t2 : g.col_tiles;
+    const int64_t ntile = row_tiles * col_tiles;
     const int64_t rest = (int64_t)blockIdx.x / ntile;
+    if (rest >= parts) return;  // the grid covers the larger of both forms' tile counts
     const int64_t b = (int64_t)blockIdx.x - rest * ntile;
     const int64_t comp = rest % comps, split = SPLIT ? rest / comps : 0;
     e2 += comp * g.e2_elems;
@@ -615,8 +638,8 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
     int64_t rt, ct;
     {
         const int64_t xcd = b & 7, w = b >> 3;
-        const int64_t R = g.row_tiles;
-        if (R <= 8 && (8 % R) == 0 && (g.col_tiles % (8 / R)) == 0) {
+        const int64_t R = row_tiles;
+        if (R <= 8 && (8 % R) == 0 && (col_tiles % (8 / R)) == 0) {
             const int64_t per = 8 / R;
             rt = xcd / per;
             ct = w * per + (xcd % per);
@@ -626,11 +649,12 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
         }
     }
     const int64_t tile1 = ct / g.t2, tile2 = ct - tile1 * g.t2;
-    const int64_t i1b = tile1 * 16, i2b = tile2 * 16, row0 = rt * kMBM;
+    const int64_t i1b = tile1 * kE1, i2b = tile2 * 16, row0 = rt * kRows;
 
     // each K step, each thread fills two 16-byte LDS slots of the A tile (hi and lo: slots
     // tid and tid + 256, row q >> 2) and one of E: threads 0..127 -> E1, 128..255 -> E2
-    // (row (tid & 127) >> 3); 32 modes per step: one of E1 and one of E2 (row tid >> 4)
+    // (row (tid & 127) >> 3); 32 modes per step: one of E1 and one of E2 (row tid >> 4);
+    // 256 A rows: four of the A tile, and E1's 8 rows by the first two waves
     const int erow = MIRROR ? tid >> 4 : (tid & 127) >> 3;
     const bool is_e1 = tid < 128;
     const int64_t i1e = i1b + erow < g.n1 ? i1b + erow : g.n1 - 1;
@@ -638,19 +662,22 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
     // global -> LDS loads: lane l of an instruction writes 16 B at the wave's LDS base + 16 l,
     // so each lane fetches the global chunk that the swizzled layout puts at its LDS slot
     const int wv = __builtin_amdgcn_readfirstlane(wave);
-    int64_t aoff[2];
+    constexpr int kAH = kRows / 64;  // A slots per thread and table
+    int64_t aoff[kAH];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kAH; ++h) {
         const int q = h * 256 + wv * 64 + lane;
         const int r = q >> 2;
         aoff[h] = (row0 + r) * apitch + (((q & 3) ^ ((r >> 1) & 3)) * 4);
     }
     const int echunk = ((tid & (kECh - 1)) ^ (erow & 7)) * 2;
-    const float2* ebase = (MIRROR || is_e1) ? e1 + i1e * g.Np + echunk : e2 + i2e * g.Np + echunk;
+    // the wide form's E1 rows are not swizzled: four addresses a read, in different banks
+    const int e1chunk = kWide ? (tid & (kECh - 1)) * 2 : echunk;
+    const float2* ebase = (MIRROR || is_e1) ? e1 + i1e * g.Np + e1chunk : e2 + i2e * g.Np + echunk;
     const float2* ebase2 = e2 + i2e * g.Np + echunk;  // MIRROR only
-    auto load = [&](int64_t step, Stage3& S) {
+    auto load = [&](int64_t step, Stage3<WIDE>& S) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < kAH; ++h) {
             const int slot = (h * 256 + wv * 64) * 4;
             __builtin_amdgcn_global_load_lds((const void*)(a_hi + aoff[h] + step * kMKM),
                                              (__attribute__((address_space(3))) void*)&S.ah[slot], 16, 0, 0);
@@ -658,18 +685,19 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
                                              (__attribute__((address_space(3))) void*)&S.al[slot], 16, 0, 0);
         }
         float* es = MIRROR ? S.e1 + wv * 256 : (wv < 2 ? S.e1 : S.e2) + (wv & 1) * 256;
-        __builtin_amdgcn_global_load_lds((const void*)(ebase + step * kStep),
-                                         (__attribute__((address_space(3))) void*)es, 16, 0, 0);
+        if (!kWide || wv < kE1 / 4)
+            __builtin_amdgcn_global_load_lds((const void*)(ebase + step * kStep),
+                                             (__attribute__((address_space(3))) void*)es, 16, 0, 0);
         if constexpr (MIRROR)
             __builtin_amdgcn_global_load_lds((const void*)(ebase2 + step * kStep),
                                              (__attribute__((address_space(3))) void*)(S.e2 + wv * 256), 16, 0, 0);
     };
 
-    f32x4 acc[kMRF][kMCF];
+    f32x4 acc[kRF][kCF];
 #pragma unroll
-    for (int rf = 0; rf < kMRF; ++rf)
+    for (int rf = 0; rf < kRF; ++rf)
 #pragma unroll
-        for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int cf = 0; cf < kCF; ++cf) acc[rf][cf] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int64_t steps = g.Np / kStep;
     const int64_t per = MIRROR ? steps_per / 2 : steps_per;  // steps_per: even, in steps of 16 modes
@@ -680,7 +708,7 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
     __syncthreads();
     const int zsw = l16 & 7;
     // one K step on stage C while stage Nx receives the next step's tiles
-    auto step = [&](const Stage3& C, Stage3& Nx, int64_t s) {
+    auto step = [&](const Stage3<WIDE>& C, Stage3<WIDE>& Nx, int64_t s) {
         if (s + 1 < s1) load(s + 1, Nx);
         // B fragments: E2 of this lane's i2 (row l16) times E1 of each fragment's i1; lane
         // group grp takes modes kQ grp ... of the step (a fragment's K elements 8 grp ...: the
@@ -701,7 +729,7 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
         constexpr int kLoBits = MIRROR ? 2 : 1;
         const float* zr = C.e2 + l16 * kEP + (grp ^ (zsw >> kLoBits)) * (2 * kQ);
         const int zlo = zsw & ((1 << kLoBits) - 1);
-        float2 zf[kQ], yf[kMCF][kQ];
+        float2 zf[kQ], yf[kCF][kQ];
 #pragma unroll
         for (int q = 0; q < kQ / 2; ++q) {
             const float4 v = *reinterpret_cast<const float4*>(zr + ((q ^ zlo) * 4));
@@ -710,11 +738,12 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
         }
         auto read_y = [&](int cf) {
             // row er = 4 wave + cf, swizzle er & 7 = 4 (wave & 1) + cf
-            const float* yr = C.e1 + (wave * kMCF + cf) * kEP +
-                              (MIRROR ? (grp ^ (wave & 1)) : (grp ^ ((wave & 1) * 2 + (cf >> 1)))) * (2 * kQ);
+            const float* yr =
+                C.e1 + (wave * kCF + cf) * kEP +
+                (kWide ? grp : MIRROR ? (grp ^ (wave & 1)) : (grp ^ ((wave & 1) * 2 + (cf >> 1)))) * (2 * kQ);
 #pragma unroll
             for (int q = 0; q < kQ / 2; ++q) {
-                const float4 v = *reinterpret_cast<const float4*>(yr + ((q ^ (cf & ((1 << kLoBits) - 1))) * 4));
+                const float4 v = *reinterpret_cast<const float4*>(yr + ((q ^ (kWide ? 0 : cf & ((1 << kLoBits) - 1))) * 4));
                 yf[cf][2 * q] = {v.x, v.y};
                 yf[cf][2 * q + 1] = {v.z, v.w};
             }
@@ -724,12 +753,12 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
 
         // fragments [real, imaginary parts][column fragment]; without MIRROR one of the pairs
         constexpr int kParts = MIRROR ? 2 : 1;
-        u32x4 bh[kParts][kMCF], bl[kParts][kMCF];
+        u32x4 bh[kParts][kCF], bl[kParts][kCF];
 #pragma unroll
-        for (int cf = 0; cf < kMCF; ++cf) {
+        for (int cf = 0; cf < kCF; ++cf) {
             __builtin_amdgcn_sched_barrier(0);
-            if (cf + 2 < kMCF) read_y(cf + 2);
-            if (cf + 2 == kMCF) read_a(0);
+            if (cf + 2 < kCF) read_y(cf + 2);
+            if (cf + 2 == kCF) read_a(0);
             uint32_t h, l;
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -751,17 +780,17 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
         }
 
 #pragma unroll
-        for (int rf = 0; rf < kMRF; ++rf) {
-            const int part = MIRROR && rf >= kMRF / 2 ? 1 : 0;
-            if (rf + 1 < kMRF) read_a(rf + 1);
+        for (int rf = 0; rf < kRF; ++rf) {
+            const int part = MIRROR && rf >= kRF / 2 ? 1 : 0;
+            if (rf + 1 < kRF) read_a(rf + 1);
             __builtin_amdgcn_sched_barrier(0);
-            // the products of one accumulator lie kMCF instructions apart
+            // the products of one accumulator lie kCF instructions apart
 #pragma unroll
-            for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = mfma<FP16>(ah[rf & 1], bh[part][cf], acc[rf][cf]);
+            for (int cf = 0; cf < kCF; ++cf) acc[rf][cf] = mfma<FP16>(ah[rf & 1], bh[part][cf], acc[rf][cf]);
 #pragma unroll
-            for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = mfma<FP16>(ah[rf & 1], bl[part][cf], acc[rf][cf]);
+            for (int cf = 0; cf < kCF; ++cf) acc[rf][cf] = mfma<FP16>(ah[rf & 1], bl[part][cf], acc[rf][cf]);
 #pragma unroll
-            for (int cf = 0; cf < kMCF; ++cf) acc[rf][cf] = mfma<FP16>(al[rf & 1], bh[part][cf], acc[rf][cf]);
+            for (int cf = 0; cf < kCF; ++cf) acc[rf][cf] = mfma<FP16>(al[rf & 1], bh[part][cf], acc[rf][cf]);
         }
         // the next step's LDS loads have landed (the barrier's own wait covers LDS, not them)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -775,25 +804,25 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
     const float fa = SPLIT ? 1.0f : (float)alpha;  // partial sums are scaled when added
     const int64_t i2 = i2b + l16;
 #pragma unroll
-    for (int cf = 0; cf < kMCF; ++cf) {
-        const int64_t i1 = i1b + wave * kMCF + cf;
+    for (int cf = 0; cf < kCF; ++cf) {
+        const int64_t i1 = i1b + wave * kCF + cf;
         if (i1 >= g.n1 || i2 >= g.n2) continue;
         if (i1 * g.n2 + i2 >= g.out_cols) continue;  // past the end of a split axis
         const int64_t col = i1 * g.c1s + i2;
         if constexpr (MIRROR) {
 #pragma unroll
-            for (int rf = 0; rf < kMRF / 2; ++rf) {
+            for (int rf = 0; rf < kRF / 2; ++rf) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int64_t row = rt * (kMBM / 2) + rf * 16 + grp * 4 + i;
-                    const float c = acc[rf][cf][i], sn = acc[rf + kMRF / 2][cf][i];
+                    const int64_t row = rt * (kRows / 2) + rf * 16 + grp * 4 + i;
+                    const float c = acc[rf][cf][i], sn = acc[rf + kRF / 2][cf][i];
                     if (2 * row < g.n0) out[row * g.rs + col] = fa * (c + sn);
                     if (2 * row + 1 < g.n0) out[(g.n0 - 1 - row) * g.rs + col] = fa * (c - sn);
                 }
             }
         } else {
 #pragma unroll
-            for (int rf = 0; rf < kMRF; ++rf) {
+            for (int rf = 0; rf < kRF; ++rf) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int64_t row = row0 + rf * 16 + grp * 4 + i;
@@ -804,7 +833,8 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3& st0, Stage3& st1, const 
     }
 }
 
-template <bool FP16, bool SPLIT>
+// WIDE: g.mhalf is 128
+template <bool FP16, bool SPLIT, bool WIDE>
 __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, double alpha,
                                                                 const double* __restrict__ ax0,
                                                                 const uint32_t* __restrict__ a_hi,
@@ -812,19 +842,19 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid3(MfmaGeom g, doub
                                                                 const float2* __restrict__ e1,
                                                                 const float2* __restrict__ e2,
                                                                 float* __restrict__ out, int64_t out_stride,
-                                                                int64_t comps, int64_t steps_per,
+                                                                int64_t comps, int64_t parts, int64_t steps_per,
                                                                 float* __restrict__ partial) {
     // two stages as separate LDS objects, the step loop unrolled by two: the compiler
     // then sees that a step's LDS reads and the next step's global -> LDS loads touch
     // different objects and does not wait for those loads before the reads
-    __shared__ Stage3 st0;
-    __shared__ Stage3 st1;
+    __shared__ Stage3<WIDE> st0;
+    __shared__ Stage3<WIDE> st1;
     if (mirrored_axis(ax0, g.n0))  // one value for the launch, and that of its tables
-        mfma_grid3_tile<FP16, SPLIT, true>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
-                                           steps_per, partial);
+        mfma_grid3_tile<FP16, SPLIT, true, WIDE>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
+                                                 parts, steps_per, partial);
     else
-        mfma_grid3_tile<FP16, SPLIT, false>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
-                                            steps_per, partial);
+        mfma_grid3_tile<FP16, SPLIT, false, WIDE>(st0, st1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
+                                                  parts, steps_per, partial);
 }
 
 // out[i] = alpha * sum_k partial[k * n + i], k in order (K-split partial sums)
@@ -899,12 +929,17 @@ int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t c
                                            ceil_div(mfma_table_bytes(g, comps), (int64_t)256) * 256);
     const dim3 grid((unsigned)blocks), block(kMWaves * 64);
     if (g.g2 == 1) {
-        if (ksplit > 1)
-            hipLaunchKernelGGL((k_mfma_grid3<FP16, true>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2, out,
-                               stride, comps, steps_per, partial);
+        // blocks of the form with more tiles (the axis is looked at on the device)
+        const int64_t parts = ksplit * comps, mtiles = g.mrow_tiles * g.mt1 * g.t2;
+        const dim3 grid3((unsigned)(mtiles * parts > blocks ? mtiles * parts : blocks));
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid3, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2, out, stride, comps, parts,
+                               steps_per, partial);
+        };
+        if (g.mhalf == 128)
+            ksplit > 1 ? go(k_mfma_grid3<FP16, true, true>) : go(k_mfma_grid3<FP16, false, true>);
         else
-            hipLaunchKernelGGL((k_mfma_grid3<FP16, false>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2,
-                               out, stride, comps, steps_per, partial);
+            ksplit > 1 ? go(k_mfma_grid3<FP16, true, false>) : go(k_mfma_grid3<FP16, false, false>);
     } else if (d == 2) {
         if (ksplit > 1)
             hipLaunchKernelGGL((k_mfma_grid<FP16, true, true>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2,
@@ -957,7 +992,7 @@ int mfma_entry(int64_t d, int64_t N, const int64_t* shape, const double* axes, c
     const MfmaPlan plan = mfma_plan(d, N, shape, comps, uniform_last, fill, !no_swap);
     const MfmaGeom& g = plan.g;
     const bool split = plan.split;
-    if (mfma_ksplit(g, comps, fill) * comps * g.row_tiles * g.col_tiles > 0x7fffffffLL ||
+    if (mfma_ksplit(g, comps, fill) * comps * (g.row_tiles + 1) * (g.col_tiles + g.t2) > 0x7fffffffLL ||
         ceil_div(comps * P, (int64_t)256) > 0x7fffffffLL)
         return GSX_E_INVALID;
     if (!workspace || workspace_bytes < mfma_plan_ws_bytes(plan, comps)) return GSX_E_WORKSPACE;
