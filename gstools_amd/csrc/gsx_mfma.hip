@@ -250,7 +250,9 @@ __device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int6
 }
 
 // --------------------------------------------------------------- tables ----
-// One thread per table entry: A (n0p x Np), E1 (n1 x Np), E2 (comps x n2 x Np).
+// A (n0p x Np), E1 (n1 x Np), E2 (comps x n2 x Np): a block takes 256 modes of one row at a time,
+// so that rows and modes need no division per entry (two 64-bit ones per entry, and a phase
+// for each component, were a quarter of 20 us for 3 x 128^3 with N = 4096; now 15).
 // comps > 1 (incompressible fields): E2 of component c carries the projector
 // weight p_c(k_j) = delta_c0 - k_jc k_j0 / |k_j|^2 (generator.py:479-494) in
 // place of the spectrum factor.
@@ -262,7 +264,7 @@ __device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int6
 // cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, g.mhalf of them per tile
 // of twice as many table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
 // thread per mode pair); E2 takes the phase of the axis's centre.  At most kMTableBlocks
-// blocks, so that the look at the axis is not repeated for every 256 entries.
+// blocks, so that the look at the axis is not repeated for every 256 modes.
 constexpr int64_t kMTableBlocks = 4096;
 
 template <bool FP16>
@@ -280,86 +282,97 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                                                      float2* __restrict__ e1,
                                                      float2* __restrict__ e2) {
     const bool mir = g.g2 == 1 && mirrored_axis(ax0, g.n0);
-    const int64_t na = mir ? g.mrow_tiles * g.mhalf * (g.Np / 2) : g.n0p * g.Np;
-    const int64_t n1 = g.e1_elems, n2 = comps * g.e2_elems;
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < na + n1 + n2; t += (int64_t)gridDim.x * 256) {
-        if (mir && t < na) {
-            const int64_t pitch = g.Np / 2;
-            const int64_t r = t / pitch, jp = t - r * pitch;
-            float c2[2] = {0.0f, 0.0f}, s2[2] = {0.0f, 0.0f};
-            if (2 * r < g.n0) {
-                const double h = 0.5 * (ax0[g.n0 - 1 - r] - ax0[r]);
+    const auto phase = [](double th, double* sn, double* cs) {
+        if (fabs(th) <= kFastPhaseMax) sincos_fast(th, sn, cs); else sincos(th, sn, cs);
+    };
+    const unsigned na = (unsigned)(mir ? g.mrow_tiles * g.mhalf : g.n0p), n1 = (unsigned)g.n1, n2 = (unsigned)g.n2;
+    const unsigned cha = (unsigned)(((mir ? g.Np / 2 : g.Np) + 255) / 256), ch = (unsigned)((g.Np + 255) / 256);
+    const unsigned items = na * cha + (n1 + n2) * ch;  // fits (the launch refuses more)
+    for (unsigned it = blockIdx.x; it < items; it += gridDim.x) {
+        if (it < na * cha) {
+            const unsigned row = it / cha;
+            const int64_t q = (int64_t)(it - row * cha) * 256 + threadIdx.x;
+            uint32_t hi, lo;
+            if (mir) {
+                const int64_t pitch = g.Np / 2, r = row;
+                if (q >= pitch) continue;
+                float c2[2] = {0.0f, 0.0f}, s2[2] = {0.0f, 0.0f};
+                if (2 * r < g.n0) {
+                    const double h = 0.5 * (ax0[g.n0 - 1 - r] - ax0[r]);
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const int64_t j = 2 * jp + e;
-                    if (j < N) {
-                        double sn, cs;
-                        const double th = cov[ka_row * N + j] * h;
-                        if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &sn, &cs); else sincos(th, &sn, &cs);
-                        c2[e] = (float)cs;
-                        s2[e] = (float)sn;
+                    for (int e = 0; e < 2; ++e) {
+                        const int64_t j = 2 * q + e;
+                        if (j < N) {
+                            double sn, cs;
+                            phase(cov[ka_row * N + j] * h, &sn, &cs);
+                            c2[e] = (float)cs;
+                            s2[e] = (float)sn;
+                        }
                     }
                 }
+                const int64_t at = ((r / g.mhalf) * 2 * g.mhalf + r % g.mhalf) * pitch + q;
+                split2<FP16>(c2[0], c2[1], hi, lo);
+                a_hi[at] = hi;
+                a_lo[at] = lo;
+                split2<FP16>(s2[0], s2[1], hi, lo);
+                a_hi[at + g.mhalf * pitch] = hi;
+                a_lo[at + g.mhalf * pitch] = lo;
+            } else {
+                if (q >= g.Np) continue;
+                float re = 0.0f, im = 0.0f;
+                if (row < g.n0 && q < N) {
+                    double sn, cs;
+                    phase(cov[ka_row * N + q] * ax0[row], &sn, &cs);
+                    re = (float)cs;
+                    im = (float)(-sn);
+                }
+                split2<FP16>(re, im, hi, lo);
+                a_hi[row * g.Np + q] = hi;  // element pair (2q, 2q+1) of row `row`
+                a_lo[row * g.Np + q] = lo;
             }
-            const int64_t at = ((r / g.mhalf) * 2 * g.mhalf + r % g.mhalf) * pitch + jp;
-            uint32_t hi, lo;
-            split2<FP16>(c2[0], c2[1], hi, lo);
-            a_hi[at] = hi;
-            a_lo[at] = lo;
-            split2<FP16>(s2[0], s2[1], hi, lo);
-            a_hi[at + g.mhalf * pitch] = hi;
-            a_lo[at + g.mhalf * pitch] = lo;
-        } else if (t < na) {
-            const int64_t row = t / g.Np, j = t - row * g.Np;
-            float re = 0.0f, im = 0.0f;
-            if (row < g.n0 && j < N) {
-                double s, c;
-                const double th = cov[ka_row * N + j] * ax0[row];
-                if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
-                re = (float)c;
-                im = (float)(-s);
-            }
-            uint32_t hi, lo;
-            split2<FP16>(re, im, hi, lo);
-            a_hi[t] = hi;  // element pair (2j, 2j+1) of row `row`
-            a_lo[t] = lo;
-        } else if (t < na + n1) {
-            const int64_t u = t - na;
-            const int64_t i1 = u / g.Np, j = u - i1 * g.Np;
+            continue;
+        }
+        const unsigned rest = it - na * cha, row = rest / ch;
+        const int64_t j = (int64_t)(rest - row * ch) * 256 + threadIdx.x;
+        if (j >= g.Np) continue;
+        if (row < n1) {
             float2 v = {0.0f, 0.0f};
             if (j < N) {
                 if (d == 3) {
-                    double s, c;
-                    const double th = cov[k1_row * N + j] * ax1[i1];
-                    if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
-                    v = {(float)c, (float)s};
+                    double sn, cs;
+                    phase(cov[k1_row * N + j] * ax1[row], &sn, &cs);
+                    v = {(float)cs, (float)sn};
                 } else {
                     v = {1.0f, 0.0f};
                 }
             }
-            e1[u] = v;
-        } else if (t < na + n1 + n2) {
-            const int64_t u = t - na - n1;
-            const int64_t comp = u / g.e2_elems, uc = u - comp * g.e2_elems;
-            const int64_t i2 = uc / g.Np, j = uc - i2 * g.Np;
+            e1[row * g.Np + j] = v;
+            continue;
+        }
+        // E2: one phase for all components
+        const unsigned i2 = row - n1;
+        double sn = 0.0, cs = 0.0, a = 0.0, b = 0.0, k0 = 0.0, k2 = 1.0;
+        if (j < N) {
+            double th = cov[kz_row * N + j] * (d == 3 ? ax2[i2] : ax1[i2]);
+            if (mir) th += cov[ka_row * N + j] * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
+            phase(th, &sn, &cs);
+            a = z1[j];
+            b = z2[j];
+            if (comps > 1) {
+                k0 = cov[j];
+                k2 = 0.0;
+                for (int64_t e = 0; e < d; ++e) k2 += cov[e * N + j] * cov[e * N + j];
+            }
+        }
+        for (int64_t comp = 0; comp < comps; ++comp) {
             float2 v = {0.0f, 0.0f};
             if (j < N) {
-                double s, c;
-                const double kz = cov[kz_row * N + j];
-                double th = kz * (d == 3 ? ax2[i2] : ax1[i2]);
-                if (mir) th += cov[ka_row * N + j] * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
-                if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &s, &c); else sincos(th, &s, &c);
-                double f = fac ? fac[j] : 1.0;
-                if (comps > 1) {
-                    double k2 = 0.0;
-                    for (int64_t e = 0; e < d; ++e) k2 += cov[e * N + j] * cov[e * N + j];
-                    f = (comp == 0 ? 1.0 : 0.0) - cov[comp * N + j] * cov[j] / k2;
-                }
-                const double a = f * z1[j], b = f * z2[j];
-                // (a - i b)(c + i s)
-                v = {(float)(a * c + b * s), (float)(a * s - b * c)};
+                const double f = comps > 1 ? (comp == 0 ? 1.0 : 0.0) - cov[comp * N + j] * k0 / k2 : fac ? fac[j] : 1.0;
+                const double fa = f * a, fb = f * b;
+                // (fa - i fb)(c + i s)
+                v = {(float)(fa * cs + fb * sn), (float)(fa * sn - fb * cs)};
             }
-            e2[u] = v;
+            e2[comp * g.e2_elems + i2 * g.Np + j] = v;
         }
     }
 }
@@ -913,8 +926,9 @@ int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t c
     uint32_t* a_lo = a_hi + g.a_elems / 2;
     float2* e1 = reinterpret_cast<float2*>(a_lo + g.a_elems / 2);
     float2* e2 = e1 + g.e1_elems;
-    const int64_t entries = g.n0p * g.Np + g.e1_elems + comps * g.e2_elems;
-    const int64_t tblocks = ceil_div(entries, (int64_t)256) < kMTableBlocks ? ceil_div(entries, (int64_t)256) : kMTableBlocks;
+    const int64_t items = (g.n0p + g.n1 + g.n2) * ceil_div(g.Np, (int64_t)256);
+    if (items > 0x7fffffffLL) return GSX_E_INVALID;
+    const int64_t tblocks = items < kMTableBlocks ? items : kMTableBlocks;
     hipLaunchKernelGGL((k_mfma_tables<FP16>), dim3((unsigned)tblocks), dim3(256), 0, s, g, d,
                        N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, a_hi, a_lo, e1, e2);
     int st = launch_status();
