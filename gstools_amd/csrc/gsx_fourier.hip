@@ -38,15 +38,14 @@ namespace gsx {
 
 typedef __attribute__((ext_vector_type(4))) double f64x4;
 
-constexpr int kFR = 128;     // C rows per block
 constexpr int kFK = 16;      // K per LDS stage
 constexpr int kFApad = kFK + 2;  // 16-byte aligned rows, operand reads over all banks
 
 // Batched real FP64 GEMM, row-major: C_b = A_b B_b, A_b (M x K, lda), B_b (K x N,
 // ldb), C_b (M x N, ldc), operand b at A + b sA, B + b sB, C + b sC.  Block =
-// (batch, row tile, column tile) of kFR x 64 WC: 4 waves in (4 / WC) x WC, each
-// (kFR WC / 4) rows x 64 columns of 16 x 16 MFMA tiles (WC = 2: 4 x 4; WC = 1,
-// for launches with few tiles or N <= 64: 2 x 4); A and B tiles staged through
+// (batch, row tile, column tile) of FR x 64 WC: 4 waves in (4 / WC) x WC, each
+// (FR WC / 4) rows x 64 columns of 16 x 16 MFMA tiles (128 x 128: 4 x 4; 128 x 64: 2 x 4;
+// 64 x 64: 1 x 4, for launches with fewer tiles); A and B tiles staged through
 // LDS with the next stage prefetched into registers.  Rows and columns past the end
 // are read from clamped addresses and not stored; K entries past the end are zero.
 // kPair: N, lda, ldb, sA, sB even and A, B 16-byte aligned, so whole stages are read as
@@ -56,13 +55,14 @@ constexpr int kFApad = kFK + 2;  // 16-byte aligned rows, operand reads over all
 // Bound by the FP64 matrix cores, which share the vector unit's issue: a vector
 // instruction in the loop costs its time, so the loop carries as few as it can.
 // 4096^2 points, 256^2 modes: the last stage (4096 x 4096 x 512) 307 -> 290 us, the first
-// (8192 x 256 x 512, 64-column tiles) 56 -> 52, from reads of 8 bytes with a check each;
-// the matrix cores are then busy 80% of the time at 2.17 GHz.  A second LDS buffer (one
+// (8192 x 256 x 512) 56 -> 52, from reads of 8 bytes with a check each, and -> 45 in 512 tiles
+// of 64 x 64 instead of 256 of 128 x 64 (two waves per SIMD); the matrix cores are busy 80%
+// of the last stage at 2.17 GHz.  A second LDS buffer (one
 // barrier a stage) changed neither.
 // v_mfma_f64_16x16x4 layouts (g = lane / 16): A: lane holds row lane % 16, K
 // element g; B: column lane % 16, K element g; C: column lane % 16, register r
 // holds row g + 4 r.
-template <int WC, bool kPair>
+template <int FR, int WC, bool kPair>
 __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, int64_t K,
                                                           const double* __restrict__ A, int64_t lda, int64_t sA,
                                                           const double* __restrict__ B, int64_t ldb, int64_t sB,
@@ -71,10 +71,11 @@ __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, 
     typedef __attribute__((ext_vector_type(2))) double f64x2;
     constexpr int kBC = 64 * WC;            // block columns
     constexpr int kBpad = kBC + 16;
-    constexpr int kRF = kFR * WC / 4 / 16;  // 16-row MFMA tiles per wave
+    constexpr int kRF = FR * WC / 4 / 16;  // 16-row MFMA tiles per wave
     constexpr int kBW = kPair ? 2 : 1;      // columns per staging thread
     constexpr int kBT = 256 * kBW / kBC;    // B rows staged per pass
-    __shared__ __align__(16) double As[kFR * kFApad];
+    constexpr int kAC = FR / 16;            // A columns per staging thread
+    __shared__ __align__(16) double As[FR * kFApad];
     __shared__ __align__(16) double Bs[kFK * kBpad];
     const int t = threadIdx.x;
     const int lane = t & 63, wave = t >> 6;
@@ -87,20 +88,20 @@ __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, 
     A += bt * sA;
     B += bt * sB;
     C += bt * sC;
-    const int64_t i0 = rt * kFR, p0 = ct * kBC;
+    const int64_t i0 = rt * FR, p0 = ct * kBC;
 
-    // staging: A kFR x 16 (two threads per row, 8 consecutive each); B 16 x kBC (kBW
+    // staging: A FR x 16 (kAC consecutive columns per thread); B 16 x kBC (kBW
     // columns of rows t / (kBC / kBW) + kBT u)
-    const int ar = t >> 1, ac = (t & 1) * 8;
+    const int ar = t / (16 / kAC), ac = t % (16 / kAC) * kAC;
     const int br = t / (kBC / kBW), bc = t % (kBC / kBW) * kBW;
     const double* arow = A + (i0 + ar < M ? i0 + ar : M - 1) * lda + ac;
     const int64_t pc = p0 + bc < N ? p0 + bc : (kPair ? (N - 1) / 2 * 2 : N - 1);
     const double* brow = B + br * ldb + pc;
-    double pa[8], pb[kBW * kFK / kBT];
+    double pa[kAC], pb[kBW * kFK / kBT];
     auto load_whole = [&](int64_t j0) {
         if constexpr (kPair) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
+            for (int u = 0; u < kAC / 2; ++u) {
                 const f64x2 v = *reinterpret_cast<const f64x2*>(arow + j0 + 2 * u);
                 pa[2 * u] = v.x;
                 pa[2 * u + 1] = v.y;
@@ -113,14 +114,14 @@ __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, 
             }
         } else {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) pa[u] = arow[j0 + u];
+            for (int u = 0; u < kAC; ++u) pa[u] = arow[j0 + u];
 #pragma unroll
             for (int u = 0; u < kFK / kBT; ++u) pb[u] = brow[(j0 + kBT * u) * ldb];
         }
     };
     auto load_tail = [&](int64_t j0) {  // the last stage when K is no multiple of 16
 #pragma unroll
-        for (int u = 0; u < 8; ++u) pa[u] = j0 + ac + u < K ? arow[j0 + u] : 0.0;
+        for (int u = 0; u < kAC; ++u) pa[u] = j0 + ac + u < K ? arow[j0 + u] : 0.0;
 #pragma unroll
         for (int u = 0; u < kFK / kBT; ++u)
 #pragma unroll
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(256, 2) void k_fourier_dgemm(int64_t M, int64_t N, 
     };
     auto store = [&]() {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < kAC / 2; ++u)
             *reinterpret_cast<f64x2*>(&As[ar * kFApad + ac + 2 * u]) = f64x2{pa[2 * u], pa[2 * u + 1]};
 #pragma unroll
         for (int u = 0; u < kFK / kBT; ++u) {
@@ -287,12 +288,15 @@ inline bool fourier_tensor_plan(int64_t d, const int64_t* mode_no, const int64_t
 inline int dgemm(int64_t M, int64_t N, int64_t K, int64_t batch, const double* A, int64_t lda, int64_t sA,
                  const double* B, int64_t ldb, int64_t sB, double* C, int64_t ldc, int64_t sC, hipStream_t s) {
     if (M == 0 || N == 0 || batch == 0) return GSX_OK;
-    const int64_t rt = ceil_div(M, (int64_t)kFR);
-    // 128-column tiles unless that leaves the chip (256 CUs) under-filled or
-    // half of each tile empty: then 64-column tiles
-    const int64_t ct2 = ceil_div(N, (int64_t)128), ct1 = ceil_div(N, (int64_t)64);
-    const bool narrow = N <= 64 || batch * rt * ct2 < 256;
-    const int64_t ct = narrow ? ct1 : ct2;
+    // 128 x 128 tiles unless that leaves the chip (256 CUs) under-filled or half of each tile
+    // empty, then 128 x 64, and 64 x 64 where those come to less than two per CU
+    const int64_t ct2 = ceil_div(N, (int64_t)128), ct1 = ceil_div(N, (int64_t)64), rt2 = ceil_div(M, (int64_t)128);
+    const bool narrow = N <= 64 || batch * rt2 * ct2 < 256;
+    const bool low = narrow && batch * rt2 * ct1 < 512;
+    // 64 x 128 where 128-row tiles would pad the rows by an eighth more (150 rows: 256, not 192)
+    const int64_t rt1 = ceil_div(M, (int64_t)64);
+    const bool flat = !narrow && rt1 * 64 * 9 < rt2 * 128 * 8;
+    const int64_t ct = narrow ? ct1 : ct2, rt = low || flat ? rt1 : rt2;
     if (batch * rt * ct > 0x7fffffffLL) return GSX_E_INVALID;
     const bool pair = lda % 2 == 0 && ldb % 2 == 0 && sA % 2 == 0 && sB % 2 == 0 && N % 2 == 0 &&
                       reinterpret_cast<uintptr_t>(A) % 16 == 0 && reinterpret_cast<uintptr_t>(B) % 16 == 0;
@@ -300,10 +304,14 @@ inline int dgemm(int64_t M, int64_t N, int64_t K, int64_t batch, const double* A
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, M, N, K, A, lda, sA, B, ldb, sB, C, ldc, sC, rt, ct);
     };
-    if (narrow)
-        pair ? go(k_fourier_dgemm<1, true>) : go(k_fourier_dgemm<1, false>);
+    if (low)
+        pair ? go(k_fourier_dgemm<64, 1, true>) : go(k_fourier_dgemm<64, 1, false>);
+    else if (flat)
+        pair ? go(k_fourier_dgemm<64, 2, true>) : go(k_fourier_dgemm<64, 2, false>);
+    else if (narrow)
+        pair ? go(k_fourier_dgemm<128, 1, true>) : go(k_fourier_dgemm<128, 1, false>);
     else
-        pair ? go(k_fourier_dgemm<2, true>) : go(k_fourier_dgemm<2, false>);
+        pair ? go(k_fourier_dgemm<128, 2, true>) : go(k_fourier_dgemm<128, 2, false>);
     return launch_status();
 }
 

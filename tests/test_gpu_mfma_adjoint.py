@@ -203,6 +203,26 @@ def test_fp64gemm_grid_matches_oracle(shape, n):
     assert rel_max <= 1e-12
 
 
+@pytest.mark.parametrize("shape,n", [
+    ((150, 130, 160), 33),  # 64 x 128 tiles, a last K stage of 2
+    ((250, 130, 160), 40),  # 128 x 128 tiles, whole K stages
+    ((150, 131, 161), 37),  # the same with an odd row length: single reads
+    ((250, 131, 161), 8),
+    ((300, 61, 64), 17),    # 128 x 64 tiles
+    ((65, 50, 3), 50),      # 64 x 64 tiles
+    ((1, 1, 7), 1),
+])
+def test_fp64gemm_tile_forms(shape, n):
+    """Every tile form of the FP64 GEMM, with ragged rows, columns and K, against the direct
+    FP64 sum: phases of at most a few hundred radians, so within 1e-12."""
+    _say(f"fp64gemm tiles shape={shape} N={n}")
+    cov, z1, z2 = _modes(3, n, 5 + n, kscale=0.6)
+    axes = [np.linspace(-3.0 * (i + 1), 11.0 + 2 * i, s) for i, s in enumerate(shape)]
+    ref = summate_grid_device(cov, z1, z2, axes, "fp64").cpu().numpy()
+    got = summate_grid_device(cov, z1, z2, axes, "fp64gemm").cpu().numpy()
+    assert oracle.rel_errors(got, ref)[0] <= 1e-12
+
+
 def test_fp64gemm_generators():
     """RandMeth.structured and the Fourier method's direct route take "fp64gemm"; the
     incompressible grid entry refuses it."""
