@@ -105,12 +105,24 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
 constexpr int64_t kMFillBlocks = 512;
 constexpr int kMFillLog2Min = 8, kMFillLog2Max = 11;
 
+// Between two and four fifths of that (k_mfma_grid3), half of the CUs have one block and a
+// step of two blocks on a CU takes 4576 cycles, of one 2900: twice the splits, two blocks
+// and then one on every CU, save about 840 cycles (0.4 us) per 32-mode step of the fewer
+// splits, and cost the partial sums' way through memory (about 9 TB/s) once more.
+// 3 x 128^3, N = 4096: 384 blocks 216 us, 768 blocks 202.
+//
 // (>= 1 also with no K steps or no tiles: those launch nothing)
 inline int64_t mfma_steps_per_split(const MfmaGeom& g, int64_t comps, int64_t fill = kMFillBlocks) {
     const int64_t blocks = comps * g.row_tiles * g.col_tiles;
     const int64_t steps = g.Np / kMKM;
     if (steps < 1 || blocks < 1) return 1;
     int64_t k = blocks >= fill ? 1 : fill / blocks;
+    if (g.g2 == 1 && blocks * k * 2 > fill && blocks * k * 5 <= fill * 4) {
+        const double partial_bytes = 4.0 * (double)(comps * g.n0) * (double)g.out_cols;
+        // k == 1 writes no partial sums at all
+        const double more = 2.0 * (double)(k == 1 ? 2 : k) * partial_bytes / 9e12;
+        if (0.4e-6 * (double)(steps / 2) / (double)k > 1.2 * more) k *= 2;
+    }
     if (k > steps / 8) k = steps / 8;
     if (k < 1) k = 1;
     const int64_t per = ceil_div(steps, k);
