@@ -64,7 +64,7 @@ struct MfmaGeom {
     int g2;               // 1: k_mfma_grid3 (16 i1 x 16 i2 column tiles); 16: k_mfma_grid
     int64_t t1, t2;       // column tiles along i1 / i2 (k_mfma_grid: 1 x tiles of 256 flat columns)
     int64_t row_tiles, col_tiles;
-    // mirrored row axis (k_mfma_grid3): half rows per tile, row tiles, column tiles along i1
+    // mirrored row axis: half rows per tile, row tiles, column tiles along i1
     int64_t mhalf, mrow_tiles, mt1;
     int64_t a_elems, e1_elems, e2_elems;
 };
@@ -76,8 +76,7 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
     g.n2 = d == 3 ? shape[2] : shape[1];
     g.n0p = ceil_div(g.n0, kMBM) * kMBM;
     g.g2 = (g.n1 >= 16 && g.n2 >= 16) ? 1 : 16;
-    // k_mfma_grid3 may step 32 modes at a time
-    g.Np = g.g2 == 1 ? ceil_div(N, 2 * kMKM) * 2 * kMKM : ceil_div(N, kMKM) * kMKM;
+    g.Np = ceil_div(N, 2 * kMKM) * 2 * kMKM;  // a mirrored row axis steps 32 modes at a time
     g.ncols = g.n1 * g.n2;
     g.out_cols = g.ncols;
     g.rs = g.ncols;
@@ -86,9 +85,9 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
     g.t2 = g.g2 == 1 ? ceil_div(g.n2, (int64_t)16) : ceil_div(g.ncols, (int64_t)256);
     g.row_tiles = g.n0p / kMBM;
     g.col_tiles = g.t1 * g.t2;
-    // 128 half rows per tile where that pads the rows hardly more than 64 do
+    // (k_mfma_grid3) 128 half rows per tile where that pads the rows hardly more than 64 do
     const int64_t half = (g.n0 + 1) / 2, narrow = ceil_div(half, (int64_t)64), wide = ceil_div(half, (int64_t)128);
-    g.mhalf = wide * 128 * 7 <= narrow * 64 * 8 ? 128 : 64;
+    g.mhalf = g.g2 == 1 && wide * 128 * 7 <= narrow * 64 * 8 ? 128 : 64;
     g.mrow_tiles = g.mhalf == 128 ? wide : narrow;
     g.mt1 = g.mhalf == 128 ? ceil_div(g.n1, (int64_t)8) : g.t1;
     g.a_elems = g.n0p * 2 * g.Np;  // 16-bit elements, hi and lo tables each
@@ -126,7 +125,7 @@ inline int64_t mfma_steps_per_split(const MfmaGeom& g, int64_t comps, int64_t fi
     if (k > steps / 8) k = steps / 8;
     if (k < 1) k = 1;
     const int64_t per = ceil_div(steps, k);
-    return g.g2 == 1 ? ceil_div(per, (int64_t)2) * 2 : per;  // whole 32-mode steps
+    return ceil_div(per, (int64_t)2) * 2;  // whole 32-mode steps
 }
 
 inline int64_t mfma_ksplit(const MfmaGeom& g, int64_t comps, int64_t fill = kMFillBlocks) {
@@ -244,7 +243,7 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
 // ---------------------------------------------------------------- mirror ---
 // Whether the row axis x (n0 points) is its own mirror image, x_r + x_(n0-1-r) == x_0 +
 // x_(n0-1) to 4 ulp of max(|x_0|, |x_(n0-1)|) for every r (a NaN or infinity: no).  Every
-// block of the tables and of k_mfma_grid3 looks for itself (about a microsecond for 512
+// block of the tables and of the GEMMs looks for itself (about a microsecond for 512
 // points, less than a launch to look once); longer axes than kMMirrorMax count as not
 // mirrored.  Called by the whole block.
 constexpr int64_t kMMirrorMax = 4096;
@@ -272,7 +271,7 @@ __device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int6
 // and E2 (0, 1, d - 1; 1, 1 for a split axis's two virtual axes; 1, 0, 2 with axes 0
 // and 1 swapped).  The projector weight always uses cov's own rows.
 //
-// The row axis its own mirror image (and k_mfma_grid3 to follow): the A entries are
+// The row axis its own mirror image: the A entries are
 // cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, g.mhalf of them per tile
 // of twice as many table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
 // thread per mode pair); E2 takes the phase of the axis's centre.  At most kMTableBlocks
@@ -293,7 +292,8 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                                                      uint32_t* __restrict__ a_lo,
                                                      float2* __restrict__ e1,
                                                      float2* __restrict__ e2) {
-    const bool mir = g.g2 == 1 && mirrored_axis(ax0, g.n0);
+    // (the flat kernel's 3D form takes no account of it: its second E table leaves no registers)
+    const bool mir = (g.g2 == 1 || d == 2) && mirrored_axis(ax0, g.n0);
     const auto phase = [](double th, double* sn, double* cs) {
         if (fabs(th) <= kFastPhaseMax) sincos_fast(th, sn, cs); else sincos(th, sn, cs);
     };
@@ -407,23 +407,19 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
 
 // E1ONE: the grid has a one-point middle axis (2D grids), E1 == 1, so B is E2.
 // SPLIT: the K steps are split over blocks (small grids), partial sums written.
-template <bool FP16, bool E1ONE, bool SPLIT>
-__global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, double alpha,
-                                                               const uint32_t* __restrict__ a_hi,
-                                                               const uint32_t* __restrict__ a_lo,
-                                                               const float2* __restrict__ e1,
-                                                               const float2* __restrict__ e2,
-                                                               float* __restrict__ out, int64_t out_stride,
-                                                               int64_t comps, int64_t steps_per,
-                                                               float* __restrict__ partial) {
-    // two stages [hi/lo][row * 16 + chunk * 4]: 64-byte A rows, 16-byte chunk c of row r
-    // stored at c ^ ((r >> 1) & 3) (the 8 lanes of a 16-byte LDS access phase hit 8 bank
-    // groups).  The stages are separate LDS objects and the step loop is unrolled by two,
-    // so the compiler sees that a step's LDS reads and the next step's global -> LDS loads
-    // touch different objects and does not wait for those loads before the reads.
-    __shared__ __align__(16) uint32_t lds0[2][kMBM * 16];
-    __shared__ __align__(16) uint32_t lds1[2][kMBM * 16];
+// MIRROR: as in mfma_grid3_tile, 64 half rows per tile; 2D grids (E1ONE).  2 x 2000 x 2000 points,
+// N = 4096: a call 553 -> 432 us; 3000 x 200, N = 4000: 132 -> 106.
+typedef uint32_t AStage[2][kMBM * 16];
 
+template <bool FP16, bool E1ONE, bool SPLIT, bool MIRROR>
+__device__ __forceinline__ void mfma_grid_tile(AStage& lds0, AStage& lds1, const MfmaGeom& g, double alpha,
+                                               const uint32_t* __restrict__ a_hi, const uint32_t* __restrict__ a_lo,
+                                               const float2* __restrict__ e1, const float2* __restrict__ e2,
+                                               float* __restrict__ out, int64_t out_stride, int64_t comps,
+                                               int64_t steps_per, float* __restrict__ partial) {
+    constexpr int kStep = MIRROR ? 2 * kMKM : kMKM;  // modes per K step
+    constexpr int kQ = kStep / 4;                    // and per lane group
+    const int64_t apitch = MIRROR ? g.Np / 2 : g.Np;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int grp = lane >> 4;  // K group g
@@ -463,8 +459,8 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
         const int64_t c = ct * 256 + 16 * (wave * kMCF + cf) + l16;
         const int64_t cc = c < g.ncols ? c : g.ncols - 1;
         const int64_t i1 = cc / g.n2, i2 = cc - i1 * g.n2;
-        e1p[cf] = e1 + i1 * g.Np + 4 * grp;
-        e2p[cf] = e2 + i2 * g.Np + 4 * grp;
+        e1p[cf] = e1 + i1 * g.Np + kQ * grp;
+        e2p[cf] = e2 + i2 * g.Np + kQ * grp;
     }
 
     f32x4 acc[kMRF][kMCF];
@@ -484,9 +480,8 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
     for (int h = 0; h < 2; ++h) {
         const int q = h * 256 + wv * 64 + lane;
         const int r = q >> 2;
-        aoff[h] = (row0 + r) * g.Np + (((q & 3) ^ ((r >> 1) & 3)) * 4);
+        aoff[h] = (row0 + r) * apitch + (((q & 3) ^ ((r >> 1) & 3)) * 4);
     }
-    typedef uint32_t AStage[2][kMBM * 16];
     auto load_a = [&](int64_t step, AStage& S) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -498,9 +493,10 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
         }
     };
 
-    const int64_t steps = g.Np / kMKM;
-    const int64_t s0 = SPLIT ? split * steps_per : 0;
-    const int64_t s1 = SPLIT ? (s0 + steps_per < steps ? s0 + steps_per : steps) : steps;
+    const int64_t steps = g.Np / kStep;
+    const int64_t per = MIRROR ? steps_per / 2 : steps_per;  // steps_per: even, in steps of 16 modes
+    const int64_t s0 = SPLIT ? split * per : 0;
+    const int64_t s1 = SPLIT ? (s0 + per < steps ? s0 + per : steps) : steps;
     load_a(s0, lds0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -510,49 +506,57 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
     auto step = [&](const AStage& C, AStage& Nx, int64_t s) {
         if (s + 1 < s1) load_a(s + 1, Nx);
 
-        // B fragments for this K step, built in registers.
-        u32x4 bh[kMCF], bl[kMCF];
-        const int64_t moff = s * kMKM;
-        float2 zf[4];
+        // B fragments for this K step, built in registers: [real, imaginary parts][column
+        // fragment], without MIRROR one of the pairs
+        constexpr int kParts = MIRROR ? 2 : 1;
+        u32x4 bh[kParts][kMCF], bl[kParts][kMCF];
+        const int64_t moff = s * kStep;
 #pragma unroll
         for (int cf = 0; cf < kMCF; ++cf) {
-            float2 yf[4];
-            if constexpr (!E1ONE) {
-                const float4* p = reinterpret_cast<const float4*>(e1p[cf] + moff);
-                const float4 q0 = p[0], q1 = p[1];
-                yf[0] = {q0.x, q0.y};
-                yf[1] = {q0.z, q0.w};
-                yf[2] = {q1.x, q1.y};
-                yf[3] = {q1.z, q1.w};
+            float2 yf[kQ], zf[kQ];
+#pragma unroll
+            for (int q = 0; q < kQ / 2; ++q) {
+                if constexpr (!E1ONE) {
+                    const float4 v = reinterpret_cast<const float4*>(e1p[cf] + moff)[q];
+                    yf[2 * q] = {v.x, v.y};
+                    yf[2 * q + 1] = {v.z, v.w};
+                }
+                const float4 v = reinterpret_cast<const float4*>(e2p[cf] + moff)[q];
+                zf[2 * q] = {v.x, v.y};
+                zf[2 * q + 1] = {v.z, v.w};
             }
-            {
-                const float4* p = reinterpret_cast<const float4*>(e2p[cf] + moff);
-                const float4 q0 = p[0], q1 = p[1];
-                zf[0] = {q0.x, q0.y};
-                zf[1] = {q0.z, q0.w};
-                zf[2] = {q1.x, q1.y};
-                zf[3] = {q1.z, q1.w};
-            }
-            uint32_t h4[4], l4[4];
+            auto value = [&](int t) { return E1ONE ? zf[t] : cmul(yf[t], zf[t]); };
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const float2 v = E1ONE ? zf[t] : cmul(yf[t], zf[t]);
-                split2<FP16>(v.x, v.y, h4[t], l4[t]);
+                uint32_t h, l;
+                if constexpr (MIRROR) {
+                    const float2 v = value(2 * t), w = value(2 * t + 1);
+                    split2<FP16>(v.x, w.x, h, l);
+                    bh[0][cf][t] = h;
+                    bl[0][cf][t] = l;
+                    split2<FP16>(v.y, w.y, h, l);
+                    bh[1][cf][t] = h;
+                    bl[1][cf][t] = l;
+                } else {
+                    const float2 v = value(t);
+                    split2<FP16>(v.x, v.y, h, l);
+                    bh[0][cf][t] = h;
+                    bl[0][cf][t] = l;
+                }
             }
-            bh[cf] = u32x4{h4[0], h4[1], h4[2], h4[3]};
-            bl[cf] = u32x4{l4[0], l4[1], l4[2], l4[3]};
         }
 
 #pragma unroll
         for (int rf = 0; rf < kMRF; ++rf) {
+            const int part = MIRROR && rf >= kMRF / 2 ? 1 : 0;
             const int pos = (rf * 16 + l16) * 16 + ((grp ^ asw) * 4);
             const u32x4 ah = *reinterpret_cast<const u32x4*>(&C[0][pos]);
             const u32x4 al = *reinterpret_cast<const u32x4*>(&C[1][pos]);
 #pragma unroll
             for (int cf = 0; cf < kMCF; ++cf) {
-                acc[rf][cf] = mfma<FP16>(ah, bh[cf], acc[rf][cf]);
-                acc[rf][cf] = mfma<FP16>(ah, bl[cf], acc[rf][cf]);
-                acc[rf][cf] = mfma<FP16>(al, bh[cf], acc[rf][cf]);
+                acc[rf][cf] = mfma<FP16>(ah, bh[part][cf], acc[rf][cf]);
+                acc[rf][cf] = mfma<FP16>(ah, bl[part][cf], acc[rf][cf]);
+                acc[rf][cf] = mfma<FP16>(al, bh[part][cf], acc[rf][cf]);
             }
         }
         // the next step's LDS loads have landed (the barrier's own wait covers LDS, not them)
@@ -575,18 +579,63 @@ __global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, doubl
         const int64_t i1 = c / g.n2;
         col[cf] = i1 * g.c1s + (c - i1 * g.n2);
     }
+    if constexpr (MIRROR) {
 #pragma unroll
-    for (int rf = 0; rf < kMRF; ++rf) {
+        for (int rf = 0; rf < kMRF / 2; ++rf) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t row = row0 + rf * 16 + grp * 4 + i;
-            if (row < g.n0) {
+            for (int i = 0; i < 4; ++i) {
+                const int64_t row = rt * (kMBM / 2) + rf * 16 + grp * 4 + i;
 #pragma unroll
-                for (int cf = 0; cf < kMCF; ++cf)
-                    if (cok[cf]) out[row * g.rs + col[cf]] = fa * acc[rf][cf][i];
+                for (int cf = 0; cf < kMCF; ++cf) {
+                    if (!cok[cf]) continue;
+                    const float c = acc[rf][cf][i], sn = acc[rf + kMRF / 2][cf][i];
+                    if (2 * row < g.n0) out[row * g.rs + col[cf]] = fa * (c + sn);
+                    if (2 * row + 1 < g.n0) out[(g.n0 - 1 - row) * g.rs + col[cf]] = fa * (c - sn);
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int rf = 0; rf < kMRF; ++rf) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t row = row0 + rf * 16 + grp * 4 + i;
+                if (row < g.n0) {
+#pragma unroll
+                    for (int cf = 0; cf < kMCF; ++cf)
+                        if (cok[cf]) out[row * g.rs + col[cf]] = fa * acc[rf][cf][i];
+                }
             }
         }
     }
+}
+
+template <bool FP16, bool E1ONE, bool SPLIT>
+__global__ __launch_bounds__(kMWaves * 64, 2) void k_mfma_grid(MfmaGeom g, double alpha,
+                                                               const double* __restrict__ ax0,
+                                                               const uint32_t* __restrict__ a_hi,
+                                                               const uint32_t* __restrict__ a_lo,
+                                                               const float2* __restrict__ e1,
+                                                               const float2* __restrict__ e2,
+                                                               float* __restrict__ out, int64_t out_stride,
+                                                               int64_t comps, int64_t steps_per,
+                                                               float* __restrict__ partial) {
+    // two stages [hi/lo][row * 16 + chunk * 4]: 64-byte A rows, 16-byte chunk c of row r
+    // stored at c ^ ((r >> 1) & 3) (the 8 lanes of a 16-byte LDS access phase hit 8 bank
+    // groups).  The stages are separate LDS objects and the step loop is unrolled by two,
+    // so the compiler sees that a step's LDS reads and the next step's global -> LDS loads
+    // touch different objects and does not wait for those loads before the reads.
+    __shared__ __align__(16) AStage lds0;
+    __shared__ __align__(16) AStage lds1;
+    if constexpr (E1ONE) {
+        if (mirrored_axis(ax0, g.n0)) {  // one value for the launch, and that of its tables
+            mfma_grid_tile<FP16, true, SPLIT, true>(lds0, lds1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
+                                                    steps_per, partial);
+            return;
+        }
+    }
+    mfma_grid_tile<FP16, E1ONE, SPLIT, false>(lds0, lds1, g, alpha, a_hi, a_lo, e1, e2, out, out_stride, comps,
+                                              steps_per, partial);
 }
 
 // 3D grids with n1, n2 >= 16: block tile = 128 rows x (16 i1 x 16 i2) columns.
@@ -968,17 +1017,17 @@ int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t c
             ksplit > 1 ? go(k_mfma_grid3<FP16, true, false>) : go(k_mfma_grid3<FP16, false, false>);
     } else if (d == 2) {
         if (ksplit > 1)
-            hipLaunchKernelGGL((k_mfma_grid<FP16, true, true>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2,
+            hipLaunchKernelGGL((k_mfma_grid<FP16, true, true>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2,
                                out, stride, comps, steps_per, partial);
         else
-            hipLaunchKernelGGL((k_mfma_grid<FP16, true, false>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2,
+            hipLaunchKernelGGL((k_mfma_grid<FP16, true, false>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2,
                                out, stride, comps, steps_per, partial);
     } else {
         if (ksplit > 1)
-            hipLaunchKernelGGL((k_mfma_grid<FP16, false, true>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1, e2,
+            hipLaunchKernelGGL((k_mfma_grid<FP16, false, true>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1, e2,
                                out, stride, comps, steps_per, partial);
         else
-            hipLaunchKernelGGL((k_mfma_grid<FP16, false, false>), grid, block, 0, s, g, alpha, a_hi, a_lo, e1,
+            hipLaunchKernelGGL((k_mfma_grid<FP16, false, false>), grid, block, 0, s, g, alpha, ax0, a_hi, a_lo, e1,
                                e2, out, stride, comps, steps_per, partial);
     }
     st = launch_status();

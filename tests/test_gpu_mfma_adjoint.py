@@ -133,6 +133,7 @@ def test_mfma_uniform_last_axis(shape, n):
     ((1, 17, 16), 31, 1), ((2, 16, 33), 32, 1), ((3, 16, 16), 33, 3), ((64, 18, 20), 100, 1), ((65, 16, 17), 65, 1),
     ((127, 16, 16), 64, 3), ((128, 17, 16), 40, 1), ((129, 16, 19), 300, 1), ((33, 260), 70, 1), ((258, 257), 129, 1),
     ((250, 21, 16), 90, 3), ((400, 16, 17), 40, 1), ((200, 40, 50), 600, 1),  # 128 half rows per tile
+    ((64, 33), 31, 2), ((129, 70), 33, 1), ((300, 255), 500, 1), ((131, 400), 96, 2),  # flat columns
 ])
 def test_mfma_mirrored_row_axis(shape, n, comps):
     """A row axis that is its own mirror image is summed over half its rows (cosine and sine
