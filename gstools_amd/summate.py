@@ -84,6 +84,7 @@ def _axes(axes, name, dev):
     before it, 40 to 50 us of an idle GPU per call.  While the stream is being captured they
     are copied the plain way, which a capture refuses: a recorded copy would read the buffer
     again at every replay."""
+    axes = list(axes)  # an iterator serves one pass only
     if any(isinstance(a, torch.Tensor) for a in axes) or torch.cuda.is_current_stream_capturing():
         parts = [_as_f64(a, name, dev).reshape(-1) for a in axes]
         flat = torch.cat(parts) if parts else torch.empty(0, dtype=torch.float64, device=dev)
@@ -303,8 +304,8 @@ def summate_incompr_grid_device(cov_samples, z_1, z_2, axes, precision="fp64", a
     if d < 2:
         raise ValueError(f"summate_incompr: incompressible sums need d = 2 or 3, got d = {d}")
     flat, shape = _axes(axes, "axes", dev)
-    if len(axes) != d:
-        raise ValueError(f"expected {d} axes, got {len(axes)}")
+    if len(shape) != d:
+        raise ValueError(f"expected {d} axes, got {len(shape)}")
     npts = int(np.prod(shape))
     shape_c = (ctypes.c_int64 * 3)(*(shape + [1] * (3 - d)))
     if precision not in INCOMPR_GRID_PRECISIONS:
