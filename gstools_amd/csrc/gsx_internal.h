@@ -20,6 +20,20 @@ inline int launch_status() {
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// `blocks` blocks of `threads` threads in launches of fewer than 2^32 threads each, one in
+// all but the largest calls: of a larger grid the runtime takes the number of threads
+// modulo 2^32 and reports nothing.  go(first block, grid).
+template <class Launch>
+inline int launch_parts(int64_t blocks, int64_t threads, Launch go) {
+    const int64_t most = 0xffffffffLL / threads;
+    for (int64_t first = 0; first < blocks; first += most) {
+        go(first, dim3((unsigned)(blocks - first < most ? blocks - first : most)));
+        const int st = launch_status();
+        if (st != GSX_OK) return st;
+    }
+    return GSX_OK;
+}
+
 // Points of an unstructured (d, P) row-major array.
 template <int D>
 struct UnstructuredPoints {

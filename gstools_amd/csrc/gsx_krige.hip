@@ -325,14 +325,14 @@ __global__ void k_krige_reduce(int64_t tiles, int64_t P, const double* __restric
 // field_p = sum_j a_j V[j, p]: 128 points per block (512 blocks for 65536 points,
 // where one thread per four points made 64), wave w the rows j = w mod 4 from the last
 // 16-row step down, the four sums added as in k_krige_gemm.  kPair (P even, V 16-byte
-// aligned): a point pair per lane, else two points 64 apart.
+// aligned): a point pair per lane, else two points 64 apart.  first: the launch's first block.
 template <bool kPair>
-__global__ __launch_bounds__(256) void k_krige_field(int64_t K, int64_t P, const double* __restrict__ a,
+__global__ __launch_bounds__(256) void k_krige_field(int64_t first, int64_t K, int64_t P, const double* __restrict__ a,
                                                      const double* __restrict__ V, double* __restrict__ field) {
     typedef __attribute__((ext_vector_type(2))) double f64x2;
     __shared__ double red[4][kKrPts];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t p0 = (int64_t)blockIdx.x * kKrPts;
+    const int64_t p0 = (first + blockIdx.x) * kKrPts;
     const int c0 = kPair ? 2 * lane : lane, c1 = kPair ? 2 * lane + 1 : lane + 64;
     // clamped (valid) addresses past P
     const int64_t q0 = p0 + c0 < P ? p0 + c0 : (kPair ? P - 2 : P - 1), q1 = p0 + c1 < P ? p0 + c1 : P - 1;
@@ -524,14 +524,13 @@ int gsx_krige_f64(int64_t K, int64_t P, const double* krig_mat, const double* kr
     int st = gsx::launch_status();
     if (st != GSX_OK) return st;
     const bool pair_b = P % 2 == 0 && reinterpret_cast<uintptr_t>(krig_vecs) % 16 == 0;
-    if (!variance) {
-        const dim3 grid((unsigned)col_blocks);
-        if (pair_b)
-            hipLaunchKernelGGL(gsx::k_krige_field<true>, grid, dim3(256), 0, s, K, P, a, krig_vecs, field);
-        else
-            hipLaunchKernelGGL(gsx::k_krige_field<false>, grid, dim3(256), 0, s, K, P, a, krig_vecs, field);
-        return gsx::launch_status();
-    }
+    if (!variance)
+        return gsx::launch_parts(col_blocks, 256, [&](int64_t first, dim3 grid) {
+            if (pair_b)
+                hipLaunchKernelGGL(gsx::k_krige_field<true>, grid, dim3(256), 0, s, first, K, P, a, krig_vecs, field);
+            else
+                hipLaunchKernelGGL(gsx::k_krige_field<false>, grid, dim3(256), 0, s, first, K, P, a, krig_vecs, field);
+        });
     // error = v^T M2 v over the block upper triangle
     const int64_t col8 = gsx::ceil_div(col_blocks, (int64_t)8) * 8;
     const dim3 grid((unsigned)(col8 * tiles));
