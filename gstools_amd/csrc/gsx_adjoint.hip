@@ -260,8 +260,9 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
 // modes per stage-2 block (16 doubles: one 128-byte line) and threads per mode
 constexpr int kAdj2Modes = 16, kAdj2Slices = 64;
 
+// first: the launch's first block
 template <int D, bool F64>
-__global__ __launch_bounds__(kAdj2Modes * kAdj2Slices) void k_adjoint_stage2(int64_t N, int64_t chunks,
+__global__ __launch_bounds__(kAdj2Modes * kAdj2Slices) void k_adjoint_stage2(int64_t first, int64_t N, int64_t chunks,
                                                                              const double* __restrict__ z1,
                                                                              const double* __restrict__ z2,
                                                                              const double* __restrict__ part,
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(kAdj2Modes * kAdj2Slices) void k_adjoint_stage2(int
     static_assert(Q <= kAdj2Slices, "one slice adds the slices' sums of one quantity");
     __shared__ double red[kAdj2Slices][Q][kAdj2Modes];
     const int m = threadIdx.x % kAdj2Modes, w = threadIdx.x / kAdj2Modes;
-    const int64_t j = (int64_t)blockIdx.x * kAdj2Modes + m;
+    const int64_t j = (first + blockIdx.x) * kAdj2Modes + m;
     double acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) acc[q] = 0.0;
@@ -333,9 +334,11 @@ int adjoint_launch(const AdjPlan& pl, int64_t N, int64_t P, const double* cov, c
     }
     int st = launch_status();
     if (st != GSX_OK) return st;
-    hipLaunchKernelGGL((k_adjoint_stage2<D, sizeof(GT) == 8>), dim3((unsigned)ceil_div(N, (int64_t)kAdj2Modes)),
-                       dim3(kAdj2Modes * kAdj2Slices), 0, s, N, pl.chunks, z1, z2, part, gz1, gz2, gk);
-    return launch_status();
+    constexpr int kBlock = kAdj2Modes * kAdj2Slices;
+    return launch_parts(ceil_div(N, (int64_t)kAdj2Modes), kBlock, [&](int64_t first, dim3 grid) {
+        hipLaunchKernelGGL((k_adjoint_stage2<D, sizeof(GT) == 8>), grid, dim3(kBlock), 0, s, first, N, pl.chunks, z1,
+                           z2, part, gz1, gz2, gk);
+    });
 }
 
 // Fills the gradients with zeros when there are no points.

@@ -1,12 +1,16 @@
 """Calls whose threads number 2^32 or more: a grid of that size is cut off by the runtime without
 an error, so they take several launches.  Values are constants or one-line sums, on 20 to 80 GB."""
 
+import importlib
+import math
 import sys
 
 import pytest
 import torch
 
 from gstools_amd.krige import krige_sum_device
+
+summate = importlib.import_module("gstools_amd.summate")
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +36,18 @@ def test_kriging_field_of_many_points(p):
     _say(f"krige field P={p}")
     field = krige_sum_device(_full((1, 1), 1.0), _full((1, p), 2.0), _full((1,), 1.5), variance=False)
     assert bool((field == 3.0).all())
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_adjoint_of_many_modes(precision):
+    """2^26 modes and a few: every one gets its gradients."""
+    _say(f"adjoint of 2^26 modes {precision}")
+    n = 2**26 + 21
+    g = torch.tensor([1.0, 3.0], dtype=torch.float64 if precision == "fp64" else torch.float32, device="cuda")
+    pos = torch.tensor([[1.0, 2.0]], dtype=torch.float64, device="cuda")
+    gz1, gz2, gk = summate.summate_adjoint_device(_full((1, n), 0.5), _full((n,), 1.0), _full((n,), 0.0), pos, g,
+                                                  precision)
+    c1, s1, c2, s2 = math.cos(0.5), math.sin(0.5), math.cos(1.0), math.sin(1.0)
+    tol = 1e-14 if precision == "fp64" else 1e-5
+    for got, want in ((gz1, c1 + 3 * c2), (gz2, s1 + 3 * s2), (gk, -(s1 + 6 * s2))):
+        assert float((got - want).abs().max()) <= tol * 10
