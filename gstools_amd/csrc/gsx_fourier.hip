@@ -205,6 +205,7 @@ __device__ __forceinline__ void phase_sincos(double th, double* s, double* c) {
 //  * the other axes' tables in rotation form, rows (point, part) x columns (part', m):
 //    row (i, 0) = [cos(k_m x_i), -sin(k_m x_i)], row (i, 1) = [sin, cos] (2 n x 2 M).
 struct FourierPrep {
+    int64_t first;  // the launch's first block
     int64_t N, d;
     int64_t M[3], n[3];
     const double *fac, *z1, *z2, *x[3], *k[3];
@@ -212,7 +213,7 @@ struct FourierPrep {
 };
 
 __global__ __launch_bounds__(256) void k_fourier_prepare(FourierPrep f) {
-    int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    int64_t e = (f.first + blockIdx.x) * 256 + threadIdx.x;
     if (e < f.N) {
         f.c[e] = f.fac[e] * f.z1[e];
         f.c[f.N + e] = -(f.fac[e] * f.z2[e]);
@@ -345,7 +346,7 @@ int gsx_summate_fourier_tensor_f64(int64_t d, const int64_t* mode_no, const doub
     const double* ax[3] = {axes, axes + p.n[0], axes + p.n[0] + p.n[1]};
     const double* ka[3] = {kaxes, kaxes + p.M[0], kaxes + p.M[0] + p.M[1]};
     double* c = ws + p.off_c;
-    gsx::FourierPrep f{p.N, d, {}, {}, spectrum_factor, z1, z2, {}, {}, c, {}};
+    gsx::FourierPrep f{0, p.N, d, {}, {}, spectrum_factor, z1, z2, {}, {}, c, {}};
     int64_t entries = p.N;
     for (int i = 0; i < d; ++i) {
         f.M[i] = p.M[i];
@@ -356,9 +357,10 @@ int gsx_summate_fourier_tensor_f64(int64_t d, const int64_t* mode_no, const doub
         entries += p.n[i] * p.M[i];
     }
     if (gsx::ceil_div(entries, (int64_t)256) > 0x7fffffffLL) return GSX_E_INVALID;
-    hipLaunchKernelGGL(gsx::k_fourier_prepare, dim3((unsigned)gsx::ceil_div(entries, (int64_t)256)), dim3(256), 0, s,
-                       f);
-    int st = gsx::launch_status();
+    int st = gsx::launch_parts(gsx::ceil_div(entries, (int64_t)256), 256, [&](int64_t first, dim3 grid) {
+        f.first = first;
+        hipLaunchKernelGGL(gsx::k_fourier_prepare, grid, dim3(256), 0, s, f);
+    });
     if (st != GSX_OK) return st;
     const int64_t Md = p.M[d - 1], nd = p.n[d - 1];
     double* last = ws + p.off_last;

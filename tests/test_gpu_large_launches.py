@@ -51,3 +51,16 @@ def test_adjoint_of_many_modes(precision):
     tol = 1e-14 if precision == "fp64" else 1e-5
     for got, want in ((gz1, c1 + 3 * c2), (gz2, s1 + 3 * s2), (gk, -(s1 + 6 * s2))):
         assert float((got - want).abs().max()) <= tol * 10
+
+
+def test_fourier_tables_of_many_entries():
+    """4096 points and 2^20 - 1 modes: the coefficients and the table make 2^32 entries and more."""
+    _say("Fourier tensor 4096 x (2^20 - 1)")
+    n, m = 4096, 2**20 - 1
+    k = torch.linspace(0.0, 1.0, m, dtype=torch.float64, device="cuda")
+    x = torch.linspace(0.0, 1.0, n, dtype=torch.float64, device="cuda")
+    w = _full((m,), 1.0 / m)
+    u = summate.summate_fourier_tensor_device(_full((m,), 1.0), [k], w, w, [x])
+    for i in (0, 1, 2047, n - 1):
+        want = float((torch.cos(k * x[i]) + torch.sin(k * x[i])).mean())
+        assert abs(float(u[i]) - want) <= 1e-10, i  # 2^20 terms added in one chain: below 2^20 2^-53
