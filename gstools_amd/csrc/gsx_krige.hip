@@ -75,16 +75,17 @@ inline int64_t krige_kp(int64_t K) { return ceil_div(K, (int64_t)kKrK) * kKrK; }
 // Blocks [0, ceil(K / 64)): a_j = sum_i cond_i M[i, j] for 64 columns, 16 waves of
 // every 16th row, added in order.  The blocks after them (variance form): M2.  Both
 // read M once and neither waits for the other, so one launch serves them (three took
-// 4.5 us each).
-__global__ __launch_bounds__(1024) void k_krige_prepare(int64_t K, int64_t Rp, int64_t Kp,
+// 4.5 us each).  first: the launch's first block.
+__global__ __launch_bounds__(1024) void k_krige_prepare(int64_t first, int64_t K, int64_t Rp, int64_t Kp,
                                                         const double* __restrict__ M,
                                                         const double* __restrict__ cond, double* __restrict__ a,
                                                         double* __restrict__ M2) {
     __shared__ double red[16][64];
     const int64_t wblocks = (K + 63) / 64;
-    if ((int64_t)blockIdx.x < wblocks) {
+    const int64_t block = first + blockIdx.x;
+    if (block < wblocks) {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const int64_t j = (int64_t)blockIdx.x * 64 + lane;
+        const int64_t j = block * 64 + lane;
         double s = 0.0;
         if (j < K) {
 #pragma unroll 8
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(1024) void k_krige_prepare(int64_t K, int64_t Rp, i
         }
         return;
     }
-    const int64_t idx = ((int64_t)blockIdx.x - wblocks) * 1024 + threadIdx.x;
+    const int64_t idx = (block - wblocks) * 1024 + threadIdx.x;
     if (idx >= Rp * Kp) return;
     const int64_t i = idx / Kp, l = idx - i * Kp;
     const int64_t b0 = (i / kKrDiag) * kKrDiag;
@@ -520,8 +521,9 @@ int gsx_krige_f64(int64_t K, int64_t P, const double* krig_mat, const double* kr
     double* m2 = ws + (tiles * P + K + 1) / 2 * 2;
     if (variance && reinterpret_cast<uintptr_t>(m2) % 16 != 0) return GSX_E_INVALID;
     const int64_t prep = gsx::ceil_div(K, (int64_t)64) + (variance ? gsx::ceil_div(Rp * Kp, (int64_t)1024) : 0);
-    hipLaunchKernelGGL(gsx::k_krige_prepare, dim3((unsigned)prep), dim3(1024), 0, s, K, Rp, Kp, krig_mat, cond, a, m2);
-    int st = gsx::launch_status();
+    int st = gsx::launch_parts(prep, 1024, [&](int64_t first, dim3 grid) {
+        hipLaunchKernelGGL(gsx::k_krige_prepare, grid, dim3(1024), 0, s, first, K, Rp, Kp, krig_mat, cond, a, m2);
+    });
     if (st != GSX_OK) return st;
     const bool pair_b = P % 2 == 0 && reinterpret_cast<uintptr_t>(krig_vecs) % 16 == 0;
     if (!variance)

@@ -38,6 +38,16 @@ def test_kriging_field_of_many_points(p):
     assert bool((field == 3.0).all())
 
 
+def test_kriging_variance_of_a_large_system():
+    """65505 conditions: the weights and the padded matrix make 2^32 entries."""
+    k, p = 65505, 64
+    _say(f"krige variance K={k}")
+    m = torch.zeros((k, k), dtype=torch.float64, device="cuda")
+    m.diagonal().fill_(2.0)
+    field, error = krige_sum_device(m, _full((k, p), 1.0), _full((k,), 1.0))
+    assert bool((field == 2.0 * k).all()) and bool((error == 2.0 * k).all())
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 def test_adjoint_of_many_modes(precision):
     """2^26 modes and a few: every one gets its gradients."""
