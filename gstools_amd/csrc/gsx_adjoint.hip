@@ -68,6 +68,13 @@ inline AdjPlan adj_plan(int64_t N, int64_t P, int64_t max_chunks_cap = 0) {
     return pl;
 }
 
+// Chunks whose partial sums a workspace has to hold: as many as there are with the same
+// number of whole 256-point stages in each.  More room takes the plan's number.
+inline int64_t adj_least_chunks(int64_t N, int64_t P) {
+    const int64_t stages = ceil_div(P, (int64_t)kAdjPts), most = ceil_div(kAdjTargetBlocks, ceil_div(N, (int64_t)kThreads));
+    return ceil_div(stages, ceil_div(stages, most < stages ? most : stages));
+}
+
 inline int adj_modes(const AdjPlan& pl, int64_t N) {
     return N > kThreads && ceil_div(N, (int64_t)kThreads * kAdjModesF32) * pl.chunks >= 512 ? kAdjModesF32 : 1;
 }
@@ -389,9 +396,9 @@ int adjoint_entry(int64_t d, int64_t N, int64_t P, const double* cov, const doub
     bool done;
     const int st = adjoint_prologue<GT>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, s, &done);
     if (done) return st;
-    const int64_t need = gsx_summate_adjoint_workspace(d, N, P);
-    if (!ws || ws_bytes < need) return GSX_E_WORKSPACE;
-    return adjoint_run<GT>(adj_plan<sizeof(GT) == 8>(N, P), d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
+    const int64_t per_chunk = (2 + 2 * d) * N * (int64_t)sizeof(double);
+    if (!ws || ws_bytes < adj_least_chunks(N, P) * per_chunk) return GSX_E_WORKSPACE;
+    return adjoint_run<GT>(adj_plan<sizeof(GT) == 8>(N, P, ws_bytes / per_chunk), d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -456,7 +463,7 @@ extern "C" {
 int64_t gsx_summate_adjoint_workspace(int64_t d, int64_t N, int64_t P) {
     if (d < 1 || d > 3 || N < 0 || P < 0) return GSX_E_INVALID;
     if (N == 0 || P == 0) return 0;
-    const gsx::AdjPlan pl = gsx::adj_plan<true>(N, P);  // FP32: fewer chunks
+    const gsx::AdjPlan pl = gsx::adj_plan<true>(N, P);  // FP32 has no more chunks
     return pl.chunks * (2 + 2 * d) * N * (int64_t)sizeof(double);
 }
 
@@ -465,7 +472,7 @@ int gsx_summate_adjoint_f64(int64_t d, int64_t N, int64_t P, const double* cov, 
                             double* gz2, double* gk, void* workspace, int64_t workspace_bytes,
                             void* stream) {
     return gsx::adjoint_entry<double>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, workspace,
-                                   workspace_bytes, stream);
+                                      workspace_bytes, stream);
 }
 
 int gsx_summate_adjoint_f32(int64_t d, int64_t N, int64_t P, const double* cov, const double* z1,
@@ -473,7 +480,7 @@ int gsx_summate_adjoint_f32(int64_t d, int64_t N, int64_t P, const double* cov, 
                             double* gz2, double* gk, void* workspace, int64_t workspace_bytes,
                             void* stream) {
     return gsx::adjoint_entry<float>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, workspace,
-                                   workspace_bytes, stream);
+                                     workspace_bytes, stream);
 }
 
 int gsx_summate_adjoint_f32_noalloc(int64_t d, int64_t N, int64_t P, const double* cov,
