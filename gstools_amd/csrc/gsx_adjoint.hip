@@ -13,7 +13,7 @@
 // walks the chunk's points, which are staged through LDS with g_i x_id
 // precomputed (every lane reads the same point: LDS broadcast).  It writes
 // the 2 + 2D partial sums of its (chunk, mode) to the workspace.  Stage 2
-// sums the chunks of each mode in a fixed order (64 threads of every 64th chunk, the
+// sums the chunks of each mode in a fixed order (S threads of every Sth chunk, the
 // threads in order), so results are bitwise reproducible run to run (no atomics).
 //
 // 2D, 2048 modes, FP32, 1e6 points: stage 1 719 -> 694 us (bound by the vector unit),
@@ -264,47 +264,67 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
     }
 }
 
-// modes per stage-2 block (16 doubles: one 128-byte line) and threads per mode
-constexpr int kAdj2Modes = 16, kAdj2Slices = 64;
-
-// first: the launch's first block
-template <int D, bool F64>
-__global__ __launch_bounds__(kAdj2Modes * kAdj2Slices) void k_adjoint_stage2(int64_t first, int64_t N, int64_t chunks,
-                                                                             const double* __restrict__ z1,
-                                                                             const double* __restrict__ z2,
-                                                                             const double* __restrict__ part,
-                                                                             double* __restrict__ gz1,
-                                                                             double* __restrict__ gz2,
-                                                                             double* __restrict__ gk) {
+// Stage 2: MODES modes per block and SLICES threads per mode, each adding every SLICESth
+// chunk, then the threads in order.  Bound by the latency of a thread's reads, and with many
+// modes by the traffic.  There are at most 2048 / (mode tiles of 256) chunks, so many chunks
+// come with few modes: 64 slices of 16 modes (one 128-byte line of a row) where there are
+// more than 32 (2048 modes, 245 chunks: 70 us with one thread per mode, 8 with 64), but with
+// few they only take up room: 65536 modes with 8 chunks 17 us (4 slices of 64 modes: 7),
+// 32768 with 16 chunks 10 (4), and with up to 4 chunks one thread per mode is best
+// (10^6 modes, one chunk: 200, 25 and 12 us).  first: the launch's first block.
+template <int D, bool F64, int MODES, int SLICES>
+__global__ __launch_bounds__(MODES * SLICES) void k_adjoint_stage2(int64_t first, int64_t N, int64_t chunks,
+                                                                   const double* __restrict__ z1,
+                                                                   const double* __restrict__ z2,
+                                                                   const double* __restrict__ part,
+                                                                   double* __restrict__ gz1,
+                                                                   double* __restrict__ gz2,
+                                                                   double* __restrict__ gk) {
     constexpr int Q = adj_sums<D, F64>();
-    static_assert(Q <= kAdj2Slices, "one slice adds the slices' sums of one quantity");
-    __shared__ double red[kAdj2Slices][Q][kAdj2Modes];
-    const int m = threadIdx.x % kAdj2Modes, w = threadIdx.x / kAdj2Modes;
-    const int64_t j = (first + blockIdx.x) * kAdj2Modes + m;
+    const int m = threadIdx.x % MODES, w = threadIdx.x / MODES;
+    const int64_t j = (first + blockIdx.x) * MODES + m;
     double acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) acc[q] = 0.0;
-    if (j < N) {
+    if constexpr (SLICES == 1) {
+        if (j < N) {
 #pragma unroll 4
-        for (int64_t c = w; c < chunks; c += kAdj2Slices) {
-            const double* src = part + c * Q * N;
+            for (int64_t c = 0; c < chunks; ++c)
 #pragma unroll
-            for (int q = 0; q < Q; ++q) acc[q] += src[q * N + j];
+                for (int q = 0; q < Q; ++q) acc[q] += part[(c * Q + q) * N + j];
         }
-    }
+    } else {
+        constexpr int kAhead = 4;  // chunks read together, from clamped rows
+        if (j < N) {
+            for (int64_t c = w; c < chunks; c += kAhead * SLICES) {
+                double v[kAhead][Q];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) red[w][q][m] = acc[q];
-    __syncthreads();
-    if (w < Q) {
-        double r = 0.0;
+                for (int u = 0; u < kAhead; ++u) {
+                    const int64_t cu = c + u * SLICES < chunks ? c + u * SLICES : chunks - 1;
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) v[u][q] = part[(cu * Q + q) * N + j];
+                }
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) acc[q] += c + u * SLICES < chunks ? v[u][q] : 0.0;
+            }
+        }
+        __shared__ double red[SLICES][Q][MODES];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) red[w][q][m] = acc[q];
+        __syncthreads();
+        for (int q = w; q < Q; q += SLICES) {
+            double r = 0.0;
 #pragma unroll 16
-        for (int v = 0; v < kAdj2Slices; ++v) r += red[v][w][m];
-        red[0][w][m] = r;  // read by this thread only until the barrier
-    }
-    __syncthreads();
-    if (w != 0 || j >= N) return;
+            for (int v = 0; v < SLICES; ++v) r += red[v][q][m];
+            red[0][q][m] = r;  // read by this thread only until the barrier
+        }
+        __syncthreads();
 #pragma unroll
-    for (int q = 0; q < Q; ++q) acc[q] = red[0][q][m];
+        for (int q = 0; q < Q; ++q) acc[q] = red[0][q][m];
+    }
+    if (w != 0 || j >= N) return;
     const double a1 = z1[j], a2 = z2[j];
     if constexpr (F64) {
         gz1[j] = acc[0];
@@ -341,11 +361,16 @@ int adjoint_launch(const AdjPlan& pl, int64_t N, int64_t P, const double* cov, c
     }
     int st = launch_status();
     if (st != GSX_OK) return st;
-    constexpr int kBlock = kAdj2Modes * kAdj2Slices;
-    return launch_parts(ceil_div(N, (int64_t)kAdj2Modes), kBlock, [&](int64_t first, dim3 grid) {
-        hipLaunchKernelGGL((k_adjoint_stage2<D, sizeof(GT) == 8>), grid, dim3(kBlock), 0, s, first, N, pl.chunks, z1,
-                           z2, part, gz1, gz2, gk);
-    });
+    constexpr bool F64 = sizeof(GT) == 8;
+    auto stage2 = [&](auto kernel, int modes, int slices) {
+        return launch_parts(ceil_div(N, (int64_t)modes), modes * slices, [&](int64_t first, dim3 grid) {
+            hipLaunchKernelGGL(kernel, grid, dim3(modes * slices), 0, s, first, N, pl.chunks, z1, z2, part, gz1, gz2,
+                               gk);
+        });
+    };
+    if (pl.chunks <= 4) return stage2(k_adjoint_stage2<D, F64, 256, 1>, 256, 1);
+    if (pl.chunks <= 32) return stage2(k_adjoint_stage2<D, F64, 64, 4>, 64, 4);
+    return stage2(k_adjoint_stage2<D, F64, 16, 64>, 16, 64);
 }
 
 // Fills the gradients with zeros when there are no points.
