@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
         if constexpr (F64) {
             const double xmax = __longlong_as_double((long long)s_xmax);
             if (__all(k1 * xmax <= 0x1.0p+45)) {
-                for (int m = 0; m < cnt; ++m) {
+                auto point = [&](int m) {
                     double x[D];
 #pragma unroll
                     for (int d = 0; d < D; ++d) x[d] = s_x[m * D + d];
@@ -217,7 +217,15 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
                         acc[0][2 + d] = fma_(gg[1 + d], cs, acc[0][2 + d]);
                         acc[0][2 + D + d] = fma_(gg[1 + d], sn, acc[0][2 + D + d]);
                     }
+                };
+                // two points per iteration, by hand (the compiler does not unroll a loop of
+                // unknown length around inline assembly)
+                int m = 0;
+                for (; m + 1 < cnt; m += 2) {
+                    point(m);
+                    point(m + 1);
                 }
+                if (m < cnt) point(m);
             } else {
                 for (int m = 0; m < cnt; ++m) {
                     double x[D];
