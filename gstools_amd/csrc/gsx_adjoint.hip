@@ -52,27 +52,44 @@ constexpr int64_t kAdjTargetBlocks = 2048;
 constexpr int kAdjModesF32 = 2;
 
 struct AdjPlan {
-    int64_t chunks, units;  // chunk c: units [c units / chunks, (c + 1) units / chunks)
+    int64_t chunks, units;  // chunks of units / chunks units, the first units % chunks one longer
 };
+
+// The fewest chunks with the same number of whole stages in the longest one as 2048 blocks
+// of 256 modes allow.
+inline int64_t adj_whole_stages(int64_t N, int64_t P) {
+    const int64_t stages = ceil_div(P, (int64_t)kAdjPts), most = ceil_div(kAdjTargetBlocks, ceil_div(N, (int64_t)kThreads));
+    return ceil_div(stages, ceil_div(stages, most < stages ? most : stages));
+}
 
 // Point chunks of the stage-1 grid.  max_chunks_cap (> 0) bounds the number
 // of chunks, and with it the partial sums (chunks x (2 + 2D) x N doubles).
+//
+// As many chunks as 2048 blocks allow, rounded down while a chunk more is less than a block
+// more per CU (10000 modes make 40 mode tiles: 52 chunks, a few blocks over a whole number
+// per CU, take 1226 us for 300000 points in FP32, 51 take 1023; FP64 4130 and 3670).  Their
+// lengths are a unit apart, the longer ones first: in turn, blocks a multiple of 256 apart,
+// which land on one CU, were long ones together (FP32, 32768 modes, 5000 points: 95 us, 68
+// so).  Chunks of less than four 64-point units (FP64) are hardly worth a block's start: whole
+// stages, or finer where these come to less than 768 blocks, three per CU (2048 modes, 5000
+// points: 20 chunks 43 us, 79 32; but 65536 modes, 600 points: 3 chunks 63, 8 73, and 256
+// modes, 10^5 points: 391 chunks 65, 1563 75).
 template <bool F64>
 inline AdjPlan adj_plan(int64_t N, int64_t P, int64_t max_chunks_cap = 0) {
     AdjPlan pl;
     pl.units = ceil_div(P, adj_unit<F64>());
-    pl.chunks = ceil_div(kAdjTargetBlocks, ceil_div(N, (int64_t)kThreads));
-    if (pl.chunks > pl.units) pl.chunks = pl.units;
+    const int64_t tiles = ceil_div(N, (int64_t)kThreads);
+    const int64_t most = tiles <= 256 ? kAdjTargetBlocks / tiles : ceil_div(kAdjTargetBlocks, tiles);
+    if (!F64 || pl.units >= 4 * most) {
+        pl.chunks = pl.units < most ? pl.units : most;
+    } else {
+        pl.chunks = adj_whole_stages(N, P);
+        const int64_t fine = pl.units < 768 / tiles ? pl.units : 768 / tiles;
+        if (pl.chunks < fine) pl.chunks = fine;
+    }
     if (max_chunks_cap > 0 && pl.chunks > max_chunks_cap) pl.chunks = max_chunks_cap;
     if (pl.chunks < 1) pl.chunks = 1;
     return pl;
-}
-
-// Chunks whose partial sums a workspace has to hold: as many as there are with the same
-// number of whole 256-point stages in each.  More room takes the plan's number.
-inline int64_t adj_least_chunks(int64_t N, int64_t P) {
-    const int64_t stages = ceil_div(P, (int64_t)kAdjPts), most = ceil_div(kAdjTargetBlocks, ceil_div(N, (int64_t)kThreads));
-    return ceil_div(stages, ceil_div(stages, most < stages ? most : stages));
 }
 
 inline int adj_modes(const AdjPlan& pl, int64_t N) {
@@ -177,8 +194,9 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_stage1(int64_t N, int64_t 
         for (int q = 0; q < Q; ++q) acc[u][q] = 0.0;
 
     constexpr int64_t kUnit = adj_unit<F64>();
-    const int64_t p0 = blockIdx.y * units / gridDim.y * kUnit;
-    const int64_t pe = (blockIdx.y + 1) * units / gridDim.y * kUnit;
+    const int64_t y = blockIdx.y, each = units / gridDim.y, longer = units - each * gridDim.y;
+    const int64_t p0 = (y * each + (y < longer ? y : longer)) * kUnit;
+    const int64_t pe = p0 + (each + (y < longer ? 1 : 0)) * kUnit;
     const int64_t p1 = pe < P ? pe : P;
     for (int64_t s0 = p0; s0 < p1; s0 += kAdjPts) {
         const int cnt = (int)((p1 - s0) < kAdjPts ? (p1 - s0) : kAdjPts);
@@ -302,20 +320,22 @@ __global__ __launch_bounds__(MODES * SLICES) void k_adjoint_stage2(int64_t first
                 for (int q = 0; q < Q; ++q) acc[q] += part[(c * Q + q) * N + j];
         }
     } else {
-        constexpr int kAhead = 4;  // chunks read together, from clamped rows
+        // chunks read together (3D, blocks of 1024 threads: more take the registers of the
+        // CU's second block)
+        constexpr int kAhead = D == 3 && SLICES == 64 ? 2 : 4;
         if (j < N) {
             for (int64_t c = w; c < chunks; c += kAhead * SLICES) {
                 double v[kAhead][Q];
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u) {
-                    const int64_t cu = c + u * SLICES < chunks ? c + u * SLICES : chunks - 1;
+                    const int64_t cu = c + u * SLICES;
 #pragma unroll
-                    for (int q = 0; q < Q; ++q) v[u][q] = part[(cu * Q + q) * N + j];
+                    for (int q = 0; q < Q; ++q) v[u][q] = cu < chunks ? part[(cu * Q + q) * N + j] : 0.0;
                 }
 #pragma unroll
                 for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-                    for (int q = 0; q < Q; ++q) acc[q] += c + u * SLICES < chunks ? v[u][q] : 0.0;
+                    for (int q = 0; q < Q; ++q) acc[q] += v[u][q];
             }
         }
         __shared__ double red[SLICES][Q][MODES];
@@ -430,7 +450,10 @@ int adjoint_entry(int64_t d, int64_t N, int64_t P, const double* cov, const doub
     const int st = adjoint_prologue<GT>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, s, &done);
     if (done) return st;
     const int64_t per_chunk = (2 + 2 * d) * N * (int64_t)sizeof(double);
-    if (!ws || ws_bytes < adj_least_chunks(N, P) * per_chunk) return GSX_E_WORKSPACE;
+    // room for the plan's chunks, or for those of whole stages
+    const AdjPlan pl = adj_plan<sizeof(GT) == 8>(N, P);
+    const int64_t whole = adj_whole_stages(N, P), least = whole < pl.chunks ? whole : pl.chunks;
+    if (!ws || ws_bytes < least * per_chunk) return GSX_E_WORKSPACE;
     return adjoint_run<GT>(adj_plan<sizeof(GT) == 8>(N, P, ws_bytes / per_chunk), d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
 }
 
@@ -496,8 +519,8 @@ extern "C" {
 int64_t gsx_summate_adjoint_workspace(int64_t d, int64_t N, int64_t P) {
     if (d < 1 || d > 3 || N < 0 || P < 0) return GSX_E_INVALID;
     if (N == 0 || P == 0) return 0;
-    const gsx::AdjPlan pl = gsx::adj_plan<true>(N, P);  // FP32 has no more chunks
-    return pl.chunks * (2 + 2 * d) * N * (int64_t)sizeof(double);
+    const int64_t c64 = gsx::adj_plan<true>(N, P).chunks, c32 = gsx::adj_plan<false>(N, P).chunks;
+    return (c64 > c32 ? c64 : c32) * (2 + 2 * d) * N * (int64_t)sizeof(double);
 }
 
 int gsx_summate_adjoint_f64(int64_t d, int64_t N, int64_t P, const double* cov, const double* z1,
