@@ -58,6 +58,7 @@ constexpr int kMKM = 16;             // modes per K step
 struct MfmaGeom {
     int64_t n0, n1, n2;   // grid (n1 = 1 for 2D grids)
     int64_t n0p, Np;      // padded rows / modes
+    int64_t ksteps;       // 16-mode steps that hold a mode: the steps without a mirrored axis
     int64_t ncols;        // n1 * n2
     int64_t out_cols;     // valid flat columns i1 * n2 + i2: n1 * n2, or the split axis' length
     int64_t rs, c1s;      // output offset of (row, i1, i2) = row * rs + i1 * c1s + i2
@@ -77,6 +78,7 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
     g.n0p = ceil_div(g.n0, kMBM) * kMBM;
     g.g2 = (g.n1 >= 16 && g.n2 >= 16) ? 1 : 16;
     g.Np = ceil_div(N, 2 * kMKM) * 2 * kMKM;  // a mirrored row axis steps 32 modes at a time
+    g.ksteps = ceil_div(N, (int64_t)kMKM);
     g.ncols = g.n1 * g.n2;
     g.out_cols = g.ncols;
     g.rs = g.ncols;
@@ -493,7 +495,7 @@ __device__ __forceinline__ void mfma_grid_tile(AStage& lds0, AStage& lds1, const
         }
     };
 
-    const int64_t steps = g.Np / kStep;
+    const int64_t steps = MIRROR ? g.Np / kStep : g.ksteps;
     const int64_t per = MIRROR ? steps_per / 2 : steps_per;  // steps_per: even, in steps of 16 modes
     const int64_t s0 = SPLIT ? split * per : 0;
     const int64_t s1 = SPLIT ? (s0 + per < steps ? s0 + per : steps) : steps;
@@ -773,7 +775,7 @@ __device__ __forceinline__ void mfma_grid3_tile(Stage3<WIDE>& st0, Stage3<WIDE>&
 #pragma unroll
         for (int cf = 0; cf < kCF; ++cf) acc[rf][cf] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int64_t steps = g.Np / kStep;
+    const int64_t steps = MIRROR ? g.Np / kStep : g.ksteps;
     const int64_t per = MIRROR ? steps_per / 2 : steps_per;  // steps_per: even, in steps of 16 modes
     const int64_t s0 = SPLIT ? split * per : 0;
     const int64_t s1 = SPLIT ? (s0 + per < steps ? s0 + per : steps) : steps;
