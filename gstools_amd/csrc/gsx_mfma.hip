@@ -263,9 +263,14 @@ __device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int6
 }
 
 // --------------------------------------------------------------- tables ----
-// A (n0p x Np), E1 (n1 x Np), E2 (comps x n2 x Np): a block takes 256 modes of one row at a time,
-// so that rows and modes need no division per entry (two 64-bit ones per entry, and a phase
-// for each component, were a quarter of 20 us for 3 x 128^3 with N = 4096; now 15).
+// E1 (n1 x Np), E2 (comps x n2 x Np) and A (n0p x Np), their rows one after the other: a
+// wavefront takes 64 modes of a run of rows, so that a mode's wave vector and coefficients are
+// read once per run, rows are wave-uniform, their coordinates come out of a register, and one
+// place evaluates the phase, whatever the entry is.  The run's loop reads nothing: a wait for
+// a read would wait for the stores of the row before, too (that, and half of the threads idle
+// for less than 129 modes, is what blocks of 256 modes that went from row to row lost).  Bound
+// by the instructions of the FP64 phases.  3 x 128^3, N = 4096: 16 -> 10.5 us; 512^3 30 -> 26;
+// 2000 x 2000 irregular, N = 1000, 26 -> 19.5; 8192 x 500, N = 100, 13 -> 9.6.
 // comps > 1 (incompressible fields): E2 of component c carries the projector
 // weight p_c(k_j) = delta_c0 - k_jc k_j0 / |k_j|^2 (generator.py:479-494) in
 // place of the spectrum factor.
@@ -275,14 +280,15 @@ __device__ __forceinline__ bool mirrored_axis(const double* __restrict__ x, int6
 //
 // The row axis its own mirror image: the A entries are
 // cos and sin of k (x_(n0-1-r) - x_r) / 2 for the half rows r, g.mhalf of them per tile
-// of twice as many table rows, cosines then sines, two modes per 32-bit element (row stride Np / 2, one
-// thread per mode pair); E2 takes the phase of the axis's centre.  At most kMTableBlocks
-// blocks, so that the look at the axis is not repeated for every 256 modes.
-constexpr int64_t kMTableBlocks = 4096;
+// of twice as many table rows, cosines then sines, two modes per 32-bit element (row stride
+// Np / 2; the even thread of a mode pair packs the cosines, the odd one the sines); E2 takes
+// the phase of the axis's centre.
+constexpr int64_t kMTableWaves = 4096;  // resident at 4 per SIMD: one round
 
+// parts: runs of rows, at most 64 in each; chunks: 64-mode chunks of a row
 template <bool FP16>
-__global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int64_t N, int64_t comps,
-                                                     int64_t ka_row, int64_t k1_row, int64_t kz_row,
+__global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, unsigned parts, unsigned chunks, int64_t d, int64_t N,
+                                                     int64_t comps, int64_t ka_row, int64_t k1_row, int64_t kz_row,
                                                      const double* __restrict__ ax0,
                                                      const double* __restrict__ ax1,
                                                      const double* __restrict__ ax2,
@@ -294,101 +300,116 @@ __global__ __launch_bounds__(256) void k_mfma_tables(MfmaGeom g, int64_t d, int6
                                                      uint32_t* __restrict__ a_lo,
                                                      float2* __restrict__ e1,
                                                      float2* __restrict__ e2) {
+    const unsigned wave = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned part = wave / chunks, lane = threadIdx.x & 63u;
+    const int64_t j = (int64_t)(wave - part * chunks) * 64 + lane;
+    const bool mode = j < N;
+    double ka = 0.0, k1 = 0.0, kz = 0.0;
+    if (mode) {
+        ka = cov[ka_row * N + j];
+        kz = cov[kz_row * N + j];
+        if (d == 3) k1 = cov[k1_row * N + j];  // E1 of a 2D grid: 1
+    }
     // (the flat kernel's 3D form takes no account of it: its second E table leaves no registers)
     const bool mir = (g.g2 == 1 || d == 2) && mirrored_axis(ax0, g.n0);
-    const auto phase = [](double th, double* sn, double* cs) {
-        if (fabs(th) <= kFastPhaseMax) sincos_fast(th, sn, cs); else sincos(th, sn, cs);
-    };
-    const unsigned na = (unsigned)(mir ? g.mrow_tiles * g.mhalf : g.n0p), n1 = (unsigned)g.n1, n2 = (unsigned)g.n2;
-    const unsigned cha = (unsigned)(((mir ? g.Np / 2 : g.Np) + 255) / 256), ch = (unsigned)((g.Np + 255) / 256);
-    const unsigned items = na * cha + (n1 + n2) * ch;  // fits (the launch refuses more)
-    for (unsigned it = blockIdx.x; it < items; it += gridDim.x) {
-        if (it < na * cha) {
-            const unsigned row = it / cha;
-            const int64_t q = (int64_t)(it - row * cha) * 256 + threadIdx.x;
-            uint32_t hi, lo;
-            if (mir) {
-                const int64_t pitch = g.Np / 2, r = row;
-                if (q >= pitch) continue;
-                float c2[2] = {0.0f, 0.0f}, s2[2] = {0.0f, 0.0f};
-                if (2 * r < g.n0) {
-                    const double h = 0.5 * (ax0[g.n0 - 1 - r] - ax0[r]);
+    if (part >= parts) return;
+    const unsigned n1 = (unsigned)g.n1, n12 = n1 + (unsigned)g.n2;  // rows fit (the launch refuses more)
+    const unsigned na = (unsigned)(mir ? g.mrow_tiles * g.mhalf : g.n0p), rows = n12 + na;
+    // rows of A that hold points: the ones past them are zero, as modes past N
+    const unsigned full = n12 + (unsigned)(mir ? (g.n0 + 1) / 2 : g.n0);
+    const unsigned r0 = (unsigned)((uint64_t)rows * part / parts), r1 = (unsigned)((uint64_t)rows * (part + 1) / parts);
+    const bool in = j < g.Np;  // Np is a multiple of 32: both threads of a mode pair are in or out
+    double kc = 0.0, a = 0.0, b = 0.0, w[3] = {1.0, 0.0, 0.0};
+    if (mode && r0 < n12) {
+        if (mir) kc = ka * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
+        a = z1[j];
+        b = z2[j];
+        if (comps > 1) {
+            const double k0 = cov[j];
+            double k2 = 0.0;
+            for (int64_t e = 0; e < d; ++e) k2 += cov[e * N + j] * cov[e * N + j];
 #pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        const int64_t j = 2 * q + e;
-                        if (j < N) {
-                            double sn, cs;
-                            phase(cov[ka_row * N + j] * h, &sn, &cs);
-                            c2[e] = (float)cs;
-                            s2[e] = (float)sn;
-                        }
-                    }
-                }
-                const int64_t at = ((r / g.mhalf) * 2 * g.mhalf + r % g.mhalf) * pitch + q;
-                split2<FP16>(c2[0], c2[1], hi, lo);
-                a_hi[at] = hi;
-                a_lo[at] = lo;
-                split2<FP16>(s2[0], s2[1], hi, lo);
-                a_hi[at + g.mhalf * pitch] = hi;
-                a_lo[at + g.mhalf * pitch] = lo;
-            } else {
-                if (q >= g.Np) continue;
-                float re = 0.0f, im = 0.0f;
-                if (row < g.n0 && q < N) {
-                    double sn, cs;
-                    phase(cov[ka_row * N + q] * ax0[row], &sn, &cs);
-                    re = (float)cs;
-                    im = (float)(-sn);
-                }
-                split2<FP16>(re, im, hi, lo);
-                a_hi[row * g.Np + q] = hi;  // element pair (2q, 2q+1) of row `row`
-                a_lo[row * g.Np + q] = lo;
-            }
-            continue;
-        }
-        const unsigned rest = it - na * cha, row = rest / ch;
-        const int64_t j = (int64_t)(rest - row * ch) * 256 + threadIdx.x;
-        if (j >= g.Np) continue;
-        if (row < n1) {
-            float2 v = {0.0f, 0.0f};
-            if (j < N) {
-                if (d == 3) {
-                    double sn, cs;
-                    phase(cov[k1_row * N + j] * ax1[row], &sn, &cs);
-                    v = {(float)cs, (float)sn};
-                } else {
-                    v = {1.0f, 0.0f};
-                }
-            }
-            e1[row * g.Np + j] = v;
-            continue;
-        }
-        // E2: one phase for all components
-        const unsigned i2 = row - n1;
-        double sn = 0.0, cs = 0.0, a = 0.0, b = 0.0, k0 = 0.0, k2 = 1.0;
-        if (j < N) {
-            double th = cov[kz_row * N + j] * (d == 3 ? ax2[i2] : ax1[i2]);
-            if (mir) th += cov[ka_row * N + j] * (0.5 * (ax0[0] + ax0[g.n0 - 1]));
-            phase(th, &sn, &cs);
-            a = z1[j];
-            b = z2[j];
-            if (comps > 1) {
-                k0 = cov[j];
-                k2 = 0.0;
-                for (int64_t e = 0; e < d; ++e) k2 += cov[e * N + j] * cov[e * N + j];
-            }
-        }
-        for (int64_t comp = 0; comp < comps; ++comp) {
-            float2 v = {0.0f, 0.0f};
-            if (j < N) {
-                const double f = comps > 1 ? (comp == 0 ? 1.0 : 0.0) - cov[comp * N + j] * k0 / k2 : fac ? fac[j] : 1.0;
-                const double fa = f * a, fb = f * b;
-                // (fa - i fb)(c + i s)
-                v = {(float)(fa * cs + fb * sn), (float)(fa * sn - fb * cs)};
-            }
-            e2[comp * g.e2_elems + i2 * g.Np + j] = v;
+            for (int c = 0; c < 3; ++c)
+                if (c < comps) w[c] = (c == 0 ? 1.0 : 0.0) - cov[c * N + j] * k0 / k2;
+        } else if (fac) {
+            w[0] = fac[j];
         }
     }
+    float2* e2j = e2 + j;
+    // this lane's of the run's rows: the row's coordinate (half distance, mirrored)
+    double xs = 0.0;
+    const unsigned q = r0 + lane;
+    if (q < n1)
+        xs = d == 3 ? ax1[q] : 0.0;
+    else if (q < n12)
+        xs = (d == 3 ? ax2 : ax1)[q - n1];
+    else if (q < full)
+        xs = mir ? 0.5 * (ax0[g.n0 - 1 - (q - n12)] - ax0[q - n12]) : ax0[q - n12];
+    // everything read has arrived before the loop: a wait for reads in it would wait for
+    // the stores of the row before, too
+    asm volatile("" : "+v"(xs), "+v"(ka), "+v"(k1), "+v"(kz), "+v"(kc), "+v"(a), "+v"(b), "+v"(w[0]), "+v"(w[1]),
+                      "+v"(w[2]));
+    const uint64_t xb = __builtin_bit_cast(uint64_t, xs);
+    auto phase = [&](unsigned row) {
+        const int i = (int)(row - r0);
+        const double x = __builtin_bit_cast(
+            double, (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(xb >> 32), i) << 32 |
+                        (uint32_t)__builtin_amdgcn_readlane((int)xb, i));
+        return row >= n12 ? ka * x : row >= n1 ? fma_(kz, x, kc) : k1 * x;
+    };
+    auto entry = [&](unsigned row, double sn, double cs) {
+        if (!mode || row >= full) sn = cs = 0.0;
+        if (row >= n12) {
+            const unsigned r = row - n12;
+            uint32_t hi, lo;
+            int64_t at;
+            if (mir) {
+                // the even thread of a mode pair packs the cosines, the odd one the sines
+                const bool odd = j & 1;
+                const float mine = odd ? (float)sn : (float)cs, other = __shfl_xor(odd ? (float)cs : (float)sn, 1);
+                split2<FP16>(odd ? other : mine, odd ? mine : other, hi, lo);
+                const unsigned half = (unsigned)g.mhalf, first = r / half * half;
+                at = (int64_t)(first + r + (odd ? half : 0u)) * (g.Np / 2) + (j >> 1);
+            } else {
+                split2<FP16>((float)cs, (float)-sn, hi, lo);
+                at = (int64_t)r * g.Np + j;  // element pair (2j, 2j+1) of row r
+            }
+            if (in) {
+                a_hi[at] = hi;
+                a_lo[at] = lo;
+            }
+        } else if (row >= n1) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                if (c < comps && in) {
+                    // (f z1 - i f z2)(cos + i sin)
+                    const double fa = w[c] * a, fb = w[c] * b;
+                    e2j[c * g.e2_elems + (int64_t)(row - n1) * g.Np] = {(float)(fa * cs + fb * sn),
+                                                                        (float)(fa * sn - fb * cs)};
+                }
+        } else if (in) {
+            e1[(int64_t)row * g.Np + j] = {(float)cs, (float)sn};
+        }
+    };
+    bool wide = false;
+    for (unsigned row = r0; row < r1; ++row) {
+        const double th = phase(row);
+        if (!__all(fabs(th) <= kFastPhaseMax)) {  // (or not finite)
+            wide = true;
+            continue;
+        }
+        double sn, cs;
+        sincos_fast(th, &sn, &cs);
+        entry(row, sn, cs);
+    }
+    if (wide)  // rows with phases for the library, by themselves: its constants take registers
+        for (unsigned row = r0; row < r1; ++row) {
+            const double th = phase(row);
+            if (__all(fabs(th) <= kFastPhaseMax)) continue;
+            double sn, cs;
+            if (fabs(th) <= kFastPhaseMax) sincos_fast(th, &sn, &cs); else sincos(th, &sn, &cs);
+            entry(row, sn, cs);
+        }
 }
 
 // ---------------------------------------------------------------- GEMM -----
@@ -989,11 +1010,14 @@ int mfma_launch(const MfmaGeom& g, int64_t fill, int64_t d, int64_t N, int64_t c
     uint32_t* a_lo = a_hi + g.a_elems / 2;
     float2* e1 = reinterpret_cast<float2*>(a_lo + g.a_elems / 2);
     float2* e2 = e1 + g.e1_elems;
-    const int64_t items = (g.n0p + g.n1 + g.n2) * ceil_div(g.Np, (int64_t)256);
-    if (items > 0x7fffffffLL) return GSX_E_INVALID;
-    const int64_t tblocks = items < kMTableBlocks ? items : kMTableBlocks;
-    hipLaunchKernelGGL((k_mfma_tables<FP16>), dim3((unsigned)tblocks), dim3(256), 0, s, g, d,
-                       N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, a_hi, a_lo, e1, e2);
+    const int64_t trows = g.n0p + g.n1 + g.n2, chunks = ceil_div(g.Np, (int64_t)64);  // (a mirrored axis has fewer rows)
+    if (trows > 0x7fffffffLL || chunks > 0x7fffffffLL) return GSX_E_INVALID;
+    int64_t parts = ceil_div(kMTableWaves, chunks);
+    if (parts < ceil_div(trows, (int64_t)64)) parts = ceil_div(trows, (int64_t)64);
+    if (parts > trows) parts = trows;
+    hipLaunchKernelGGL((k_mfma_tables<FP16>), dim3((unsigned)ceil_div(parts * chunks, (int64_t)4)), dim3(256), 0, s, g,
+                       (unsigned)parts, (unsigned)chunks, d, N, comps, ka_row, k1_row, kz_row, ax0, ax1, ax2, cov, z1, z2, fac, a_hi, a_lo,
+                       e1, e2);
     int st = launch_status();
     if (st != GSX_OK) return st;
     const int64_t steps_per = mfma_steps_per_split(g, comps, fill);

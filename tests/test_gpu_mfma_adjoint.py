@@ -163,6 +163,52 @@ def test_mfma_mirrored_row_axis(shape, n, comps):
     assert np.isnan(fn(cov, z1, z2, bad, "bf16x3").cpu().numpy().reshape(comps, -1)[:, 0]).all()
 
 
+@pytest.mark.parametrize("irregular", [False, True])
+@pytest.mark.parametrize("shape,n,comps", [
+    ((150, 40, 60), 2100, 1),  # 125 runs of two or three rows, some over two tables
+    ((70, 17, 33), 4100, 3),
+    ((300, 130), 2080, 2),
+    ((8200, 20), 2100, 1),     # runs of more than 64 rows are split
+    ((40, 300), 70, 1),        # a factorised last axis, 96 table columns
+])
+def test_mfma_table_runs(shape, n, comps, irregular):
+    """Mode tables whose wavefronts take runs of several rows, against the direct FP64 sum at the
+    split precision's bars."""
+    _say(f"mfma table runs shape={shape} N={n} comps={comps} irregular={irregular}")
+    rs = np.random.RandomState(n)
+    cov, z1, z2 = _modes(len(shape), n, 7 + n, kscale=0.6)
+    axes = [np.arange(s) * (20.0 / s) - 3.0 - i for i, s in enumerate(shape)]
+    if irregular:
+        axes[0] = np.sort(rs.uniform(-10.0, 10.0, shape[0]))
+    fn = summate_incompr_grid_device if comps > 1 else summate_grid_device
+    ref = fn(cov, z1, z2, axes, "fp64").cpu().numpy().ravel()
+    for precision in ("fp16x3", "bf16x3"):
+        got = fn(cov, z1, z2, axes, precision).cpu().numpy().astype(np.float64).ravel()
+        rel_max, rel_rms = oracle.rel_errors(got, ref)
+        assert rel_rms <= 1e-5 and rel_max <= (1e-5 if precision == "fp16x3" else 5e-5)
+
+
+@pytest.mark.parametrize("shape", [(65, 20, 18), (66, 300)])
+def test_mfma_tables_of_huge_phases(shape):
+    """Row coordinates beyond the fast phase reduction (2^46 rad), mirrored about 0 and not; the
+    modes run along the rows only, so the phase is one rounded product in every form."""
+    _say(f"mfma huge phases shape={shape}")
+    rs = np.random.RandomState(shape[0])
+    cov, z1, z2 = _modes(len(shape), 90, 3, kscale=1.0)
+    cov[1:] = 0.0
+    half = np.sort(rs.uniform(1.0, 9e14, shape[0] // 2))
+    mirrored = np.concatenate([-half[::-1], np.zeros(shape[0] % 2), half])
+    irregular = mirrored * rs.uniform(0.9, 1.1, shape[0])
+    for ax0 in (mirrored, irregular):
+        assert (np.abs(cov[0][:, None] * ax0) > 2.0**46).any() and (np.abs(cov[0][:, None] * ax0) < 2.0**46).any()
+        axes = [ax0] + [np.arange(s) * 0.5 for s in shape[1:]]
+        ref = summate_grid_device(cov, z1, z2, axes, "fp64").cpu().numpy().ravel()
+        for precision in ("fp16x3", "bf16x3"):
+            got = summate_grid_device(cov, z1, z2, axes, precision).cpu().numpy().astype(np.float64).ravel()
+            rel_max, rel_rms = oracle.rel_errors(got, ref)
+            assert rel_rms <= 1e-5 and rel_max <= (1e-5 if precision == "fp16x3" else 5e-5)
+
+
 def test_mfma_uniform_flag_checked_and_ignored():
     """The flag on a non-uniform axis gives an all-NaN output (the device check); on a 3D
     grid or an axis shorter than 256 points it is ignored (same bits as without it)."""
