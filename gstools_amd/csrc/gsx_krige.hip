@@ -403,8 +403,8 @@ __device__ __forceinline__ double cov_of(const CovModelArgs& m, double inv, doub
 // registers and writes kCovRows rows (conditioning points i0 .. i0 + kCovRows - 1,
 // read as wave-uniform values), so the targets are read once per kCovRows rows.  Bound by
 // the vector unit (square root and exponential) and by stores of 512 bytes per wave: a pair
-// of points per thread where P and ld are even and out is 16-byte aligned, the model a template
-// argument, the quotient by a reciprocal.  Exponential, 300 x 40000 in 2D: 39 -> 30 us.
+// of points per thread in large launches where P and ld are even and out is 16-byte aligned, the
+// model a template argument, the quotient by a reciprocal.  Exponential, 300 x 40000 in 2D: 39 -> 30 us.
 constexpr int kCovRows = 16;
 
 template <int DIM, int KIND, bool kPair, bool kDiv>
@@ -450,7 +450,10 @@ void krige_cov_launch(const CovModelArgs& m, int64_t K, int64_t P, const double*
                       double* out, int64_t ld, hipStream_t s) {
     // lengths whose reciprocal and remainders are exact enough: far from the exponent's limits
     const bool div = !(m.len >= 0x1p-400 && m.len <= 0x1p+400);
-    const bool pair = !div && P % 2 == 0 && ld % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    // pairs where they leave four blocks per CU: below that single points, twice the blocks, are
+    // faster (Stable, 300 x 10000: 37 us in pairs, 30 singly; 300 x 40000: 96 and 100)
+    const bool enough = ceil_div(P, (int64_t)512) * ceil_div(K, (int64_t)kCovRows) >= 1024;
+    const bool pair = enough && !div && P % 2 == 0 && ld % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
     const dim3 grid((unsigned)ceil_div(P, (int64_t)(pair ? 512 : 256)), (unsigned)ceil_div(K, (int64_t)kCovRows));
     auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, m, K, P, cpos, pos, out, ld); };
     auto form = [&](auto pairs, auto singles, auto division) { pair ? go(pairs) : div ? go(division) : go(singles); };

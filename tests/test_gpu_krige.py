@@ -89,6 +89,28 @@ def test_covariance_rows_forms(p, length):
         assert np.max(np.abs(got - model.covariance(cdist(cpos.T, pos.T)))) <= 4e-15 * 1.7
 
 
+@pytest.mark.parametrize("dim", [1, 2, 3])
+def test_covariance_rows_in_pairs_equal_single_points(dim):
+    """Rows onto 200000 points are written two points to a thread, onto an odd number of points
+    and onto few points one: the same bits, and the host's covariance at some of them."""
+    from scipy.spatial.distance import cdist
+
+    from gstools_amd.krige import krige_cov_device
+
+    _say(f"krige covariance pairs dim={dim}")
+    rs = np.random.RandomState(dim)
+    k, p = 37, 200_000
+    cpos, pos = rs.uniform(0, 40, size=(dim, k)), rs.uniform(0, 40, size=(dim, p))
+    pos[:, :5] = cpos[:, :5]  # r = 0
+    for model in (gs.Gaussian(dim=dim, var=1.7, len_scale=9.0), gs.Exponential(dim=dim, var=1.7, len_scale=9.0),
+                  gs.Stable(dim=dim, var=1.7, len_scale=9.0, alpha=1.3), gs.Spherical(dim=dim, var=1.7, len_scale=9.0)):
+        pairs = krige_cov_device(model, cpos, pos)
+        assert torch.equal(pairs[:, :-1], krige_cov_device(model, cpos, np.ascontiguousarray(pos[:, :-1])))
+        assert torch.equal(pairs[:, :1000], krige_cov_device(model, cpos, np.ascontiguousarray(pos[:, :1000])))
+        ref = model.covariance(cdist(cpos.T, pos[:, :500].T))
+        assert np.max(np.abs(pairs[:, :500].cpu().numpy() - ref)) <= 8 * 2.3e-16 * model.sill
+
+
 def test_empty_conditions_and_errors():
     _say("krige empty / errors")
     f, e = calc_field_krige_and_variance(np.zeros((0, 0)), np.zeros((0, 6)), np.zeros(0))
