@@ -481,22 +481,42 @@ int launch_f32_split(Pts pts, int64_t N, int64_t P, const double* cov, const dou
     return launch_status();
 }
 
-// Whether the split kernels serve (N, P).  A plain block of 512 (FP64) or 2048 / 1024
-// (FP32 scalar / incompressible) points walks all N modes for them, so up to one block per CU a launch takes the time of one block whatever P is (10^4
-// points, 1000 modes, 2D: FP64 130 us, FP32 119 us); a split launch takes rounds
-// of 256 blocks (24 and 14 us).  Fits of the measured times (us; 2D and 3D, 64 to
-// 4096 modes, 1 to 10^6 points; C chunks of 1024 modes, R rounds):
-//   FP64  plain N / 7.7      split R (8 C + N / 46)
-//   FP32  plain 5 + N / 8.9  split R (12 C + N / 56), in 1D 5 + N / 10.5 and R (8 C + N / 66)
-// The plain fits hold up to 131072 (FP64), 524288 (FP32) and 262144 (FP32
-// incompressible) points; the rounds that the inequalities allow end before.
-template <bool F64, int D>
+// Whether the split kernels serve (N, P).  A plain launch of up to one block per CU takes the
+// time of one block walking all N modes, and takes the smallest blocks that keep it to that
+// (plain_ppt): one point per thread up to 65536 points in FP64, two up to 131072 in FP32, then
+// as many more per multiple of that.  A split launch takes rounds of 256 blocks whose waves
+// share the modes.  SplitFit: the times of both forms, in us, as fitted to measurements from
+// 8000 to 131072 points in FP64, 500000 in FP32 (incompressible 262144: where four rounds end),
+// 100 to 4000 modes; plain base + N / rate[m], m multiples less one, split rounds times (start +
+// chunk C + N / modes), C chunks of 1024 modes.  Smaller FP32 blocks (up to 65536 points) are
+// faster than the split fit and always serve from 129 modes on.
+// 10^4 points, 1000 modes in 2D: FP64 84 us plain, 18 split, FP32 58 and 15.  200 modes, 40000
+// points in 3D, incompressible, FP64: 21 plain, 34 split; 400 modes, 190000 points, FP32: 39, 46.
+struct SplitFit {
+    double base, rate[4], start, chunk, modes;
+};
+
+template <bool F64, int D, bool INCOMPR>
+constexpr SplitFit split_fit() {
+    constexpr SplitFit k64[2][3] = {
+        {{6.4, {14.3, 9.8, 9.8, 9.8}, 1.6, 7.5, 56.0}, {6.4, {12.6, 9.4, 9.4, 9.4}, 1.6, 8.1, 52.0},
+         {6.4, {12.5, 8.3, 8.3, 8.3}, 1.6, 8.2, 48.0}},
+        {{}, {5.0, {13.1, 8.4, 8.4, 8.4}, 2.3, 5.7, 45.0}, {5.0, {11.8, 7.0, 7.0, 7.0}, 3.8, 7.6, 40.0}}};
+    constexpr SplitFit k32[2][3] = {
+        {{8.0, {22.8, 15.5, 14.3, 10.8}, 3.7, 5.3, 66.0}, {8.0, {19.7, 13.9, 11.9, 8.9}, 5.0, 7.4, 57.0},
+         {6.8, {18.7, 12.7, 10.2, 8.4}, 6.7, 7.4, 47.0}},
+        {{}, {6.0, {17.4, 11.9, 10.6, 8.2}, 4.2, 3.9, 81.0}, {6.0, {15.4, 10.6, 8.7, 7.0}, 5.3, 6.6, 68.0}}};
+    return F64 ? k64[INCOMPR][D - 1] : k32[INCOMPR][D - 1];
+}
+
+template <bool F64, int D, bool INCOMPR>
 inline bool split_pays(int64_t N, int64_t P, int64_t round_points) {
-    const double R = (double)ceil_div(P, round_points), C = (double)ceil_div(N, (int64_t)kSplitModes);
-    const double n = (double)N;
-    if (R > 4.0) return false;
-    if (F64) return R * (8.0 * C + n / 46.0) <= n / 7.7;
-    return D == 1 ? R * (8.0 * C + n / 66.0) <= 5.0 + n / 10.5 : R * (12.0 * C + n / 56.0) <= 5.0 + n / 8.9;
+    constexpr SplitFit f = split_fit<F64, D, INCOMPR>();
+    const int64_t R = ceil_div(P, round_points), C = ceil_div(N, (int64_t)kSplitModes);
+    if (R > 4) return false;
+    if (!F64 && P <= 65536 && N > 128) return true;
+    const int64_t m = ceil_div(P, (int64_t)(F64 ? 65536 : 131072));  // 1 to 4: R is at most 4
+    return (double)R * (f.start + f.chunk * (double)C + (double)N / f.modes) <= f.base + (double)N / f.rate[m - 1];
 }
 
 template <int D, bool INCOMPR, class Pts, class OutT>
@@ -504,7 +524,7 @@ int launch_forward(Pts pts, int64_t N, int64_t P, const double* cov, const doubl
                    const double* z2, const double* fac, OutT* out, hipStream_t s) {
     if constexpr (sizeof(OutT) == 8) {
         // the smallest blocks that keep the launch within one round of 256
-        if (split_pays<true, D>(N, P, 256 * 128)) {
+        if (split_pays<true, D, INCOMPR>(N, P, 256 * 128)) {
             if (P <= 256 * 32) return launch_f64_split<D, 1, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             if (P <= 256 * 64) return launch_f64_split<D, 2, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             return launch_f64_split<D, 2, 1, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
@@ -526,7 +546,7 @@ int launch_forward(Pts pts, int64_t N, int64_t P, const double* cov, const doubl
             plain(k_forward_f64<D, 1, INCOMPR, Pts>);
     } else {
         constexpr int big = INCOMPR ? 4 : 8;  // points per thread of the largest split block
-        if (split_pays<false, D>(N, P, 256 * 64 * big)) {
+        if (split_pays<false, D, INCOMPR>(N, P, 256 * 64 * big)) {
             if (P <= 256 * 64) return launch_f32_split<D, 1, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             if (P <= 256 * 128) return launch_f32_split<D, 2, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
             if (P <= 256 * 256) return launch_f32_split<D, 4, INCOMPR>(pts, N, P, cov, z1, z2, fac, out, s);
