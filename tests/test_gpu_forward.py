@@ -265,3 +265,49 @@ def test_plain_launches_agree_whatever_their_blocks(d, precision, incompr):
     for p in (140_003, 262_145, 393_217, 524_289, 600_000, 700_001, 800_000, 1_048_576):
         got = fn(cov, z1, z2, pos[:, :p].contiguous(), precision).reshape(-1, p)
         assert torch.equal(got, want[:, :p]), (p, precision)
+
+
+@pytest.mark.parametrize("incompr", [False, True])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("d,n", [(1, 129), (1, 1500), (2, 129), (3, 191)])
+def test_split_launches_that_end_inside_a_group(d, n, precision, incompr):
+    """As above for mode counts one past a group and for 1D, with points beyond 2^46 rad in FP64."""
+    d = max(d, 2) if incompr else d
+    _say(f"split launches d={d} N={n} {precision} incompr={incompr}")
+    big = 600_001
+    rs = np.random.RandomState(n + d)
+    cov = torch.from_numpy(rs.standard_cauchy(size=(d, n))).cuda()
+    z1, z2 = torch.from_numpy(rs.normal(size=(2, n))).cuda()
+    pos = torch.from_numpy(rs.uniform(-200.0, 200.0, size=(d, big))).cuda()
+    pos[:, ::2048] *= 5e3 if precision == "fp32" else 1e12
+    fn = summate_incompr_device if incompr else summate_device
+    want = fn(cov, z1, z2, pos, precision).reshape(-1, big)
+    for p in (1, 31, 33, 64, 65, 127, 129, 8192, 8193, 16385, 32768):
+        got = fn(cov, z1, z2, pos[:, :p].contiguous(), precision).reshape(-1, p)
+        assert torch.equal(got, want[:, :p]), (p, precision)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("d,n,p", [(1, 300, 600_001), (2, 64, 40_000), (3, 300, 600_001)])
+def test_plain_launches_with_huge_and_non_finite_coordinates(d, n, p, precision):
+    """Launches too large or of too few modes to be split: phases beyond 2^46 rad (FP64) or 2^18
+    revolutions (FP32) take the guarded reductions and agree with the oracle; a NaN or infinite
+    coordinate gives NaN at its point and changes no other's value beyond the bars."""
+    _say(f"plain launches, odd coordinates d={d} N={n} P={p} {precision}")
+    cov, z1, z2, pos = _case(d, n, p, 50 + d, 1.0, 100.0)
+    pos[:, 1000:1500] *= 3e12 if precision == "fp64" else 3e4
+    pos[0, 777], pos[-1, 2500], pos[0, p - 1] = np.nan, np.inf, -np.inf
+    got = summate_device(cov, z1, z2, pos, precision).cpu().numpy().astype(np.float64)
+    hit = np.zeros(p, bool)
+    hit[[777, 2500, p - 1]] = True
+    assert np.all(np.isnan(got[hit])) and np.all(np.isfinite(got[~hit]))
+    some = np.flatnonzero(~hit)
+    some = np.concatenate([some[:6000], some[-3000:]])
+    ref = oracle.summate_c(cov, z1, z2, np.ascontiguousarray(pos[:, some]))
+    tol = FP64_TOL if precision == "fp64" else FP32_TOL
+    rel_max, rel_rms = oracle.rel_errors(got[some], ref)
+    assert rel_max <= tol and rel_rms <= tol, (rel_max, rel_rms)
+    few = np.ascontiguousarray(pos[:, 996:1600])  # FP64: the same bits from a launch of few points
+    if precision == "fp64":
+        part = summate_device(cov, z1, z2, few, precision).cpu().numpy()
+        assert np.array_equal(part, got[996:1600])
