@@ -274,3 +274,22 @@ def test_one_field_pairs_at_tile_and_sorting_edges(kind, dim, p):
             assert np.allclose(g, g_ref, rtol=1e-12, atol=1e-300, equal_nan=True)
             g2, c2 = v.unstructured(f, edges, pos, est)
             assert np.array_equal(g, g2, equal_nan=True) and np.array_equal(c, c2)
+
+
+@pytest.mark.parametrize("kind", ["uniform", "crowded", "odd"])
+def test_one_field_pairs_in_groups_of_tiles(kind):
+    """One field of 50000 points: from about 46000 on a work item is a group of tiles.  Most tile
+    pairs lie beyond the last edge where the points are sorted ("uniform"); "crowded" points keep
+    their given order, with 5e8 pairs in one bin.  A field of small whole numbers makes every
+    sum of squares exact in any order, so counts and estimates are those of the oracle."""
+    _say(f"vario groups {kind}")
+    rs = np.random.RandomState(11)
+    dim, p = 2, 50_001
+    pos = _iso_points(kind, dim, p, rs)
+    f = rs.randint(-8, 9, size=p).astype(float)
+    f[rs.choice(p, p // 50, replace=False)] = np.nan
+    edges = np.linspace(0.0, 4.0, 17)
+    g, c = v.unstructured(f, edges, pos, "m")
+    g_ref, c_ref = oracle.vario_unstructured_c(f[None], edges, pos, "m")
+    assert np.array_equal(c, c_ref)
+    assert np.array_equal(g, g_ref)
