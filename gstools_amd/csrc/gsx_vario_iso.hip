@@ -560,9 +560,10 @@ __device__ __forceinline__ IsoFast iso_fast(const IsoEdges& e, double diag, int 
     // differences to 2^-24, so |d32 - d| <= 2^-24 (diag + d) plus 3.5 roundings of the
     // squares, sums and root (v_sqrt_f32: one ulp); scaling and offset add
     // 2^-24 (d / w + |e0| / w + B + 2).  Up to the last edge d <= emax; doubled, and the
-    // edges' own deviation from uniform on top.
+    // edges' own deviation from uniform on top.  Squares below 2^-126 count as 0 (v_sqrt_f32
+    // takes no denormal numbers): up to sqrt(3) 2^-63 of a distance, below 2^-62.
     IsoFast r;
-    r.eps = 0x1p-23 * ((diag + 6.5 * e.emax) * e.inv_w + fabs(e.e0) * e.inv_w + B + 4.0) + e.dev;
+    r.eps = 0x1p-23 * ((diag + 6.5 * e.emax) * e.inv_w + fabs(e.e0) * e.inv_w + B + 4.0) + e.dev + 0x1p-62 * e.inv_w;
     // (a batch of 256 pairs is done again with a chance of up to 512 eps)
     r.on = e.uniform != 0 && diag < 1.0e18 && r.eps <= 0x1p-11;
     return r;

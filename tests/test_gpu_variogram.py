@@ -293,3 +293,18 @@ def test_one_field_pairs_in_groups_of_tiles(kind):
     g_ref, c_ref = oracle.vario_unstructured_c(f[None], edges, pos, "m")
     assert np.array_equal(c, c_ref)
     assert np.array_equal(g, g_ref)
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-3, 1e3])
+def test_one_field_pairs_whose_squares_underflow_fp32(scale):
+    """Distances about an edge at 5e-20, bins of 1e-15 and points 1e-15 apart: the squares of the
+    short distances lie below FP32's normal range."""
+    _say(f"vario tiny distances scale={scale}")
+    rs = np.random.RandomState(5)
+    pos = np.concatenate([np.arange(40) * 7e-21, 1e-15 + np.arange(30) * 9e-21, rs.uniform(0, 2e-15, 60)])[None]
+    f = rs.normal(size=pos.shape[1])
+    edges = (5e-20 + np.arange(4) * 1e-15) * scale
+    g, c = v.unstructured(f, edges, pos * scale, "m")
+    g_ref, c_ref = oracle.vario_unstructured_c(f[None], edges, pos * scale, "m")
+    assert np.array_equal(c, c_ref)
+    _close(g, g_ref)
