@@ -9,8 +9,8 @@
 // error into the kriging variance max(sill - error, 0).
 //
 // Field (both forms): field = (M^T cond) . v_k: a weight vector a (K), then a sum
-// over the rows of V in four classes j mod 4, each from the last row down, added
-// as (0 + 1) + (2 + 3).  The variance form takes it from the rows of V that the
+// over the rows of V in four classes j mod 4, each in steps of 16 rows from the last step
+// down, up within a step, added as (0 + 1) + (2 + 3).  The variance form takes it from the rows of V that the
 // GEMM stages anyway (a pass over V saved); k_krige_field adds the same numbers
 // in the same order, so the field's bits do not depend on the form or on P.
 //

@@ -106,7 +106,7 @@ inline MfmaGeom mfma_geom(int64_t d, int64_t N, const int64_t* shape) {
 constexpr int64_t kMFillBlocks = 512;
 constexpr int kMFillLog2Min = 8, kMFillLog2Max = 11;
 
-// Between two and four fifths of that (k_mfma_grid3), half of the CUs have one block and a
+// Between a half and four fifths of that (k_mfma_grid3), half of the CUs have one block and a
 // step of two blocks on a CU takes 4576 cycles, of one 2900: twice the splits, two blocks
 // and then one on every CU, save about 840 cycles (0.4 us) per 32-mode step of the fewer
 // splits, and cost the partial sums' way through memory (about 9 TB/s) once more.

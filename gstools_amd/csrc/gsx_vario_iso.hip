@@ -65,7 +65,7 @@ struct IsoEdges {
 };
 
 struct IsoArgs {
-    int64_t P, Pp, B;
+    int64_t B;
     int64_t h0, h1;      // slots (bins) of this launch
     int gl2;             // log2 of the k tiles per work item (<= 6)
 };
@@ -171,12 +171,12 @@ __device__ void edge_setup(int B, const double* __restrict__ edges, double* __re
         thp[i + 1] = sq_threshold(e);
         if (i < B) mono_l = mono_l && (e <= edges[i + 1]);
         const double x = fabs(e - (e0 + i * w)) / w;
-        dev = x <= dev ? dev : x;  // NaN is kept
+        dev = x <= dev || dev != dev ? dev : x;  // NaN is kept
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         const double x = __shfl_xor(dev, o);
-        dev = x <= dev ? dev : x;
+        dev = x <= dev || dev != dev ? dev : x;
     }
     const bool mono = __all(mono_l);
     // uniform: the FP32 guess of the FP64 form is exact after one threshold step
@@ -983,8 +983,6 @@ int iso_run(const IsoLayout& l, int64_t P, int64_t B, const double* f, const dou
     if ((st = launch_status()) != GSX_OK) return st;
     for (int64_t h0 = 0; h0 < B; h0 += l.slots) {
         IsoArgs a;
-        a.P = P;
-        a.Pp = l.Pp;
         a.B = B;
         a.h0 = h0;
         a.h1 = h0 + l.slots < B ? h0 + l.slots : B;
