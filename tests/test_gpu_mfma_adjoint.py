@@ -188,6 +188,20 @@ def test_mfma_table_runs(shape, n, comps, irregular):
         assert rel_rms <= 1e-5 and rel_max <= (1e-5 if precision == "fp16x3" else 5e-5)
 
 
+@pytest.mark.parametrize("n0", [4095, 4096, 4097, 4098])
+def test_mfma_row_axes_around_the_mirrored_limit(n0):
+    """Regular row axes of up to 4096 points take the mirrored form, longer ones the general."""
+    _say(f"mfma rows {n0}")
+    cov, z1, z2 = _modes(2, 70, 5, kscale=0.6)
+    for cols in (20, 300):  # flat columns and a factorised last axis
+        axes = [np.arange(n0) * 0.004 - 3.0, np.arange(cols) * 0.1]
+        ref = summate_grid_device(cov, z1, z2, axes, "fp64").cpu().numpy()
+        for precision in ("fp16x3", "bf16x3"):
+            got = summate_grid_device(cov, z1, z2, axes, precision).cpu().numpy().astype(np.float64)
+            rel_max, rel_rms = oracle.rel_errors(got, ref)
+            assert rel_rms <= 1e-5 and rel_max <= (1e-5 if precision == "fp16x3" else 5e-5)
+
+
 @pytest.mark.parametrize("shape", [(65, 20, 18), (66, 300)])
 def test_mfma_tables_of_huge_phases(shape):
     """Row coordinates beyond the fast phase reduction (2^46 rad), mirrored about 0 and not; the
