@@ -92,6 +92,12 @@ inline AdjPlan adj_plan(int64_t N, int64_t P, int64_t max_chunks_cap = 0) {
     return pl;
 }
 
+// Chunks that the workspace query answers for: enough for both precisions.
+inline int64_t adj_query_chunks(int64_t N, int64_t P) {
+    const int64_t c64 = adj_plan<true>(N, P).chunks, c32 = adj_plan<false>(N, P).chunks;
+    return c64 > c32 ? c64 : c32;
+}
+
 inline int adj_modes(const AdjPlan& pl, int64_t N) {
     return N > kThreads && ceil_div(N, (int64_t)kThreads * kAdjModesF32) * pl.chunks >= 512 ? kAdjModesF32 : 1;
 }
@@ -450,9 +456,10 @@ int adjoint_entry(int64_t d, int64_t N, int64_t P, const double* cov, const doub
     const int st = adjoint_prologue<GT>(d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, s, &done);
     if (done) return st;
     const int64_t per_chunk = (2 + 2 * d) * N * (int64_t)sizeof(double);
-    // room for the plan's chunks, or for those of whole stages
-    const AdjPlan pl = adj_plan<sizeof(GT) == 8>(N, P);
-    const int64_t whole = adj_whole_stages(N, P), least = whole < pl.chunks ? whole : pl.chunks;
+    // room for the query's chunks; FP32, which hardly ever has as many, for those of whole
+    // stages if that is less (10000 modes, 52 stages: 51 by the query, 52 of whole stages)
+    const int64_t query = adj_query_chunks(N, P), whole = adj_whole_stages(N, P);
+    const int64_t least = sizeof(GT) == 4 && whole < query ? whole : query;
     if (!ws || ws_bytes < least * per_chunk) return GSX_E_WORKSPACE;
     return adjoint_run<GT>(adj_plan<sizeof(GT) == 8>(N, P, ws_bytes / per_chunk), d, N, P, cov, z1, z2, pos, g, gz1, gz2, gk, ws, s);
 }
@@ -519,8 +526,7 @@ extern "C" {
 int64_t gsx_summate_adjoint_workspace(int64_t d, int64_t N, int64_t P) {
     if (d < 1 || d > 3 || N < 0 || P < 0) return GSX_E_INVALID;
     if (N == 0 || P == 0) return 0;
-    const int64_t c64 = gsx::adj_plan<true>(N, P).chunks, c32 = gsx::adj_plan<false>(N, P).chunks;
-    return (c64 > c32 ? c64 : c32) * (2 + 2 * d) * N * (int64_t)sizeof(double);
+    return gsx::adj_query_chunks(N, P) * (2 + 2 * d) * N * (int64_t)sizeof(double);
 }
 
 int gsx_summate_adjoint_f64(int64_t d, int64_t N, int64_t P, const double* cov, const double* z1,

@@ -263,8 +263,8 @@ int gsx_summate_fourier_tensor_f64(int64_t d, const int64_t* mode_no,
  *   gk[d][j] = sum_i g_i x_id (z2_j cos(k_j.x_i) - z1_j sin(k_j.x_i))
  * (unscaled, like the forward).  Deterministic two-stage reduction over
  * points.  Workspace bytes from gsx_summate_adjoint_workspace(), enough for
- * both precisions.  A smaller one that holds (2 + 2d) N c 8 bytes is taken
- * too, c = ceil(s / ceil(s / m)) point chunks, s = ceil(P / 256), m = min(s,
+ * both precisions.  The FP32 entry takes a smaller one that holds (2 + 2d) N c 8
+ * bytes, too, c = ceil(s / ceil(s / m)) point chunks, s = ceil(P / 256), m = min(s,
  * ceil(2048 / ceil(N / 256))); sums over fewer chunks differ in rounding only. */
 int64_t gsx_summate_adjoint_workspace(int64_t d, int64_t N, int64_t P);
 int gsx_summate_adjoint_f64(int64_t d, int64_t N, int64_t P, const double* cov,
